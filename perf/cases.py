@@ -88,7 +88,7 @@ def _size(rng, lo, hi, nb_lo, nb_hi, nt_lo):
 def _cubes(rng):
     """(N, NB) of a 3-D problem: tiles of 8 x 8 x 8 grid points, whose ranks stay below half of their rows, the
     last one a few rows short."""
-    return 512 * rng.randint(6, 9) - rng.randint(0, 40), 512
+    return 512 * rng.randint(6, 8) - rng.randint(0, 40), 512
 
 
 def draw(rng):
