@@ -28,7 +28,9 @@ __device__ __forceinline__ mk_d4 mk_mfma(double a, double b, mk_d4 c)
 // (AK = "k contiguous", i.e. A given transposed).  B element (k, j):
 // BK ? B[k + j ldb] : B[j + k ldb].  TE: the element type in memory, widened
 // to double on load (double, float, or a type that converts to double).
-template <bool AK, bool BK, typename TE = double>
+// COH: read past this CU's vector L1 (agent-scope loads, served by the L2),
+// for operands that another workgroup of the running kernel wrote.
+template <bool AK, bool BK, typename TE = double, bool COH = false>
 struct MkOps {
     const TE *A;
     long lda;
@@ -41,8 +43,14 @@ struct MkOps {
 // their (row, k) / (column, k) indices, A(i, k) = 0 for k > i and
 // B(k, j) = 0 for k > j, whatever memory holds there.  All 256 threads must
 // call it uniformly.
-template <bool AK, bool BK, bool TRI = false, typename TE = double>
-__device__ __forceinline__ void mk_accum(const MkOps<AK, BK, TE> &op, int M, int N, int i0, int j0, long k0, long k1,
+template <bool COH, typename TE>
+__device__ __forceinline__ double mk_load(const TE *p)
+{
+    if constexpr (COH) return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    else return (double)*p;
+}
+template <bool AK, bool BK, bool TRI = false, typename TE = double, bool COH = false>
+__device__ __forceinline__ void mk_accum(const MkOps<AK, BK, TE, COH> &op, int M, int N, int i0, int j0, long k0, long k1,
                                          mk_d4 (&acc)[2][2], double *sm)
 {
     double *As = sm, *Bs = sm + MK_KC * MK_LD;
@@ -61,7 +69,7 @@ __device__ __forceinline__ void mk_accum(const MkOps<AK, BK, TE> &op, int M, int
             const long gk = kc + kk;
             const int gi = i0 + ii;
             pa[q] = (gi < M && gk < k1 && (!TRI || gk <= gi))
-                        ? (double)(AK ? op.A[gk + (long)gi * op.lda] : op.A[gi + gk * op.lda])
+                        ? mk_load<COH>(AK ? op.A + gk + (long)gi * op.lda : op.A + gi + gk * op.lda)
                         : 0.0;
             int jj;
             if (BK) { kk = e & (MK_KC - 1); jj = e >> 4; }
@@ -69,7 +77,7 @@ __device__ __forceinline__ void mk_accum(const MkOps<AK, BK, TE> &op, int M, int
             const long gk2 = kc + kk;
             const int gj = j0 + jj;
             pb[q] = (gj < N && gk2 < k1 && (!TRI || gk2 <= gj))
-                        ? (double)(BK ? op.B[gk2 + (long)gj * op.ldb] : op.B[gj + gk2 * op.ldb])
+                        ? mk_load<COH>(BK ? op.B + gk2 + (long)gj * op.ldb : op.B + gj + gk2 * op.ldb)
                         : 0.0;
         }
     };

@@ -298,10 +298,14 @@ __device__ int diag_factor_blk(double *Lr, double *Wc, double *Ts, int *s_bad)
 // worker, the first workgroup to start elects its XCD (hardware register
 // XCC_ID) and workgroups on other XCDs leave at once.  Publishing a block:
 // its stores, a wait in every thread until they have completed (the vector L1
-// writes through to L2), a barrier and the done flag; reading: the flags,
-// one invalidation of this CU's L1 for all dependencies already done, a
-// barrier.  No L2 write-back or invalidation is needed (an agent-scope fence
-// would write back or drop the whole L2, which the concurrent kernels use).
+// writes through to L2), a barrier and the done flag; reading: the flags, a
+// barrier, then loads past this CU's L1 (agent scope: MkOps COH, mk_load), so
+// a line that an earlier read brought into the L1 before its other part was
+// written is never used, wherever blocks begin within a line.  No L2 write-back or
+// invalidation is needed (an agent-scope fence would write back or drop the
+// whole L2, which the concurrent kernels use).  One launch alone on the
+// device: 0.333 ms at NB 270 and 1.34 ms at NB 900, against 0.332 and 1.32 ms
+// with loads through the L1.
 // The kernel's end publishes the results to other XCDs as every kernel end
 // does.
 #define DAG_SPIN_LIMIT (1 << 21)
@@ -312,8 +316,8 @@ __device__ __forceinline__ int dag_fac(int i, int j, int nb) { return j * nb + (
 __device__ __forceinline__ int dag_inv(int i, int j, int nb) { return i * nb + (nb - i) + j; }
 
 // Waits until tasks t0(l) and t1(l) are done, then counts how many of the
-// following chunks l+1 .. lend-1 are done as well, and acquires once for all
-// of them.  Returns the first chunk not yet acquired.  dep(l, &a, &b) names
+// following chunks l+1 .. lend-1 are done as well.  Returns the first chunk
+// not known to be done.  dep(l, &a, &b) names
 // chunk l's two tasks.
 template <typename Dep>
 __device__ __forceinline__ int dag_acquire(int *flags, int l, int lend, Dep dep, int *err)
@@ -336,8 +340,6 @@ __device__ __forceinline__ int dag_acquire(int *flags, int l, int lend, Dep dep,
         }
         int r = l + 1;
         while (r < lend && done(r)) r++;
-        // drop this CU's L1 copies: the blocks are read from the XCD's L2
-        asm volatile("buffer_inv sc0\n\ts_waitcnt vmcnt(0)" ::: "memory");
         s_ready = r;
     }
     __syncthreads();
@@ -400,7 +402,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
             for (int l = j; l < i; l++) {
                 if (l >= ready) ready = dag_acquire(flags, l, i, dep, err);
                 const double *blk = (l == j) ? Winv + (size_t)j * PBK * PBK : Linv + ((size_t)l * nb + j) * PBK * PBK;
-                const MkOps<false, true> op{A + r0, NB, blk - (long)PBK * l, PBK};
+                const MkOps<false, true, double, true> op{A + r0, NB, blk - (long)PBK * l, PBK};
                 mk_accum(op, ri, cj, 0, 0, (long)PBK * l, (long)PBK * l + PBK, acc, Mk);
             }
             mk_store(acc, [&](int ii, int jj, double v) { Lr[ii * PLR + jj] = v; });  // S(ii, jj)
@@ -408,7 +410,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
             const double *Wi = Winv + (size_t)i * PBK * PBK;
             for (int e = tid; e < PBK * PBK; e += BS) {
                 const int ii = e % PBK, l = e / PBK;  // W_i(ii, l), column major
-                Wc[ii * PLR + l] = (ii < ri && l < ri) ? Wi[ii + l * PBK] : 0.0;
+                Wc[ii * PLR + l] = (ii < ri && l < ri) ? mk_load<true>(Wi + ii + l * PBK) : 0.0;
             }
             __syncthreads();
             // Linv_ij(ii, c) = -sum_{l <= ii} W_i(ii, l) S(l, c); thread: row ii, columns cg + 4 q
@@ -423,7 +425,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
             }
         } else {
             // S = A_ij - sum_l L_il L_jl^T
-            const MkOps<false, false> op{A + r0, NB, A + c0, NB};
+            const MkOps<false, false, double, true> op{A + r0, NB, A + c0, NB};
             auto dep = [&](int c, int &a, int &b) {
                 a = dag_fac(i, c, nb);
                 b = dag_fac(j, c, nb);
@@ -464,7 +466,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
                 const double *Wj = Winv + (size_t)j * PBK * PBK;
                 for (int e = tid; e < PBK * PBK; e += BS) {
                     const int ii = e % PBK, c = e / PBK;  // W(ii, c), column major
-                    Wc[c * PLR + ii] = (ii < cj && c < cj) ? Wj[ii + c * PBK] : 0.0;
+                    Wc[c * PLR + ii] = (ii < cj && c < cj) ? mk_load<true>(Wj + ii + c * PBK) : 0.0;
                 }
                 __syncthreads();
                 // L_ij(ii, c) = sum_{l <= c} S(ii, l) W(c, l); thread: row ii, columns cg + 4 q
