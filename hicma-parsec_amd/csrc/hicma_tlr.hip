@@ -5,7 +5,6 @@
 // every task of a step; tile ranks never leave HBM (kernels read them).
 #include "internal.hpp"
 #include "tlr_kernels.hpp"
-#include "rc_fast.hpp"
 #include "rc_wave.hpp"
 
 #include <math.h>
@@ -711,58 +710,59 @@ extern "C" int parsec_band_regenerate(hicma_ctx *ctx, int uplo, hicma_tlr_desc *
 // low-rank x dense gemm (W, X per pair), recompression slots of the
 // persistent grids (sized for the context's CUs), task lists.
 struct PotrfWs {
-    RcWs g;
-    int ns, nsf, wgrid, wres, wcap;
-    bool fast, wave;
-    size_t rc_lds, fstride, winv_d, dag_d, linv_d, tasks_d, wws_d, wbs_d, wlist_d, lrd_pairs, syrk_d, lrd_d, qn_d,
-        total;
+    RcWs g;     // k_lr_gemm (tiles k_rc_big does not take)
+    RbWs gb;    // k_rc_big
+    int ns, nbig, wgrid, wres, wcap;
+    bool big, wave;
+    size_t rc_lds, winv_d, dag_d, linv_d, wws_d, wlist_d, lrd_pairs, syrk_d, lrd_d, qn_d, total;
 };
 
 static void plan_potrf_ws(hicma_ctx *ctx, int NT, int NB, int cap, int b, PotrfWs &P)
 {
     RcWs &g = P.g;
+    const long long maxtask = std::max(1LL, (long long)(NT - 1) * (NT - 2) / 2);
+    P.big = rb_fits(NB, cap);
     g.smax = 2 * cap;
-    g.stride = rc_slot_doubles(NB, cap);
+    g.stride = P.big ? 0 : rc_slot_doubles(NB, cap);
     size_t lds_fixed = sizeof(double) * (RC_FIXED_SMEM + 2 * (size_t)g.smax + 8);
     size_t lds_avail = ctx->lds_max > lds_fixed ? ctx->lds_max - lds_fixed : 0;
     int jl = (int)floor(sqrt((double)(lds_avail / sizeof(double)) / 2.0));
     if (jl > g.smax) jl = g.smax;
     g.jlds = jl;
     P.rc_lds = lds_fixed + sizeof(double) * 2 * (size_t)jl * jl;
-    long long maxtask = (long long)(NT - 1) * (NT - 2) / 2;
-    P.ns = nslots_for(ctx, g.stride * sizeof(double), maxtask > 0 ? maxtask : 1);
+    P.ns = P.big ? 0 : nslots_for(ctx, g.stride * sizeof(double), maxtask);
+    // one workgroup per CU (the LDS it takes), each with its own slot
+    P.gb.smax = 2 * cap;
+    P.gb.stride = P.big ? rb_slot_doubles(NB, cap) : 0;
+    P.nbig = P.big ? std::min(ctx->ncu, nslots_for(ctx, P.gb.stride * sizeof(double), maxtask)) : 0;
     P.syrk_d = (size_t)NT * NB * cap + (size_t)NT * cap * cap;
     P.lrd_pairs = (b > 1) ? (size_t)NT * (b - 1) : 0;
     P.lrd_d = P.lrd_pairs * ((size_t)cap * NB + (size_t)cap * cap);
-    // fast recompression path (1024 threads, one row per thread)
-    P.fast = (NB <= FT);
-    P.fstride = rcf_slot_doubles(NB);
-    P.nsf = P.fast ? nslots_for(ctx, P.fstride * sizeof(double), maxtask > 0 ? maxtask : 1) : 0;
-    if (P.nsf > ctx->ncu) P.nsf = ctx->ncu;
-    P.tasks_d = ((size_t)(maxtask > 0 ? maxtask : 1) + 1) / 2 + 1;  // ints packed in doubles
     P.winv_d = (size_t)((NB + PBK - 1) / PBK) * PBK * PBK;
     // the diagonal potrf's task counter and done flags (ints packed in
     // doubles) and the blocks of L_kk^-1
     const size_t nbk = (size_t)((NB + PBK - 1) / PBK);
     P.dag_d = (nbk * nbk + 2 + 1) / 2 + 1;
     P.linv_d = nbk * nbk * PBK * PBK;
-    // one-wave recompression (tasks with s <= WV_SMAX): the s <= 32 and
+    // one-wave recompression (tasks with s <= WV_S2MAX): the s <= 32 and
     // s <= 48 variants run 4 waves per workgroup, s <= 64 two
-    P.wave = (NB <= 64 * WV_KMAX);
+    P.wave = P.big && (NB <= 64 * WV_KMAX);
     P.wgrid = P.wave ? ctx->ncu : 0;  // times WvCfg<SM>::BPC resident workgroups
     // CUs left to the lookahead stream (syrk(k) + potrf(k+1)) while the
     // recompression kernels of step k run
     P.wres = (P.wave && ctx->ncu > 64 && ctx->ncu == ctx->ncu_dev) ? 16 : 0;
-    P.wcap = (int)(maxtask > 0 ? maxtask : 1);
-    // four concurrent variants (32, 48, 64 on side streams), each with up to
-    // four resident waves per CU: one quarter of the region each
-    P.wws_d = (size_t)4 * P.wgrid * 4 * wv_slot_doubles(NB);
-    P.wbs_d = P.wave ? (size_t)P.wgrid * wb_slot_doubles(NB) : 0;  // one wide-stack wave per CU
-    P.wlist_d = ((size_t)4 * P.wcap + 8) / 2 + 1;
-    // Qn = -B Av of the dense-B tasks the wave kernels take (2-flow only)
+    P.wcap = (int)maxtask;
+    // three concurrent variants, each with up to four resident waves per CU
+    P.wws_d = (size_t)3 * P.wgrid * 4 * wv_slot_doubles(NB);
+    P.wlist_d = P.big ? ((size_t)5 * P.wcap + 16) / 2 + 1 : 0;
+    // Qn = -B Av of the dense-B tasks with stacks up to QN_COLS (2-flow only)
     P.qn_d = (P.wave && b > 1) ? (size_t)(b - 1) * (NT - 1) * NB * QN_COLS : 0;
-    P.total = g.stride * P.ns + P.syrk_d + P.lrd_d + P.fstride * P.nsf + P.tasks_d + P.winv_d + P.wws_d +
-              P.wlist_d + P.wbs_d + P.dag_d + P.linv_d + P.qn_d;
+    // every part on a 128-byte line
+    for (size_t *d : {&g.stride, &P.gb.stride, &P.syrk_d, &P.lrd_d, &P.winv_d, &P.dag_d, &P.linv_d, &P.wws_d,
+                      &P.wlist_d, &P.qn_d})
+        *d = (*d + 15) / 16 * 16;
+    P.total = g.stride * P.ns + P.gb.stride * P.nbig + P.syrk_d + P.lrd_d + P.winv_d + P.wws_d + P.wlist_d + P.dag_d +
+              P.linv_d + P.qn_d;
 }
 
 // Device bytes a generation + factorization of this shape allocates on the
@@ -868,28 +868,26 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
 
     PotrfWs P;
     plan_potrf_ws(ctx, NT, NB, cap, b, P);
-    RcWs &g = P.g;
-    const int ns = P.ns, nsf = P.nsf, wgrid = P.wgrid, wres = P.wres, wcap = P.wcap;
-    const bool fast = P.fast, wave = P.wave;
-    const size_t rc_lds = P.rc_lds, fstride = P.fstride, winv_d = P.winv_d, tasks_d = P.tasks_d, wws_d = P.wws_d,
-                 wlist_d = P.wlist_d, lrd_pairs = P.lrd_pairs, total = P.total;
-    int rc = hicma_ensure_ws(ctx, total * sizeof(double));
+    const int wgrid = P.wgrid, wres = P.wres, wcap = P.wcap;
+    const bool big = P.big, wave = P.wave;
+    int rc = hicma_ensure_ws(ctx, P.total * sizeof(double));
     if (rc) return rc;
-    double *rcws = ctx->ws;
-    double *Yws = rcws + g.stride * ns;
+    double *rcws = ctx->ws;                           // k_rc_big's (or k_lr_gemm's) slots
+    double *Yws = rcws + P.g.stride * P.ns + P.gb.stride * P.nbig;
     double *Zws = Yws + (size_t)NT * NB * cap;
-    double *Wws = Zws + (size_t)NT * cap * cap;
-    double *Xws = Wws + lrd_pairs * cap * NB;
-    double *fws = Xws + lrd_pairs * cap * cap;
-    double *Winv = fws + fstride * nsf;
-    int *tasks_s = (int *)(Winv + winv_d);
-    double *wws = Winv + winv_d + tasks_d;
-    int *wcount = (int *)(wws + wws_d);
-    int *wlist = wcount + 8;  // counts [0..3], next-task counters [4..7]
-    double *wbs = (double *)wcount + wlist_d;
-    double *Linv = wbs + P.wbs_d;
+    double *Wws = Yws + P.syrk_d;
+    double *Xws = Wws + P.lrd_pairs * cap * NB;
+    double *Winv = Wws + P.lrd_d;
+    double *wws = Winv + P.winv_d;
+    int *wcount = (int *)(wws + P.wws_d);             // 16 counters (k_classify_wave)
+    int *wlist = wcount + 16;
+    double *Linv = (double *)wcount + P.wlist_d;
     double *qnws = P.qn_d ? Linv + P.linv_d : nullptr;
     int *dflags = (int *)(Linv + P.linv_d + P.qn_d);
+    const size_t big_lds = sizeof(double) * WQ_LDS;
+    // tiles (and stacks) of up to 256, 512, 1024, 2048: 1, 2, 4, 8 rows per thread in k_rc_big's panels
+    const int hi = std::max(NB, 2 * cap);
+    const auto rc_big = hi <= 256 ? k_rc_big<1> : (hi <= 512 ? k_rc_big<2> : (hi <= 1024 ? k_rc_big<4> : k_rc_big<8>));
     HIPCHK(hipFuncSetAttribute((const void *)k_potrf_dag, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)(sizeof(double) * DAG_SMEM)));
     if (!trsm_tc(NB)) return HICMA_ERR_ARG;
@@ -901,10 +899,8 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                                (int)TRSM_LDS_MAX));
     HIPCHK(hipFuncSetAttribute((const void *)k_trsm_lr_inv<2>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)TRSM_LDS_MAX));
-    if (fast)
-        HIPCHK(hipFuncSetAttribute((const void *)k_lr_gemm_fast, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(RCF_LDS * sizeof(double))));
-    HIPCHK(hipFuncSetAttribute((const void *)k_lr_gemm, hipFuncAttributeMaxDynamicSharedMemorySize, (int)rc_lds));
+    if (big) HIPCHK(hipFuncSetAttribute((const void *)rc_big, hipFuncAttributeMaxDynamicSharedMemorySize, (int)big_lds));
+    else HIPCHK(hipFuncSetAttribute((const void *)k_lr_gemm, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.rc_lds));
     const size_t wlds32 = sizeof(double) * WvCfg<32>::LDS * WvCfg<32>::WPB;
     const size_t wlds48 = sizeof(double) * WvCfg<48>::LDS * WvCfg<48>::WPB;
     const size_t wlds64 = sizeof(double) * WvCfg<64>::LDS * WvCfg<64>::WPB;
@@ -915,8 +911,6 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                                    (int)wlds48));
         HIPCHK(hipFuncSetAttribute((const void *)k_rc_wave<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                    (int)wlds64));
-        HIPCHK(hipFuncSetAttribute((const void *)k_rc_wide, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)(sizeof(double) * WB_LDS)));
     }
 
     // critical-path timing (hicma_parsec/HiCMA_dpotrf_L_2flow_wrapper.c:27-166):
@@ -1025,61 +1019,66 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         int T = NT - 1 - k;
         long long ntask = (long long)T * (T - 1) / 2;
         if (ntask > 0 && T > b) {
-            int grid = (int)std::min<long long>(ns, ntask);
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (ctx->profile) {
                 HIPCHK(hipEventCreate(&e0));
                 HIPCHK(hipEventCreate(&e1));
                 HIPCHK(hipEventRecord(e0, st));
             }
-            hipLaunchKernelGGL(k_classify, dim3((unsigned)((ntask + 255) / 256)), dim3(256), 0, st, t, k, tasks_s);
-            if (wave) {
-                hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, wcount, 8, 0);
-                const int wide_only = (ntask < ctx->wave_min_tasks) ? 1 : 0;
+            if (big) {
+                hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, wcount, 16, 0);
+                const int big_only = (!wave || ntask < ctx->wave_min_tasks) ? 1 : 0;
                 if (qnws) {
                     const int nrt = (NB + GT - 1) / GT;
                     hipLaunchKernelGGL(k_qn_dense, dim3(nrt * (QN_COLS / GT), (unsigned)((b - 1) * T)), dim3(BS), 0,
                                        st, t, k, qnws);
                 }
                 hipLaunchKernelGGL(k_classify_wave, dim3((unsigned)((ntask + 255) / 256)), dim3(256), 0, st, t, k,
-                                   tasks_s, wlist, wcount, wcap, wide_only, qnws ? 1 : 0);
-                // fork: the wide variant and variant 64 on side streams 1 and 0,
+                                   wlist, wcount, wcap, big_only, qnws ? 1 : 0);
+                // fork: k_rc_big and variant 64 on side streams 1 and 0,
                 // variants 48 and 32 on the context stream.  Launched longest
                 // tasks first: the dispatcher hands out CUs in launch order, so
                 // the long tasks start at once and the short ones fill the
                 // step's tail.
                 HIPCHK(hipEventRecord(ctx->ev_fork, st));
                 for (int i = 0; i < 2; i++) HIPCHK(hipStreamWaitEvent(ctx->side[i], ctx->ev_fork, 0));
-                int wg = (int)std::min<long long>(wgrid - wres, ntask);
-                hipLaunchKernelGGL(k_rc_wide, dim3(wg), dim3(64 * WB_WAVES), sizeof(double) * WB_LDS, ctx->side[1], t, k,
-                                   (const int *)(wlist + 3 * (size_t)wcap), (const int *)(wcount + 3), wcount + 7,
-                                   tasks_s, wbs, acc, fixed_rank, maxrank, o1, ctx->d_ovf, (const double *)qnws);
-                wg = (int)std::min<long long>((wgrid - wres) * WvCfg<64>::BPC, (ntask + WvCfg<64>::WPB - 1) / WvCfg<64>::WPB);
-                hipLaunchKernelGGL(k_rc_wave<64>, dim3(wg), dim3(64 * WvCfg<64>::WPB), wlds64, ctx->side[0], t, k,
-                                   (const int *)(wlist + 2 * (size_t)wcap), (const int *)(wcount + 2), wcount + 6,
-                                   tasks_s, wws + wws_d / 2, acc, fixed_rank, maxrank, o0, ctx->d_ovf,
-                                   (const double *)qnws);
-                wg = (int)std::min<long long>((wgrid - wres) * WvCfg<48>::BPC, (ntask + WvCfg<48>::WPB - 1) / WvCfg<48>::WPB);
-                hipLaunchKernelGGL(k_rc_wave<48>, dim3(wg), dim3(64 * WvCfg<48>::WPB), wlds48, st, t, k,
-                                   (const int *)(wlist + wcap), (const int *)(wcount + 1), wcount + 5, tasks_s,
-                                   wws + wws_d / 4, acc, fixed_rank, maxrank, o, ctx->d_ovf, (const double *)qnws);
-                wg = (int)std::min<long long>((wgrid - wres) * WvCfg<32>::BPC, (ntask + WvCfg<32>::WPB - 1) / WvCfg<32>::WPB);
-                hipLaunchKernelGGL(k_rc_wave<32>, dim3(wg), dim3(64 * WvCfg<32>::WPB), wlds32, st, t, k,
-                                   (const int *)wlist, (const int *)wcount, wcount + 4, tasks_s, wws, acc, fixed_rank,
-                                   maxrank, o, ctx->d_ovf, (const double *)qnws);
+                int *redo = wlist + 4 * (size_t)wcap;
+                int wg = (int)std::min<long long>(wave ? std::min(P.nbig, wgrid - wres) : P.nbig, ntask);
+                hipLaunchKernelGGL(rc_big, dim3(wg), dim3(BS), big_lds, ctx->side[1], t, k,
+                                   (const int *)(wlist + 3 * (size_t)wcap), (const int *)(wcount + 3), wcount + 7, rcws,
+                                   P.gb, acc, fixed_rank, maxrank, o1, ctx->d_ovf, (const double *)qnws);
+                if (wave) {
+                    const size_t wr = P.wws_d / 3;
+                    wg = (int)std::min<long long>((wgrid - wres) * WvCfg<64>::BPC, (ntask + WvCfg<64>::WPB - 1) / WvCfg<64>::WPB);
+                    hipLaunchKernelGGL(k_rc_wave<64>, dim3(wg), dim3(64 * WvCfg<64>::WPB), wlds64, ctx->side[0], t, k,
+                                       (const int *)(wlist + 2 * (size_t)wcap), (const int *)(wcount + 2), wcount + 6,
+                                       redo, wcount + 8, wws + 2 * wr, acc, fixed_rank, maxrank, o0, ctx->d_ovf,
+                                       (const double *)qnws);
+                    wg = (int)std::min<long long>((wgrid - wres) * WvCfg<48>::BPC, (ntask + WvCfg<48>::WPB - 1) / WvCfg<48>::WPB);
+                    hipLaunchKernelGGL(k_rc_wave<48>, dim3(wg), dim3(64 * WvCfg<48>::WPB), wlds48, st, t, k,
+                                       (const int *)(wlist + wcap), (const int *)(wcount + 1), wcount + 5, redo,
+                                       wcount + 8, wws + wr, acc, fixed_rank, maxrank, o, ctx->d_ovf,
+                                       (const double *)qnws);
+                    wg = (int)std::min<long long>((wgrid - wres) * WvCfg<32>::BPC, (ntask + WvCfg<32>::WPB - 1) / WvCfg<32>::WPB);
+                    hipLaunchKernelGGL(k_rc_wave<32>, dim3(wg), dim3(64 * WvCfg<32>::WPB), wlds32, st, t, k,
+                                       (const int *)wlist, (const int *)wcount, wcount + 4, redo, wcount + 8, wws, acc,
+                                       fixed_rank, maxrank, o, ctx->d_ovf, (const double *)qnws);
+                }
                 // join
                 for (int i = 0; i < 2; i++) {
                     HIPCHK(hipEventRecord(ctx->ev_join[i], ctx->side[i]));
                     HIPCHK(hipStreamWaitEvent(st, ctx->ev_join[i], 0));
                 }
+                // tasks a wave kernel could not vouch for
+                if (wave)
+                    hipLaunchKernelGGL(rc_big, dim3((unsigned)std::min<long long>(P.nbig, std::min<long long>(ntask, 32))),
+                                       dim3(BS), big_lds, st, t, k, (const int *)redo, (const int *)(wcount + 8),
+                                       wcount + 9, rcws, P.gb, acc, fixed_rank, maxrank, o, ctx->d_ovf,
+                                       (const double *)qnws);
+            } else {
+                hipLaunchKernelGGL(k_lr_gemm, dim3((unsigned)std::min<long long>(P.ns, ntask)), dim3(BS), P.rc_lds, st, t,
+                                   k, rcws, P.g, acc, fixed_rank, maxrank, o, ctx->d_ovf);
             }
-            if (fast) {
-                int gf = (int)std::min<long long>(nsf, ntask);
-                hipLaunchKernelGGL(k_lr_gemm_fast, dim3(gf), dim3(FT), RCF_LDS * sizeof(double), st, t, k,
-                                   tasks_s, fws, fstride, acc, fixed_rank, maxrank, o, ctx->d_ovf);
-            }
-            hipLaunchKernelGGL(k_lr_gemm, dim3(grid), dim3(BS), rc_lds, st, t, k, (const int *)tasks_s,
-                               fast ? FS : -1, rcws, g, acc, fixed_rank, maxrank, o, ctx->d_ovf);
             if (ctx->profile) {
                 HIPCHK(hipEventRecord(e1, st));
                 ctx->prof_ev.push_back(e0);

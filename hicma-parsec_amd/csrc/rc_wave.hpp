@@ -20,13 +20,12 @@
 // Layout: lane l holds rows l, l+64, ... of every tall (NB-row) operand, so
 // tall data is read and written coalesced and row-locally.
 #pragma once
-#include "tlr_kernels.hpp"
+#include "rc_big.hpp"
 
 #define WV_SMAX 64   // largest stack width s = rc + ra, and largest rb
 #define WV_KMAX 16   // rows per lane: NB <= 64 * WV_KMAX
 #define WV_PW 4      // Householder panel width
-#define WV_S2MAX 60  // widest stack of list 2 (k_rc_wave<64>); wider stacks go to the
-                     // four-wave k_rc_wide, which balances the two side streams
+#define WV_S2MAX 60  // widest stack of list 2 (k_rc_wave<64>); wider stacks go to k_rc_big
 
 
 // Per-variant sizes: SM = largest stack width of the variant (32, 48 or 64).
@@ -44,12 +43,6 @@ struct WvCfg {
 __host__ __device__ inline size_t wv_slot_doubles(int NB)
 {
     return (size_t)NB * 4 * WV_SMAX + 4 * (size_t)WV_SMAX * WV_SMAX;
-}
-
-__device__ __forceinline__ double rdlane(double v, int l)
-{
-    return mk64((unsigned)__builtin_amdgcn_readlane((int)lo32(v), l),
-                (unsigned)__builtin_amdgcn_readlane((int)hi32(v), l));
 }
 
 __device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -299,14 +292,6 @@ __device__ __forceinline__ double wrsN(double (&p)[N])
     else return wrs16(p);
 }
 
-// Squared-norm floor below which a Jacobi pair is not rotated (see k_rc_wave).
-__device__ __forceinline__ double wv_skip_floor(double f2, int s, double acc, int fixed_rk)
-{
-    const double nz = (2.3e-16 * s) * (2.3e-16 * s) * f2;
-    const double tz = (fixed_rk > 0 || !(acc > 0.0)) ? 0.0 : (1e-3 * acc) * (1e-3 * acc);
-    return fmax(nz, tz);
-}
-
 // Buffer resources of the columns of a stack [src0 (c0 columns) | src1] in
 // its first pass and of the workspace W afterwards (the fields are plain
 // scalars: no indexed access to a structure in private memory).
@@ -503,16 +488,6 @@ __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const doub
     }
 }
 
-// Dense-B tasks (case iv: tile (n, k) in the band, (m, k) and (m, n) low
-// rank) get Qn = -B Av precomputed by k_qn_dense into a slot of QN_COLS
-// columns: slot (n - k - 1) T + (m - k - 1), T = NT - 1 - k.
-#define QN_COLS 128
-__host__ __device__ inline size_t qn_slot(int NT, int NB, int k, int m, int n)
-{
-    const int T = NT - 1 - k;
-    return ((size_t)(n - k - 1) * T + (size_t)(m - k - 1)) * NB * QN_COLS;
-}
-
 // Qn = -B Av for the dense-B tasks of step k that the wave kernels take
 // (ra > 0, s <= 128); grid (64x64 tiles of an NB x 128 slot, (band - 1) T).
 __global__ void __launch_bounds__(BS) k_qn_dense(TLR t, int k, double *qn)
@@ -531,15 +506,15 @@ __global__ void __launch_bounds__(BS) k_qn_dense(TLR t, int k, double *qn)
                             qn + qn_slot(NT, NB, k, m, n), NB, sm);
 }
 
-// Tasks of step k whose update runs on one wave: both factors low rank,
-// s = rc + ra in [1, 128], rb <= WV_SMAX, NB <= 64 * WV_KMAX.  They are
-// appended to list 0 (s, rb <= 32), 1 (<= 48), 2 (s <= WV_S2MAX) or 3 (s <= 128,
-// rb <= WV_SMAX: k_rc_wide); the order inside
-// a list is irrelevant (tasks of one step are independent).  Listed tasks are
-// marked -1 in tasks_s; every other task keeps its k_classify value.  With
-// wide_only, every listed task goes to list 3 (four waves per task).
-__global__ void k_classify_wave(TLR t, int k, int *tasks_s, int *wlist, int *wcount, int cap, int wide_only,
-                                int qn_dense)
+// Sorts the low-rank results of step k into task lists (the order inside a
+// list is irrelevant: tasks of one step are independent): 0 (s, rb <= 32),
+// 1 (<= 48), 2 (s <= WV_S2MAX, rb <= WV_SMAX) run on one wave each; 3, every other
+// task, on one workgroup each (k_rc_big).  A dense B (band tile) needs its
+// Qn = -B Av from k_qn_dense to run on a wave.  With big_only every task goes to
+// list 3.  A low-rank update by a rank-0 factor changes nothing and is skipped.
+// wcount: [0..3] list lengths, [4..7] next-task counters, [8] length and [9]
+// next task of the redo list (list 4).
+__global__ void k_classify_wave(TLR t, int k, int *wlist, int *wcount, int cap, int big_only, int qn_dense)
 {
     const int T = t.NT - 1 - k;
     const long long ntask = (long long)T * (T - 1) / 2;
@@ -548,17 +523,15 @@ __global__ void k_classify_wave(TLR t, int k, int *tasks_s, int *wlist, int *wco
     int hi, lo;
     tri_decode(e, hi, lo);
     const int m = k + 1 + hi, n = k + 1 + lo, b = t.band_size;
-    if (m - n < b || t.NB > 64 * WV_KMAX) return;
-    // a dense B (band tile) comes with its Qn = -B Av formed by k_qn_dense
+    if (m - n < b) return;
     const bool bdense = (n - k < b);
-    if (bdense && !qn_dense) return;
     const int ra = *rank_at(t, m, k), rc = *rank_at(t, m, n), rb = bdense ? 0 : *rank_at(t, n, k);
     const int s = rc + ra;
-    if (ra > 0 && (bdense || rb > 0) && s <= 128 && rb <= WV_SMAX) {
-        const int l = wide_only ? 3 : ((s <= 32 && rb <= 32) ? 0 : ((s <= 48 && rb <= 48) ? 1 : (s <= WV_S2MAX ? 2 : 3)));
-        tasks_s[e] = -1;
-        wlist[(size_t)l * cap + atomicAdd(wcount + l, 1)] = (int)e;
-    }
+    if (ra < 0 || rb < 0 || rc < 0 || (!bdense && (ra == 0 || rb == 0))) return;
+    int l = 3;
+    if (!big_only && ra > 0 && (!bdense || qn_dense))
+        l = (s <= 32 && rb <= 32) ? 0 : ((s <= 48 && rb <= 48) ? 1 : (s <= WV_S2MAX && rb <= WV_SMAX ? 2 : 3));
+    wlist[(size_t)l * cap + atomicAdd(wcount + l, 1)] = (int)e;
 }
 
 // One-sided Jacobi on the rows of M (lane c owns row c of M in xm, zero
@@ -632,7 +605,7 @@ __device__ __forceinline__ double wv_jacobi(double (&xm)[SM], int s, double acc,
 
 template <int SM>
 __global__ void __launch_bounds__(64 * WvCfg<SM>::WPB, WvCfg<SM>::MINW)
-k_rc_wave(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *tasks_s, double *ws, double acc,
+k_rc_wave(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *redo, int *nredo, double *ws, double acc,
           int fixed_rk, int maxrank, OpLog o, int *ovf, const double *qn_dense)
 {
     using Cf = WvCfg<SM>;
@@ -870,7 +843,7 @@ k_rc_wave(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *ta
             // j then errs in the tile by at most
             // sigma_j s eps max_q sum_l |Rq(q,l)| |Kv(l,j)|; a task over the
             // tolerance, or with an exactly zero pivot, is left untouched and
-            // handed to the Householder path (k_lr_gemm).
+            // handed to the Householder path (k_rc_big).
             // Row q of Rq is loaded across the lanes (lane l: Rq(q, l), one
             // load per row, the next row's issued ahead) and read by readlane.
             bool bad = false;
@@ -897,7 +870,7 @@ k_rc_wave(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *ta
                 bad = lane < nr && (bad || !(sgp[lane] * s * 2.3e-16 * gmax <= rc_solve_tol(acc, fixed_rk, fro)));
             }
             if (__ballot(bad) != 0) {
-                if (lane == 0) tasks_s[e] = RC_REDO;
+                if (lane == 0) redo[atomicAdd(nredo, 1)] = e;
                 wv_sync();
                 continue;
             }
@@ -938,590 +911,8 @@ k_rc_wave(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *ta
         if (lane == 0) {
             *rank_at(t, m, n) = nr;
             rank_hist(o, NT, m, n, nr);
-            unsigned long long mm = tdim(t, m), ss = s;
-            unsigned long long qa = opc('q', mm, ss, 0, 0);
-            // case iv (dense B) counts the product B Av, case v the products with B's factors
-            unsigned long long qb = bdense ? opc('q', mm, ss, 0, 0) + opc('m', ra, mm, mm, 0)
-                                           : opc('m', ra, rb, mm, 0) + opc('m', ra, mm, rb, 0) + opc('q', mm, ss, 0, 0);
-            unsigned long long sv = opc('r', ss, ss, 2, 0) + opc('s', ss, 0, 0, 0) + ss * nr;
-            unsigned long long nu = opc('o', mm, nr, ss, 1), nv = opc('o', nr, mm, ss, 2);
-            oplog(o, NT, qa + qb + sv + nu + nv, m, n, false, false);
-            atomicAdd(o.stat + 4, qa + qb + sv + nu + nv);
-            atomicAdd(o.stat + 5, 1ULL);
-            unsigned long long words =
-                2ULL * NB * (ra + rc + nr) + (bdense ? (unsigned long long)NB * NB : 2ULL * NB * rb);
-            atomicAdd(o.stat + 6, 8ULL * words);
+            rc_oplog(o, t, m, n, ra, rb, rc, nr, bdense);
         }
         wv_sync();
-    }
-}
-
-// ===================== stacks wider than 64 (s <= 128) =====================
-
-#define WB_SM 128                       // largest stack width of the wide variant
-#define WB_LD (WB_SM + 1)               // LDS column stride of the Jacobi matrix
-#define WB_LDS (WB_SM * WB_LD + 3 * WB_SM)  // doubles of LDS (one workgroup per CU)
-#define WB_QR_SH (64 * (WV_KMAX * WV_PW + 1))  // doubles of LDS per QR side (two sides fit in WB_LDS)
-
-__host__ __device__ inline size_t wb_slot_doubles(int NB)
-{
-    return (size_t)NB * 4 * WB_SM + 3 * (size_t)WB_SM * WB_SM;
-}
-
-// wv_geqrf_r for s <= 128 on two waves: pivot row j lives on lane j & 63 of
-// row block j >> 6 (0 or 1); rows of block 0 are above every pivot of block 1.
-// The lead wave (part 0) factors each panel and passes its reflectors and T
-// to the helper (part 1) through `sh` (64 (16 WV_PW + 1) doubles of LDS);
-// the two then update alternate trailing columns.  Every wave of the
-// workgroup must call it with the same s (the barriers are workgroup-wide).
-// R is written column-major (R(i, j) at Rout[i + j * WB_SM]).
-__device__ __forceinline__ void wb_geqrf_r(int s, const double *src0, const double *src1, int c0, double *W, int NB,
-                                           double *Rout, int part, double *sh)
-{
-    const int lane = threadIdx.x & 63;
-    const WvRs A{src0, src1, W, c0, NB};
-    for (int j0 = 0; j0 < s; j0 += WV_PW) {
-        const int jb = min(WV_PW, s - j0);
-        const bool first = (j0 == 0);
-        const int ps = j0 >> 6;  // row block of the panel's pivots (panels never straddle 64)
-        double a[WV_KMAX][WV_PW];
-        double T[WV_PW][WV_PW];
-        double m0[WV_PW], m1[WV_PW];
-        // this wave's trailing columns t0, t0 + 2, ... in two register sets
-        // used in turn (the next column loads while the current one updates)
-        const int t0 = j0 + jb + part;
-        double p_[WV_KMAX], q_[WV_KMAX];
-        if (part == 0) {
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                const wv_rsrc r = A.rd(j0 + c, first, c < jb);
-#pragma unroll
-                for (int k = 0; k < WV_KMAX; k++) a[k][c] = wv_ld(r, (lane + 64 * k) * 8);
-            }
-            wv_ld_col(p_, A.rd(t0, first, t0 < s), lane);
-#pragma unroll
-            for (int r = 0; r < WV_PW; r++)
-#pragma unroll
-                for (int c = 0; c < WV_PW; c++) T[r][c] = 0.0;
-#pragma unroll
-            for (int jj = 0; jj < WV_PW; jj++) {
-                if (jj < jb) {
-                    const int jl = (j0 + jj) & 63;
-                    const double x0 = a[0][jj], x1 = a[1][jj];
-                    // part of column jj strictly below the pivot, per row block
-                    const double y0 = (ps == 0 && lane > jl) ? x0 : 0.0;
-                    const double y1 = (ps == 0 || lane > jl) ? x1 : 0.0;
-                    double p[WV_PW];
-#pragma unroll
-                    for (int c = 0; c < WV_PW; c++)
-                        p[c] = y0 * (c == jj ? y0 : a[0][c]) + y1 * (c == jj ? y1 : a[1][c]);
-#pragma unroll
-                    for (int k = 2; k < WV_KMAX; k++)
-#pragma unroll
-                        for (int c = 0; c < WV_PW; c++) p[c] = fma(a[k][jj], a[k][c], p[c]);
-                    const double red = wrsN<WV_PW>(p);
-                    double S[WV_PW], prow[WV_PW];
-#pragma unroll
-                    for (int c = 0; c < WV_PW; c++) {
-                        S[c] = rdlane(red, (64 / WV_PW) * c);
-                        prow[c] = rdlane(ps ? a[1][c] : a[0][c], jl);
-                    }
-                    const double alpha = prow[jj], xn2 = S[jj];
-                    double tau = 0.0, beta = alpha, scal = 0.0;
-                    if (xn2 > 0.0) {
-                        beta = -copysign(sqrt(alpha * alpha + xn2), alpha);
-                        tau = (beta - alpha) / beta;
-                        scal = 1.0 / (alpha - beta);
-                    }
-                    const double v0 = (ps == 0 && lane == jl) ? 1.0 : y0 * scal;
-                    const double v1 = (ps == 1 && lane == jl) ? 1.0 : y1 * scal;
-                    a[0][jj] = v0;
-                    a[1][jj] = v1;
-#pragma unroll
-                    for (int k = 2; k < WV_KMAX; k++) a[k][jj] *= scal;
-#pragma unroll
-                    for (int c = 0; c < WV_PW; c++) {
-                        if (c > jj) {
-                            const double td = tau * (prow[c] + S[c] * scal);
-#pragma unroll
-                            for (int k = 0; k < WV_KMAX; k++) a[k][c] = fma(-td, a[k][jj], a[k][c]);
-                        }
-                    }
-                    // R entries above the pivot and beta at the pivot; reflector below
-                    if (ps == 0) {
-                        a[0][jj] = (lane == jl) ? beta : ((lane > jl) ? v0 : x0);
-                    } else {
-                        a[0][jj] = x0;
-                        a[1][jj] = (lane == jl) ? beta : ((lane > jl) ? v1 : x1);
-                    }
-#pragma unroll
-                    for (int l = 0; l < WV_PW; l++) {
-                        if (l < jj) {
-                            double acc = 0.0;
-#pragma unroll
-                            for (int q = 0; q < WV_PW; q++)
-                                if (q >= l && q < jj) acc = fma(T[l][q], prow[q] + S[q] * scal, acc);
-                            T[l][jj] = -tau * acc;
-                        }
-                    }
-                    T[jj][jj] = tau;
-                }
-            }
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++)
-                if (c < jb) {
-#pragma unroll
-                    for (int blk = 0; blk < 2; blk++) {
-                        const int i = lane + 64 * blk;
-                        if (i < s) Rout[i + (size_t)(j0 + c) * WB_SM] = (i <= j0 + c) ? a[blk][c] : 0.0;
-                    }
-                }
-            // reflector entries of row blocks 0 and 1 (1 at the pivot, 0 above)
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                const int gl = (j0 + c) & 63;
-                const bool in = c < jb;
-                m0[c] = (!in || ps == 1) ? 0.0 : ((lane == gl) ? 1.0 : (lane > gl ? a[0][c] : 0.0));
-                m1[c] = !in ? 0.0 : (ps == 0 ? a[1][c] : ((lane == gl) ? 1.0 : (lane > gl ? a[1][c] : 0.0)));
-            }
-
-            // the panel's reflectors and T for the helper wave (value-major:
-            // consecutive lanes, consecutive banks)
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                sh[(0 * WV_PW + c) * 64 + lane] = m0[c];
-                sh[(1 * WV_PW + c) * 64 + lane] = m1[c];
-#pragma unroll
-                for (int k = 2; k < WV_KMAX; k++) sh[(k * WV_PW + c) * 64 + lane] = a[k][c];
-            }
-            if (lane == 0) {  // T is the same on every lane
-#pragma unroll
-                for (int r = 0; r < WV_PW; r++)
-#pragma unroll
-                    for (int c = 0; c < WV_PW; c++) sh[WV_KMAX * WV_PW * 64 + r * WV_PW + c] = T[r][c];
-            }
-        }
-        __syncthreads();
-        if (part == 1) {
-            wv_ld_col(p_, A.rd(t0, first, t0 < s), lane);
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                m0[c] = sh[(0 * WV_PW + c) * 64 + lane];
-                m1[c] = sh[(1 * WV_PW + c) * 64 + lane];
-#pragma unroll
-                for (int k = 2; k < WV_KMAX; k++) a[k][c] = sh[(k * WV_PW + c) * 64 + lane];
-            }
-#pragma unroll
-            for (int r = 0; r < WV_PW; r++)
-#pragma unroll
-                for (int c = 0; c < WV_PW; c++) T[r][c] = sh[WV_KMAX * WV_PW * 64 + r * WV_PW + c];
-        }
-        // trailing columns j0 + jb + part, + 2, ...: the two waves of the
-        // side take alternate columns
-        auto upd = [&](double (&b)[WV_KMAX], int t) {
-            double p[WV_PW];
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                double acc = fma(m0[c], b[0], m1[c] * b[1]);
-#pragma unroll
-                for (int k = 2; k < WV_KMAX; k++) acc = fma(a[k][c], b[k], acc);
-                p[c] = acc;
-            }
-            const double red = wrsN<WV_PW>(p);
-            double d[WV_PW], w[WV_PW];
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) d[c] = rdlane(red, (64 / WV_PW) * c);
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                double acc = 0.0;
-#pragma unroll
-                for (int q = 0; q <= c; q++) acc = fma(T[q][c], d[q], acc);
-                w[c] = acc;
-            }
-#pragma unroll
-            for (int c = 0; c < WV_PW; c++) {
-                b[0] = fma(-m0[c], w[c], b[0]);
-                b[1] = fma(-m1[c], w[c], b[1]);
-            }
-#pragma unroll
-            for (int k = 2; k < WV_KMAX; k++) {
-                double acc = b[k];
-#pragma unroll
-                for (int c = 0; c < WV_PW; c++) acc = fma(-a[k][c], w[c], acc);
-                b[k] = acc;
-            }
-            wv_st_col(b, A.wr(t, true), lane);
-        };
-        for (int t = t0; t < s; t += 4) {
-            wv_ld_col(q_, A.rd(t + 2, first, t + 2 < s), lane);
-            upd(p_, t);
-            if (t + 2 >= s) break;
-            wv_ld_col(p_, A.rd(t + 4, first, t + 4 < s), lane);
-            upd(q_, t + 2);
-        }
-        __syncthreads();  // both waves' trailing columns are in W before the next panel
-    }
-}
-
-// Tasks of step k with WV_S2MAX < s <= 128 and rb <= 64 (list 3): one workgroup of
-// four waves each.  The tall products are split by 16-row tiles over the
-// waves, the two R factors run at once on waves 0 and 1, the Jacobi SVD uses
-// four lanes per column pair, and the small s x s products and solves take a
-// thread per row or column.  The workgroup already holds a whole CU's LDS,
-// so the extra waves cost no occupancy.
-#define WB_WAVES 4
-__global__ void __launch_bounds__(64 * WB_WAVES, 1)
-k_rc_wide(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *tasks_s, double *ws, double acc,
-          int fixed_rk, int maxrank, OpLog o, int *ovf, const double *qn_dense)
-{
-    extern __shared__ double smem[];
-    __shared__ int s_idx;
-    __shared__ double s_nz, s_fro;
-    constexpr int NTH = 64 * WB_WAVES;
-    const int tid = threadIdx.x, lane = tid & 63, wid = uni(tid >> 6);
-    double *L = smem;
-    double *sg = L + WB_SM * WB_LD;
-    const int NB = t.NB, NT = t.NT;
-    double *Wq = ws + (size_t)blockIdx.x * wb_slot_doubles(NB);
-    double *Qn = Wq + (size_t)NB * WB_SM;
-    double *Out = Qn + (size_t)NB * WB_SM;
-    double *Rp = Out + (size_t)NB * 2 * WB_SM;
-    double *Rq = Rp + WB_SM * WB_SM;
-    double *Ku = Rq + WB_SM * WB_SM;
-    const int cnt = uni(*wcount);
-    for (;;) {
-        if (tid == 0) s_idx = atomicAdd(wnext, 1);
-        __syncthreads();
-        const int idx = uni(s_idx);
-        __syncthreads();
-        if (idx >= cnt) break;
-        const int e = uni(wlist[idx]);
-        int hi, lo;
-        tri_decode(e, hi, lo);
-        const int m = uni(k + 1 + hi), n = uni(k + 1 + lo);
-        const bool bdense = (n - k < t.band_size);
-        const int ra = uni(*rank_at(t, m, k)), rc = uni(*rank_at(t, m, n)), rb = bdense ? 0 : uni(*rank_at(t, n, k));
-        const int s = rc + ra;
-        const double *Au = lr_tile(t, m, k), *Av = Au + (size_t)NB * ra;
-        const double *Bu = bdense ? Au : lr_tile(t, n, k), *Bv = Bu + (size_t)NB * rb;
-        double *C = lr_tile(t, m, n);
-        // Q's second block: formed below, or precomputed for a dense B
-        const double *Qs = bdense ? qn_dense + qn_slot(NT, NB, k, m, n) : Qn;
-        const int i16 = lane & 15, k4 = lane >> 4;
-        double *J = L;
-        // ---- X = Av^T Bv (ra <= 128, rb <= 64): 16-row band ta of X on wave ta % 4 ----
-        if (!bdense) {
-            double *Xl = L;  // Xl[b * WB_SM + a]
-            for (int q = tid; q < 64 * WB_SM; q += NTH) Xl[q] = 0.0;
-            __syncthreads();
-            for (int ta = wid; 16 * ta < ra; ta += WB_WAVES) {
-                wv_d4 xacc[4];
-#pragma unroll
-                for (int tb = 0; tb < 4; tb++) xacc[tb] = wv_d4{0.0, 0.0, 0.0, 0.0};
-                const int a = 16 * ta + i16;
-                for (int r0 = 0; r0 < NB; r0 += 16) {
-                    double av[4], bv[4][4];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int row = r0 + 4 * u + k4;
-                        av[u] = (a < ra && row < NB) ? Av[row + (size_t)a * NB] : 0.0;
-#pragma unroll
-                        for (int tb = 0; tb < 4; tb++) {
-                            const int bb = 16 * tb + i16;
-                            bv[u][tb] = (16 * tb < rb && bb < rb && row < NB) ? Bv[row + (size_t)bb * NB] : 0.0;
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; u++)
-#pragma unroll
-                        for (int tb = 0; tb < 4; tb++)
-                            if (16 * tb < rb) xacc[tb] = mfma16(av[u], bv[u][tb], xacc[tb]);
-                }
-#pragma unroll
-                for (int tb = 0; tb < 4; tb++)
-                    if (16 * tb < rb) {
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const int aa = 16 * ta + k4 + 4 * r, bb = 16 * tb + i16;
-                            if (aa < ra && bb < rb) Xl[bb * WB_SM + aa] = xacc[tb][r];
-                        }
-                    }
-            }
-            __syncthreads();
-        }
-        // ---- Qn = -Bu X^T ----
-        if (!bdense)
-            wv_tall_mm<WB_SM>(NB, rb, ra, -1.0, WvSrc{Bu, rb, Bu, NB}, L, WB_SM, Qn, wid,
-                              WB_WAVES);
-        __syncthreads();
-        // ---- R factors: P = [Cu Au] on waves 0 and 2 (trailing copy in Wq),
-        //      Q = [Cv Qn] on waves 1 and 3 (trailing copy in Out, unused until
-        //      the outputs); the panels' reflectors pass through the LDS,
-        //      free until the Jacobi ----
-        {
-            const int side = wid & 1;
-            wb_geqrf_r(s, side ? C + (size_t)NB * rc : C, side ? Qs : Au, rc, side ? Out : Wq, NB, side ? Rq : Rp,
-                       wid >> 1, L + (size_t)side * WB_QR_SH);
-        }
-        __syncthreads();
-        // ---- M^T = Rq Rp^T on the matrix cores (K = Rp^T = Rp's column-major
-        //      storage read row-wise, staged in LDS) into W (ld s); column c of
-        //      M^T (= row c of M) then goes to the Jacobi matrix ----
-        for (int q = tid; q < s * WB_SM; q += NTH) {
-            const int c = q % WB_SM;
-            L[q] = (c < s) ? Rp[q] : 0.0;  // K[l][c] = Rp(c, l)
-        }
-        __syncthreads();
-        wv_tall_mm<WB_SM>(s, s, s, 1.0, WvSrc{Rq, s, Rq, WB_SM}, L, WB_SM, Wq,
-                          wid, WB_WAVES);
-        __syncthreads();
-        for (int q = tid; q < s * WB_LD; q += NTH) {
-            const int c = q / WB_LD, r = q - c * WB_LD;
-            J[q] = (r < s) ? Wq[r + (size_t)c * s] : 0.0;
-        }
-        __syncthreads();
-        // squared column norms, kept up to date through the rotations and
-        // recomputed exactly after every sweep
-        double *nrm = sg + 2 * WB_SM;
-        for (int c = tid; c < s; c += NTH) {
-            const double *x = J + c * WB_LD;
-            double v = 0.0;
-            for (int q = 0; q < s; q++) v = fma(x[q], x[q], v);
-            nrm[c] = v;
-        }
-        __syncthreads();
-        if (wid == 0) {  // skip floor of the Jacobi rotations
-            double f2 = 0.0;
-            for (int c = lane; c < s; c += 64) f2 += nrm[c];
-            const double f2t = wsum(f2);
-            const double nzv = wv_skip_floor(f2t, s, acc, fixed_rk);
-            if (lane == 0) {
-                s_nz = nzv;
-                s_fro = sqrt(f2t);
-            }
-        }
-        __syncthreads();
-        // ---- one-sided Jacobi, columns in LDS: column pair tid / 4, the four
-        //      lanes of a quad take every fourth entry (the quad sum by DPP
-        //      gives all four the same ga, so they agree on the rotation) ----
-        {
-            const int npad = s + (s & 1), npairs = npad >> 1;
-            const double tol = 4.0e-16 * sqrt((double)s);
-            const double nz = s_nz;
-            const int pk = tid >> 2, sub = tid & 3;
-            int sweep = 0;
-            for (; sweep < BLK_JACOBI_SWEEPS; sweep++) {
-                int rot_any = 0;
-                for (int r = 0; r < npad - 1; r++) {
-                    if (pk < npairs) {
-                        const int ca = (pk == 0) ? 0 : ((pk - 1 + r) % (npad - 1)) + 1;
-                        const int pb = npad - 1 - pk;
-                        const int cb = (pb == 0) ? 0 : ((pb - 1 + r) % (npad - 1)) + 1;
-                        if (ca < s && cb < s) {
-                            double *x = J + ca * WB_LD, *y = J + cb * WB_LD;
-                            const double al = nrm[ca], be = nrm[cb];
-                            double g4[4] = {0, 0, 0, 0};
-                            int q = sub;
-                            for (; q + 12 < s; q += 16) {
-                                double xv[4], yv[4];
-#pragma unroll
-                                for (int u = 0; u < 4; u++) {
-                                    xv[u] = x[q + 4 * u];
-                                    yv[u] = y[q + 4 * u];
-                                }
-#pragma unroll
-                                for (int u = 0; u < 4; u++) g4[u] = fma(xv[u], yv[u], g4[u]);
-                            }
-                            for (; q < s; q += 4) g4[0] = fma(x[q], y[q], g4[0]);
-                            const double ga = gsum<4>((g4[0] + g4[1]) + (g4[2] + g4[3]));
-                            double cs, sn;
-                            if (fmin(al, be) > nz && jacobi_rot(al, be, ga, tol, cs, sn)) {
-                                rot_any = 1;
-                                if (sub == 0) {  // norms after the rotation
-                                    nrm[ca] = cs * cs * al - 2.0 * cs * sn * ga + sn * sn * be;
-                                    nrm[cb] = sn * sn * al + 2.0 * cs * sn * ga + cs * cs * be;
-                                }
-                                int q2 = sub;
-                                for (; q2 + 12 < s; q2 += 16) {
-                                    double xv[4], yv[4];
-#pragma unroll
-                                    for (int u = 0; u < 4; u++) {
-                                        xv[u] = x[q2 + 4 * u];
-                                        yv[u] = y[q2 + 4 * u];
-                                    }
-#pragma unroll
-                                    for (int u = 0; u < 4; u++) {
-                                        x[q2 + 4 * u] = cs * xv[u] - sn * yv[u];
-                                        y[q2 + 4 * u] = sn * xv[u] + cs * yv[u];
-                                    }
-                                }
-                                for (; q2 < s; q2 += 4) {
-                                    const double xv = x[q2], yv = y[q2];
-                                    x[q2] = cs * xv - sn * yv;
-                                    y[q2] = sn * xv + cs * yv;
-                                }
-                            }
-                        }
-                    }
-                    __syncthreads();
-                }
-                for (int c = tid; c < s; c += NTH) {
-                    const double *x = J + c * WB_LD;
-                    double v = 0.0;
-                    for (int q2 = 0; q2 < s; q2++) v = fma(x[q2], x[q2], v);
-                    nrm[c] = v;
-                }
-                if (!__syncthreads_or(rot_any)) break;
-            }
-            if (sweep >= BLK_JACOBI_SWEEPS && tid == 0) atomicAdd(o.unconv, 1);
-        }
-        // ---- singular values, order, rank (every wave counts the same nr) ----
-        for (int c = tid; c < s; c += NTH) {
-            const double *x = J + c * WB_LD;
-            double v = 0.0;
-            for (int q = 0; q < s; q++) v = fma(x[q], x[q], v);
-            sg[c] = sqrt(v);
-        }
-        __syncthreads();
-        int nr = 0;
-        {
-            int cntv = 0;
-            for (int c = lane; c < s; c += 64) cntv += (sg[c] >= acc);
-            nr = (fixed_rk > 0) ? (fixed_rk < s ? fixed_rk : s) : (int)wsum((double)cntv);
-        }
-        if (nr > maxrank) {
-            if (tid == 0) atomicAdd(ovf, 1);
-            nr = maxrank;
-        }
-        nr = uni(nr);
-        if (nr > 0) {
-            // selected columns, normalized, to Out (column pos, ld WB_SM), then
-            // row-major into LDS: Vl[l * WB_SM + pos]
-            for (int c = tid; c < s; c += NTH) {
-                const double sc = sg[c];
-                int pos = 0;
-                for (int q = 0; q < s; q++) {
-                    const double o2 = sg[q];
-                    pos += (o2 > sc) || (o2 == sc && q < c);
-                }
-                if (pos < nr) {
-                    const double inv = sc > 0.0 ? 1.0 / sc : 0.0;
-                    const double *x = J + c * WB_LD;
-                    for (int q = 0; q < s; q++) Out[q + (size_t)pos * WB_SM] = x[q] * inv;
-                    sg[WB_SM + pos] = sc;
-                }
-            }
-            __syncthreads();
-            double *Vl = L;
-            for (int q = tid; q < s * WB_SM; q += NTH) {
-                const int l = q / WB_SM, j = q - l * WB_SM;
-                Vl[q] = (j < nr) ? Out[l + (size_t)j * WB_SM] : 0.0;
-            }
-            __syncthreads();
-            // Ku = Rq^T Vs_r: thread (row c, half h) takes column blocks 32 h, 32 h + 64
-            {
-                const int c = tid & (WB_SM - 1), h = tid / WB_SM;
-                if (c < s) {
-                    for (int j0 = 32 * h; j0 < nr; j0 += 64) {
-                        double ac[32];
-#pragma unroll
-                        for (int j = 0; j < 32; j++) ac[j] = 0.0;
-                        for (int l = 0; l <= c; l++) {
-                            const double rq = Rq[l + (size_t)c * WB_SM];
-                            const double *vr = Vl + l * WB_SM + j0;
-#pragma unroll
-                            for (int j = 0; j < 32; j++) ac[j] = fma(rq, vr[j], ac[j]);
-                        }
-#pragma unroll
-                        for (int j = 0; j < 32; j++)
-                            if (j0 + j < nr) Ku[c * WB_SM + j0 + j] = ac[j];
-                    }
-                }
-            }
-            __syncthreads();
-            // Kv = Rq^-1 Vs_r in place, thread j solves column j: plain back
-            // substitution with the error bound and hand-off of k_rc_wave
-            // waves 0 and 1 (thread j = column j, nr <= 128); row q of Rq is
-            // loaded across the lanes (lane l: Rq(q, l) and Rq(q, l + 64), the
-            // next row's issued ahead) and read by readlane
-            int bad = 0;
-            if (wid < 2) {
-                const double tol = rc_solve_tol(acc, fixed_rk, s_fro);
-                const int j = tid;
-                const wv_rsrc rqr = wv_col_rsrc(Rq, WB_SM * WB_SM * 8);
-                auto ldrow = [&](int q, double &r0, double &r1) {
-                    r0 = wv_ld(rqr, (q >= 0 && lane < s) ? (q + lane * WB_SM) * 8 : WV_OOB);
-                    r1 = wv_ld(rqr, (q >= 0 && lane + 64 < s) ? (q + (lane + 64) * WB_SM) * 8 : WV_OOB);
-                };
-                double n0, n1, gmax = 0.0;
-                ldrow(s - 1, n0, n1);
-                for (int q = s - 1; q >= 0; q--) {
-                    const double r0 = n0, r1 = n1;
-                    ldrow(q - 1, n0, n1);
-                    double v = Vl[q * WB_SM + j], gq = 0.0;
-                    for (int l = q + 1; l < s; l++) {
-                        const double rql = (l < 64) ? rdlane(r0, l) : rdlane(r1, l - 64), xl = Vl[l * WB_SM + j];
-                        v = fma(-rql, xl, v);
-                        gq = fma(fabs(rql), fabs(xl), gq);
-                    }
-                    const double d = (q < 64) ? rdlane(r0, q) : rdlane(r1, q - 64);
-                    const bool ok = fabs(d) > 1e-300;
-                    const double x = ok ? v / d : 0.0;
-                    if (!ok && j < nr) bad = 1;
-                    gmax = fmax(gmax, fma(fabs(d), fabs(x), gq));
-                    if (j < nr) Vl[q * WB_SM + j] = x;
-                }
-                if (j < nr && !(sg[WB_SM + j] * s * 2.3e-16 * gmax <= tol)) bad = 1;
-            }
-            if (__syncthreads_or(bad)) {
-                if (tid == 0) tasks_s[e] = RC_REDO;
-                __syncthreads();
-                continue;
-            }
-            // ---- outputs in place into the tile, ordered as in k_rc_wave (each
-            //      wave reads and writes only its own row tiles) ----
-            auto v_out = [&]() {  // Kv in LDS
-                wv_tall_mm<WB_SM>(NB, s, nr, 1.0, WvSrc{C + (size_t)rc * NB, rc, Qs, NB}, Vl, WB_SM,
-                                  C + (size_t)nr * NB, wid, WB_WAVES);
-                __syncthreads();
-            };
-            auto u_out = [&]() {  // stages Ku into LDS
-                for (int q = tid; q < s * WB_SM; q += NTH) {
-                    const int c = q / WB_SM, j = q - c * WB_SM;
-                    Vl[q] = (j < nr) ? Ku[c * WB_SM + j] : 0.0;
-                }
-                __syncthreads();
-                wv_tall_mm<WB_SM>(NB, s, nr, 1.0, WvSrc{C, rc, Au, NB}, Vl, WB_SM, C, wid, WB_WAVES);
-                __syncthreads();
-            };
-            if (nr > rc) {
-                v_out();
-                u_out();
-            } else {
-                for (int q = tid; q < s * WB_SM; q += NTH) Out[q] = Vl[q];  // Kv aside while Ku uses the LDS
-                u_out();
-                for (int q = tid; q < s * WB_SM; q += NTH) Vl[q] = Out[q];
-                __syncthreads();
-                v_out();
-            }
-        }
-        if (tid == 0) {
-            *rank_at(t, m, n) = nr;
-            rank_hist(o, NT, m, n, nr);
-            unsigned long long mm = tdim(t, m), ss = s;
-            unsigned long long qa = opc('q', mm, ss, 0, 0);
-            // case iv (dense B) counts the product B Av, case v the products with B's factors
-            unsigned long long qb = bdense ? opc('q', mm, ss, 0, 0) + opc('m', ra, mm, mm, 0)
-                                           : opc('m', ra, rb, mm, 0) + opc('m', ra, mm, rb, 0) + opc('q', mm, ss, 0, 0);
-            unsigned long long sv = opc('r', ss, ss, 2, 0) + opc('s', ss, 0, 0, 0) + ss * nr;
-            unsigned long long nu = opc('o', mm, nr, ss, 1), nv = opc('o', nr, mm, ss, 2);
-            oplog(o, NT, qa + qb + sv + nu + nv, m, n, false, false);
-            atomicAdd(o.stat + 4, qa + qb + sv + nu + nv);
-            atomicAdd(o.stat + 5, 1ULL);
-            unsigned long long words =
-                2ULL * NB * (ra + rc + nr) + (bdense ? (unsigned long long)NB * NB : 2ULL * NB * rb);
-            atomicAdd(o.stat + 6, 8ULL * words);
-        }
-        __syncthreads();
     }
 }

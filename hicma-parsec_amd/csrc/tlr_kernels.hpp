@@ -693,10 +693,6 @@ __global__ void __launch_bounds__(BS) k_gemm_lrd_update(TLR t, int k, const doub
 
 // ======================= gemm, low-rank result (cases iv, v) =======================
 
-// tasks_s value of a task handed from a fast recompression kernel to the
-// Householder path (k_lr_gemm, launched after them on the context stream)
-#define RC_REDO (1 << 30)
-
 // Accepted error of the V' = Q (Rq^-1 Vs_r) back-substitution of the fast
 // kernels, absolute in the tile: a fraction of the truncation threshold,
 // never below rounding of M (fro = ||M||_F).
@@ -704,6 +700,37 @@ __device__ __forceinline__ double rc_solve_tol(double acc, int fixed_rk, double 
 {
     const double floor_ = 1e-13 * fro;
     return (fixed_rk > 0 || !(acc > 0.0)) ? floor_ : fmax(1e-3 * acc, floor_);
+}
+
+// Squared-norm floor below which a Jacobi pair is not rotated: rounding noise
+// of M, or, when truncating at acc, (1e-3 acc)^2 (see k_rc_wave).
+__device__ __forceinline__ double wv_skip_floor(double f2, int s, double acc, int fixed_rk)
+{
+    const double nz = (2.3e-16 * s) * (2.3e-16 * s) * f2;
+    const double tz = (fixed_rk > 0 || !(acc > 0.0)) ? 0.0 : (1e-3 * acc) * (1e-3 * acc);
+    return fmax(nz, tz);
+}
+
+// op counts of one recompression (the reference's formulas) and its totals:
+// op count, tasks, algorithmic bytes (8 * (inputs A, B, C + output) words, B
+// dense in case iv)
+__device__ __forceinline__ void rc_oplog(const OpLog &o, const TLR &t, int m, int n, int ra, int rb, int rc, int nr,
+                                         bool bdense)
+{
+    const unsigned long long mm = tdim(t, m), ss = rc + ra;  // the reference counts with tile m's rows
+    const unsigned long long qa = opc('q', mm, ss, 0, 0);
+    // case iv (dense B) counts the product B Av, case v the products with B's factors
+    const unsigned long long qb = bdense ? opc('q', mm, ss, 0, 0) + opc('m', ra, mm, mm, 0)
+                                         : opc('m', ra, rb, mm, 0) + opc('m', ra, mm, rb, 0) + opc('q', mm, ss, 0, 0);
+    const unsigned long long sv = opc('r', ss, ss, 2, 0) + opc('s', ss, 0, 0, 0) + ss * nr;
+    const unsigned long long nu = opc('o', mm, nr, ss, 1), nv = opc('o', nr, mm, ss, 2);
+    const unsigned long long ops = qa + qb + sv + nu + nv;
+    oplog(o, t.NT, ops, m, n, false, false);
+    atomicAdd(o.stat + 4, ops);
+    atomicAdd(o.stat + 5, 1ULL);
+    const unsigned long long words =
+        2ULL * t.NB * (ra + rc + nr) + (bdense ? (unsigned long long)t.NB * t.NB : 2ULL * t.NB * rb);
+    atomicAdd(o.stat + 6, 8ULL * words);
 }
 
 struct RcWs {
@@ -722,13 +749,14 @@ __host__ __device__ inline size_t rc_slot_doubles(int NB, int cap)
 
 #define RC_FIXED_SMEM (BLK_GEMM_SMEM + BLK_RED_SMEM + 2 * QRB * QRB)
 
-// One workgroup per task (m,n): C' = Cu Cv^T - A B^T recompressed.
+// Tiles that k_rc_big does not take (more than 2048 rows, or ranks above
+// 1024): one workgroup per task (m,n), everything in global memory.
+// C' = Cu Cv^T - A B^T recompressed.
 // (v)  A, B low rank:  Qn = -Bu (Av^T Bv)^T
 // (iv) A low rank, B dense: Qn = -B Av
 // P = [Cu Au], Q = [Cv Qn]; QR both; M = Rp Rq^T; Jacobi SVD; keep
 // sigma >= acc (or the fixed rank) capped at maxrank; U' = Qp [Us S], V' = Qq [Vs].
-__global__ void __launch_bounds__(BS) k_lr_gemm(TLR t, int k, const int *tasks_s, int smin, double *ws, RcWs g,
-                                                double acc, int fixed_rk, int maxrank, OpLog o, int *ovf)
+__global__ void __launch_bounds__(BS) k_lr_gemm(TLR t, int k, double *ws, RcWs g, double acc, int fixed_rk, int maxrank, OpLog o, int *ovf)
 {
     extern __shared__ double sm[];
     const int NB = t.NB, NT = t.NT, cap = t.cap, b = t.band_size, tid = threadIdx.x;
@@ -752,9 +780,6 @@ __global__ void __launch_bounds__(BS) k_lr_gemm(TLR t, int k, const int *tasks_s
     const int T = NT - 1 - k;
     const long long ntask = (long long)T * (T - 1) / 2;
     for (long long task = blockIdx.x; task < ntask; task += gridDim.x) {
-        // tasks_s: stack width decided before any update of this step; this
-        // kernel takes the tasks the fast path leaves (s > smin)
-        if (tasks_s[task] <= smin) continue;
         int hi, lo;
         tri_decode(task, hi, lo);
         const int m = k + 1 + hi, n = k + 1 + lo;
@@ -762,6 +787,7 @@ __global__ void __launch_bounds__(BS) k_lr_gemm(TLR t, int k, const int *tasks_s
         const int ra = *rank_at(t, m, k), rc = *rank_at(t, m, n);
         const int rb = bdense ? 0 : *rank_at(t, n, k);
         const int s = rc + ra;
+        if (m - n < b || ra < 0 || rb < 0 || rc < 0 || (!bdense && (ra == 0 || rb == 0))) continue;
         const double *A = lr_tile(t, m, k), *Au = A, *Av = A + (size_t)NB * ra;
         double *C = lr_tile(t, m, n);
         // stacks
@@ -822,19 +848,7 @@ __global__ void __launch_bounds__(BS) k_lr_gemm(TLR t, int k, const int *tasks_s
         if (tid == 0) {
             *rank_at(t, m, n) = nr;
             rank_hist(o, NT, m, n, nr);
-            unsigned long long nn = tdim(t, m), ss = s;  // the reference counts with tile m's rows
-            unsigned long long qa = opc('q', nn, ss, 0, 0), qb;
-            if (bdense) qb = opc('q', nn, ss, 0, 0) + opc('m', ra, nn, nn, 0);
-            else qb = opc('m', ra, rb, nn, 0) + opc('m', ra, nn, rb, 0) + opc('q', nn, ss, 0, 0);
-            unsigned long long sv = opc('r', ss, ss, 2, 0) + opc('s', ss, 0, 0, 0) + ss * nr;
-            unsigned long long nu = opc('o', nn, nr, ss, 1), nv = opc('o', nr, nn, ss, 2);
-            oplog(o, NT, qa + qb + sv + nu + nv, m, n, false, false);
-            // recompression totals: op count, tasks, algorithmic bytes
-            // (8 * (inputs A, B, C + output) words, B dense in case iv)
-            atomicAdd(o.stat + 4, qa + qb + sv + nu + nv);
-            atomicAdd(o.stat + 5, 1ULL);
-            unsigned long long words = 2ULL * NB * (ra + rc + nr) + (bdense ? (unsigned long long)NB * NB : 2ULL * NB * rb);
-            atomicAdd(o.stat + 6, 8ULL * words);
+            rc_oplog(o, t, m, n, ra, rb, rc, nr, bdense);
         }
         __syncthreads();
     }

@@ -21,6 +21,13 @@ __device__ __forceinline__ double mk64(unsigned l, unsigned h)
     return __longlong_as_double((long long)(((unsigned long long)h << 32) | l));
 }
 
+// value of v on lane l (uniform)
+__device__ __forceinline__ double rdlane(double v, int l)
+{
+    return mk64((unsigned)__builtin_amdgcn_readlane((int)lo32(v), l),
+                (unsigned)__builtin_amdgcn_readlane((int)hi32(v), l));
+}
+
 // DPP controls (GFX9 encoding)
 #define DPP_XOR1 0xB1   // quad_perm [1,0,3,2]
 #define DPP_XOR2 0x4E   // quad_perm [2,3,0,1]
