@@ -5,6 +5,7 @@
 // every task of a step; tile ranks never leave HBM (kernels read them).
 #include "internal.hpp"
 #include "tlr_kernels.hpp"
+#include "gen.hpp"
 #include "rc_wave.hpp"
 
 #include <math.h>
@@ -378,6 +379,22 @@ static int apply_problem(hicma_tlr_desc *A, const void *data, const hicma_kernel
     return 0;
 }
 
+// Workspace of the compression: doubles per workgroup, workgroups, and the
+// whole with the task list of a pass
+static size_t gen_stride(int NB, int p, int cap)
+{
+    return gw_fits(NB, p) ? (gw_slot_doubles(NB, p) + 15) / 16 * 16 : gen_slot_doubles(NB, p, cap);
+}
+static int gen_slots(hicma_ctx *ctx, int NB, int p, int cap, long long ntask)
+{
+    const int ns = nslots_for(ctx, gen_stride(NB, p, cap) * sizeof(double), ntask);
+    return gw_fits(NB, p) ? std::min(ns, ctx->ncu) : ns;  // k_compress_wg: one workgroup per CU
+}
+static size_t gen_ws_doubles(hicma_ctx *ctx, int NB, int p, int cap, long long ntask)
+{
+    return gen_stride(NB, p, cap) * gen_slots(ctx, NB, p, cap, ntask) + (size_t)ntask / 2 + 8;
+}
+
 // The compression passes first .. last of STARSH_gen over the off-band
 // tiles (outside A's current band): pass 0 compresses every tile with the
 // narrow sketch, passes 1 and 2 again, at wider sketches up to the full
@@ -397,13 +414,18 @@ static int gen_lr(hicma_tlr_desc *A, double tol, int maxrank, int first, int las
         double *d_om = nullptr;
         HIPCHK(ctx_malloc(ctx, (void **)&d_om, sizeof(double) * om.size()));
         HIPCHK(hipMemcpy(d_om, om.data(), sizeof(double) * om.size(), hipMemcpyHostToDevice));  // stream idle (ctx_malloc)
-        GenWs g;
-        g.p = p;
-        g.stride = gen_slot_doubles(NB, p, t.cap);
-        int ns = nslots_for(ctx, g.stride * sizeof(double), ntask);
-        if ((rc = hicma_ensure_ws(ctx, g.stride * sizeof(double) * ns))) return rc;
-        size_t lds = sizeof(double) * (BLK_GEMM_SMEM + BLK_RED_SMEM + 2 * QRB * QRB + 3 * (size_t)p + 16);
-        HIPCHK(hipFuncSetAttribute((const void *)k_compress, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        const bool wg = gw_fits(NB, p);
+        const int ns = gen_slots(ctx, NB, p, t.cap, ntask);
+        const size_t stride = gen_stride(NB, p, t.cap);
+        if ((rc = hicma_ensure_ws(ctx, gen_ws_doubles(ctx, NB, p, t.cap, ntask) * sizeof(double)))) return rc;
+        int *ncnt = (int *)(ctx->ws + stride * ns), *list = ncnt + 4;
+        // tiles of up to 256, 512, 1024, 2048 rows: 1, 2, 4, 8 rows per thread in the QR panels
+        const auto comp = NB <= 256 ? k_compress_wg<1>
+                                    : (NB <= 512 ? k_compress_wg<2> : (NB <= 1024 ? k_compress_wg<4> : k_compress_wg<8>));
+        const size_t lds = wg ? sizeof(double) * WQ_LDS
+                              : sizeof(double) * (BLK_GEMM_SMEM + BLK_RED_SMEM + 2 * QRB * QRB + 3 * (size_t)p + 16);
+        HIPCHK(hipFuncSetAttribute(wg ? (const void *)comp : (const void *)k_compress,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         // narrow sketch first; tiles whose rank it cannot vouch for again at
         // a wider one, up to the full width
         const int ladder[3] = {GEN_FIRST_SKETCH, GEN_SECOND_SKETCH, p};
@@ -411,10 +433,21 @@ static int gen_lr(hicma_tlr_desc *A, double tol, int maxrank, int first, int las
         for (int pass = 0; pass <= last; pass++) {
             const int pw = ladder[pass] < p ? ladder[pass] : p;
             if (pw <= prev) continue;
-            if (pass >= first)
-                hipLaunchKernelGGL(k_compress, dim3(ns), dim3(BS), lds, ctx->stream, t, (const double *)d_om,
-                                   ctx->ws, g, pw, pass > 0 ? 1 : 0, tol, maxrank, ctx->d_info);
             prev = pw;
+            if (pass < first) continue;
+            if (wg) {
+                hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, ctx->stream, ncnt, 4, 0);
+                hipLaunchKernelGGL(k_gen_list, dim3((unsigned)((ntask + 255) / 256)), dim3(256), 0, ctx->stream, t,
+                                   pass > 0 ? 1 : 0, list, ncnt);
+                hipLaunchKernelGGL(comp, dim3(ns), dim3(BS), lds, ctx->stream, t, (const double *)d_om,
+                                   (const int *)list, ncnt, ctx->ws, stride, p, pw, tol, maxrank, ctx->d_info);
+            } else {
+                GenWs g;
+                g.p = p;
+                g.stride = stride;
+                hipLaunchKernelGGL(k_compress, dim3(ns), dim3(BS), lds, ctx->stream, t, (const double *)d_om, ctx->ws,
+                                   g, pw, pass > 0 ? 1 : 0, tol, maxrank, ctx->d_info);
+            }
         }
         HIPCHK(hipGetLastError());
         HIPCHK(hipStreamSynchronize(ctx->stream));
@@ -776,8 +809,7 @@ size_t hicma_work_bytes(hicma_ctx *ctx, int N, int NB, int cap, int band)
     int p = cap + 10;
     if (p > NB) p = NB;
     const long long ntask = (long long)NT * (NT - 1) / 2;
-    const size_t gs = gen_slot_doubles(NB, p, cap);
-    const size_t gen = ntask > 0 ? gs * nslots_for(ctx, gs * sizeof(double), ntask) : 0;
+    const size_t gen = ntask > 0 ? gen_ws_doubles(ctx, NB, p, cap, ntask) : 0;
     return sizeof(double) * (std::max(P.total, gen) + (size_t)NB * p);
 }
 

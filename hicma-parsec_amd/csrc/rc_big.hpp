@@ -82,16 +82,16 @@ k_rc_big(TLR t, int k, const int *list, const int *count, int *next, double *ws,
         double *C = lr_tile(t, m, n);
         // stacks
         double *Qn = Q + (size_t)rc * NB;
-        blk_copy(NB, rc, C, NB, P, NB);
-        blk_copy(NB, ra, Au, NB, P + (size_t)rc * NB, NB);
-        blk_copy(NB, rc, C + (size_t)NB * rc, NB, Q, NB);
+        wq_copy(NB, rc, C, NB, P, NB);
+        wq_copy(NB, ra, Au, NB, P + (size_t)rc * NB, NB);
+        wq_copy(NB, rc, C + (size_t)NB * rc, NB, Q, NB);
         __syncthreads();
         if (!bdense) {
             const double *Bu = lr_tile(t, n, k), *Bv = Bu + (size_t)NB * rb;
             blk_gemm<true, false>(ra, rb, NB, 1.0, Av, NB, Bv, NB, 0.0, Xr, ra, S.main);
             blk_gemm<false, true>(NB, ra, rb, -1.0, Bu, NB, Xr, ra, 0.0, Qn, NB, S.main);
         } else if (qn_dense && ra > 0 && s <= QN_COLS) {
-            blk_copy(NB, ra, qn_dense + qn_slot(NT, NB, k, m, n), NB, Qn, NB);  // formed by k_qn_dense
+            wq_copy(NB, ra, qn_dense + qn_slot(NT, NB, k, m, n), NB, Qn, NB);  // formed by k_qn_dense
         } else {
             blk_gemm<false, false>(NB, ra, NB, -1.0, band_tile(t, n, k), NB, Av, NB, 0.0, Qn, NB, S.main);
         }
@@ -103,7 +103,7 @@ k_rc_big(TLR t, int k, const int *list, const int *count, int *next, double *ws,
             wq_triu(s, Q, NB, B2, s);
             __syncthreads();
             blk_gemm<false, true>(s, s, s, 1.0, B1, s, B2, s, 0.0, Ms, s, S.main);  // M = Rp Rq^T
-            blk_copy(s, s, Ms, s, B1, s);
+            wq_copy(s, s, Ms, s, B1, s);
             const double f2 = wq_fro2(s, Ms, s, S.red);
             __syncthreads();
             if (wq_right_svd<R>(s, B1, s, B2, wv_skip_floor(f2, s, acc, fixed_rk), Tm, Vb, S) >= BLK_JACOBI_SWEEPS &&

@@ -45,8 +45,6 @@ __host__ __device__ inline size_t wv_slot_doubles(int NB)
     return (size_t)NB * 4 * WV_SMAX + 4 * (size_t)WV_SMAX * WV_SMAX;
 }
 
-__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
-
 // FP64 matrix core tile C += A B with A 16x4, B 4x16, C 16x16 (gfx950
 // V_MFMA_F64_16X16X4_F64).  Operand layout on the wave: A[i][k] on lane
 // i + 16k, B[k][j] on lane j + 16k; result C[i][j] on lane j + 16 (i & 3),

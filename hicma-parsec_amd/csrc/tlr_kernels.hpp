@@ -36,7 +36,8 @@ __host__ __device__ inline size_t gen_slot_doubles(int NB, int p, int cap)
 // rank-map marker of a tile whose first, narrow sketch was too narrow
 #define GEN_REDO (-2)
 
-// STARS-H starsh_dense_dlrrsdd restated as a workgroup pipeline:
+// STARS-H starsh_dense_dlrrsdd restated as a workgroup pipeline, everything in
+// global memory, for tiles above 2048 rows (k_compress_wg takes the others):
 // D = kernel tile; Y = D*Omega; Q = qr(Y); X = D^T Q; X = Qx Rx; Jacobi SVD of Rx;
 // rank by relative Frobenius tail <= tol; U = Q*Vr, V = Qx*(Ur*S).
 //

@@ -28,6 +28,9 @@ __device__ __forceinline__ double rdlane(double v, int l)
                 (unsigned)__builtin_amdgcn_readlane((int)hi32(v), l));
 }
 
+// a wave-uniform value into a scalar register
+__device__ __forceinline__ int uni(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
 // DPP controls (GFX9 encoding)
 #define DPP_XOR1 0xB1   // quad_perm [1,0,3,2]
 #define DPP_XOR2 0x4E   // quad_perm [2,3,0,1]
@@ -167,6 +170,15 @@ __device__ __forceinline__ void wv_st(double v, wv_rsrc r, int off)
 {
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(wv_u2, v), r, off, 0, 0);
 }
+// the same with a wave-uniform second offset (two offsets past the resource
+// stay past it)
+__device__ __forceinline__ int wv_off2(int off, int uoff)
+{
+    const unsigned s = (unsigned)off + (unsigned)uoff;
+    return off < 0 || uoff < 0 ? (int)WV_OOB : (int)s;
+}
+__device__ __forceinline__ double wv_ldc(wv_rsrc r, int off, int uoff) { return wv_ld(r, wv_off2(off, uoff)); }
+__device__ __forceinline__ void wv_stc(double v, wv_rsrc r, int off, int uoff) { wv_st(v, r, wv_off2(off, uoff)); }
 // rows lane, lane + 64, ... of a column (KR rows per lane)
 template <int KR>
 __device__ __forceinline__ void wv_ld_col(double (&x)[KR], wv_rsrc r, int lane)

@@ -24,8 +24,32 @@ struct WqLds {
 };
 __device__ __forceinline__ WqLds wq_lds(double *sm)
 {
-    double *x = sm + WQ_MAIN;
-    return WqLds{sm, x, x + 272, x + 544, x + 560, x + 688};
+    // the small parts first: their addresses are then immediates of the LDS instructions
+    return WqLds{sm + WQ_AUX, sm, sm + 272, sm + 544, sm + 560, sm + 688};
+}
+
+// f(r, c, g(r, c)) for the rows r < rows of the columns c < nc, a thread on
+// consecutive rows: eight columns' loads g are issued before the first store f,
+// so that a copy costs one latency per eight columns.
+template <typename Ld, typename St>
+__device__ __forceinline__ void wq_cols(int rows, int nc, Ld g, St f)
+{
+    for (int r = threadIdx.x; r < rows; r += BS)
+        for (int c = 0; c < nc; c += 8) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; u++) v[u] = (c + u < nc) ? g(r, c + u) : 0.0;
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                if (c + u < nc) f(r, c + u, v[u]);
+        }
+}
+
+__device__ __forceinline__ void wq_copy(int rows, int nc, const double *src, int lds, double *dst, int ldd)
+{
+    wq_cols(
+        rows, nc, [&](int r, int c) { return src[r + (size_t)c * lds]; },
+        [&](int r, int c, double v) { dst[r + (size_t)c * ldd] = v; });
 }
 
 // column stride of the V panel: 17 mod 32 keeps both reads of the panel
@@ -34,21 +58,19 @@ __device__ __forceinline__ int wq_ldv(int m) { return ((m + 63) & ~63) + 17; }
 
 // T (upper, 16 x 16) of H = I - V T V^T from G and tau, by lanes 0 .. 15 of
 // wave 0: lane i forms row i.  Into S.T and Tsave (column major).
-__device__ __forceinline__ void wq_build_t(int jb, const WqLds &S, double *Tsave)
+__device__ __forceinline__ void wq_build_t(const WqLds &S, double *Tsave)
 {
-    const int i = threadIdx.x;
+    int i = threadIdx.x;
+    asm volatile("" : "+v"(i));
     if (i < WQ_PW) {
         double tr[WQ_PW];
 #pragma unroll
         for (int j = 0; j < WQ_PW; j++) {
-            double v = 0.0;
-            if (j < jb) {
-                const double tj = S.tau[j];
-                double s = 0.0;
+            const double tj = S.tau[j];
+            double s = 0.0;
 #pragma unroll
-                for (int l = 0; l < j; l++) s = fma(l >= i ? tr[l] : 0.0, S.G[l + 17 * j], s);
-                v = (i == j) ? tj : (i < j ? -tj * s : 0.0);
-            }
+            for (int l = 0; l < j; l++) s = fma(l >= i ? tr[l] : 0.0, S.G[l + 17 * j], s);
+            const double v = (i == j) ? tj : (i < j ? -tj * s : 0.0);
             tr[j] = v;
             S.T[i * 17 + j] = v;
             Tsave[i + WQ_PW * j] = v;
@@ -66,18 +88,24 @@ template <int R>
 __device__ __forceinline__ void wq_panel(int mr, int jb, double *Ap, int lda, double *V, int ldv, double *Tsave,
                                          const WqLds &S)
 {
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    // opaque, so that the comparisons with it are not hoisted out of the panel
+    // loop into scalar registers that then spill
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, w = tid >> 6;
+    // columns past jb are zero throughout: they read 0, and their tau comes out 0
+    const wv_rsrc ar = wv_col_rsrc(Ap, ((jb - 1) * lda + mr) * 8);
+    int off[R];
+#pragma unroll
+    for (int r = 0; r < R; r++) off[r] = tid + BS * r < mr ? 8 * (tid + BS * r) : WV_OOB;
     double a[R][WQ_PW];
 #pragma unroll
     for (int c = 0; c < WQ_PW; c++)
 #pragma unroll
-        for (int r = 0; r < R; r++) {
-            const int row = tid + BS * r;
-            a[r][c] = (c < jb && row < mr) ? Ap[row + (size_t)c * lda] : 0.0;
-        }
+        for (int r = 0; r < R; r++) a[r][c] = wv_ldc(ar, off[r], c < jb ? 8 * c * lda : WV_OOB);
 #pragma unroll
     for (int jj = 0; jj < WQ_PW; jj++) {
-        if (jj < jb) {
+        {
             const int buf = jj & 1;
             const double x0 = a[0][jj], y0 = (tid > jj) ? x0 : 0.0;
             double p[WQ_PW];
@@ -129,12 +157,11 @@ __device__ __forceinline__ void wq_panel(int mr, int jb, double *Ap, int lda, do
 #pragma unroll
         for (int r = 0; r < R; r++) {
             const int row = tid + BS * r;
-            if (c < jb && row < mr) Ap[row + (size_t)c * lda] = a[r][c];
-            const double v = (c < jb && row < mr) ? (row > c ? a[r][c] : (row == c ? 1.0 : 0.0)) : 0.0;
-            if (row < mrp) V[c * ldv + row] = v;
+            wv_stc(a[r][c], ar, off[r], c < jb ? 8 * c * lda : WV_OOB);
+            if (row < mrp) V[c * ldv + row] = row > c ? a[r][c] : (row == c ? 1.0 : 0.0);
         }
     __syncthreads();  // G, tau are complete
-    wq_build_t(jb, S, Tsave);
+    wq_build_t(S, Tsave);
     __syncthreads();  // V, T for every wave
 }
 
@@ -234,11 +261,9 @@ __device__ __forceinline__ void wq_apply(int m, int nc, int k, const double *A, 
         const int j0 = WQ_PW * p, jb = min(WQ_PW, k - j0), mr = m - j0, ldv = wq_ldv(mr), mrp = (mr + 63) & ~63;
         const double *Ap = A + j0 + (size_t)j0 * lda;
         __syncthreads();
-        for (int c = 0; c < WQ_PW; c++)
-            for (int row = tid; row < mrp; row += BS) {
-                const double v = (c < jb && row < mr) ? (row > c ? Ap[row + (size_t)c * lda] : (row == c ? 1.0 : 0.0)) : 0.0;
-                V[c * ldv + row] = v;
-            }
+        wq_cols(
+            mrp, WQ_PW, [&](int r, int c) { return (c < jb && r < mr && r > c) ? Ap[r + (size_t)c * lda] : 0.0; },
+            [&](int r, int c, double v) { V[c * ldv + r] = (r == c && c < jb) ? 1.0 : v; });
         S.T[(tid & 15) * 17 + (tid >> 4)] = Tsave[(size_t)p * WQ_PW * WQ_PW + tid];
         __syncthreads();
         const int cs = TRI ? j0 : 0;
@@ -252,54 +277,78 @@ __device__ __forceinline__ void wq_apply(int m, int nc, int k, const double *A, 
 
 // ---- one-sided Jacobi -----------------------------------------------------
 
+// jacobi_rot by the hardware's approximate roots: the angle's relative error
+// (2^-23) only leaves that part of the inner product for the next sweep, and
+// c = (1 + t^2)^-1/2 gets one third-order step, so c^2 + s^2 = 1 to rounding.
+// 14 dependent instructions instead of some 50.
+__device__ __forceinline__ bool wj_rotation(double al, double be, double ga, double tol, double &c, double &s)
+{
+    if (ga == 0.0 || !(ga * ga > (tol * tol) * (al * be))) return false;
+    const double diff = be - al, g2 = 2.0 * ga, h = fma(diff, diff, g2 * g2);
+    const double den = fabs(diff) + h * __builtin_amdgcn_rsq(h);
+    if (!(den > 0.0)) return false;
+    const double t = (diff >= 0.0 ? g2 : -g2) * __builtin_amdgcn_rcp(den);
+    const double u = fma(t, t, 1.0), r = __builtin_amdgcn_rsq(u), e = fma(-u * r, r, 1.0);
+    c = fma(r * e, fma(0.375, e, 0.5), r);
+    s = c * t;
+    return true;
+}
+
 #define WJ_ROWS 40        // rows per lane
 #define WJ_SMALL2 1e-20   // squared cosine below which a rotation counts as small
 
 // One pair by a group of G lanes (lane sub of the group holds rows sub,
-// sub + G, ...; `nch` chunks of two such rows, rows past the matrix hold zeros):
+// sub + G, ...; `nch` chunks of four such rows, rows past the matrix hold zeros):
 // the pair is read once, rotated in registers and written back if it turned.
 // Returns 0 (left alone), 1 (turned by a small angle) or 3.
 template <int G>
 __device__ __forceinline__ int wj_pair(double *x, double *y, int nch, int sub, double tol, double nz)
 {
+    asm volatile("" : "+s"(nch));  // no hoisted comparison per chunk
+    constexpr int CH = 4;          // rows per chunk
     double xv[WJ_ROWS], yv[WJ_ROWS], al[2] = {0.0, 0.0}, be[2] = {0.0, 0.0}, ga[2] = {0.0, 0.0};
+    // every load first, then the products, so that the loads' latencies overlap
 #pragma unroll
-    for (int c = 0; c < WJ_ROWS / 2; c++)
+    for (int c = 0; c < WJ_ROWS / CH; c++)
         if (c < nch) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                xv[2 * c + u] = x[sub + G * (2 * c + u)];
-                yv[2 * c + u] = y[sub + G * (2 * c + u)];
+            for (int u = 0; u < CH; u++) {
+                xv[CH * c + u] = x[sub + G * (CH * c + u)];
+                yv[CH * c + u] = y[sub + G * (CH * c + u)];
             }
+        }
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                al[u] = fma(xv[2 * c + u], xv[2 * c + u], al[u]);
-                be[u] = fma(yv[2 * c + u], yv[2 * c + u], be[u]);
-                ga[u] = fma(xv[2 * c + u], yv[2 * c + u], ga[u]);
+    for (int c = 0; c < WJ_ROWS / CH; c++)
+        if (c < nch) {
+#pragma unroll
+            for (int u = 0; u < CH; u++) {
+                al[u & 1] = fma(xv[CH * c + u], xv[CH * c + u], al[u & 1]);
+                be[u & 1] = fma(yv[CH * c + u], yv[CH * c + u], be[u & 1]);
+                ga[u & 1] = fma(xv[CH * c + u], yv[CH * c + u], ga[u & 1]);
             }
         }
     const double a = gsum<G>(al[0] + al[1]), b = gsum<G>(be[0] + be[1]), g = gsum<G>(ga[0] + ga[1]);
     double cs, sn;
-    if (!(fmin(a, b) > nz) || !jacobi_rot(a, b, g, tol, cs, sn)) return 0;
+    if (!(fmin(a, b) > nz) || !wj_rotation(a, b, g, tol, cs, sn)) return 0;
 #pragma unroll
-    for (int c = 0; c < WJ_ROWS / 2; c++)
+    for (int c = 0; c < WJ_ROWS / CH; c++)
         if (c < nch) {
 #pragma unroll
-            for (int u = 0; u < 2; u++) {
-                const double xo = xv[2 * c + u], yo = yv[2 * c + u];
-                x[sub + G * (2 * c + u)] = cs * xo - sn * yo;
-                y[sub + G * (2 * c + u)] = sn * xo + cs * yo;
+            for (int u = 0; u < CH; u++) {
+                const double xo = xv[CH * c + u], yo = yv[CH * c + u];
+                x[sub + G * (CH * c + u)] = cs * xo - sn * yo;
+                y[sub + G * (CH * c + u)] = sn * xo + cs * yo;
             }
         }
     return g * g > WJ_SMALL2 * a * b ? 3 : 1;
 }
 
-// LDS column stride of m-row columns: multiples of 2 G rows, and columns of
+// LDS column stride of m-row columns: multiples of 4 G rows, and columns of
 // consecutive pairs start G banks apart
 template <int G>
 __host__ __device__ __forceinline__ int wj_ldc(int m)
 {
-    const int rows = (m + 2 * G - 1) / (2 * G) * (2 * G);
+    const int rows = (m + 4 * G - 1) / (4 * G) * (4 * G);
     return G < 32 ? rows + G : rows;
 }
 // whether G lanes per pair take columns of m rows: WJ_ROWS rows per lane, and
@@ -308,7 +357,7 @@ template <int G>
 __host__ __device__ __forceinline__ bool wj_takes(int m, int n)
 {
     const int nc = 2 * BS / G, ldc = wj_ldc<G>(m);
-    return (m + 2 * G - 1) / (2 * G) * 2 <= WJ_ROWS && (long)(n < nc ? n + (n & 1) : nc) * ldc <= WQ_MAIN;
+    return (m + 4 * G - 1) / (4 * G) * 4 <= WJ_ROWS && (long)(n < nc ? n + (n & 1) : nc) * ldc <= WQ_MAIN;
 }
 
 // One-sided Jacobi on the n columns of M (m x n, ld ldm, in place): on return
@@ -326,17 +375,17 @@ __device__ __forceinline__ int wj_jacobi(int m, int n, double *M, int ldm, doubl
 {
     constexpr int NP = BS / G, NC = 2 * NP;
     const int tid = threadIdx.x, kp = tid / G, sub = tid % G;
-    const int nch = (m + 2 * G - 1) / (2 * G), rows = nch * 2 * G, ldc = wj_ldc<G>(m);
+    const int nch = (m + 4 * G - 1) / (4 * G), rows = nch * 4 * G, ldc = wj_ldc<G>(m);
     const double tol = 4.0e-16 * sqrt((double)m);
     auto move_in = [&](int c0, int g0, int nc) {  // LDS columns c0 .. c0 + nc - 1 <- columns g0 ..
-        for (int c = 0; c < nc; c++)
-            for (int r = tid; r < rows; r += BS)
-                L[(c0 + c) * ldc + r] = (g0 + c < n && r < m) ? M[r + (size_t)(g0 + c) * ldm] : 0.0;
+        wq_cols(
+            rows, nc, [&](int r, int c) { return (g0 + c < n && r < m) ? M[r + (size_t)(g0 + c) * ldm] : 0.0; },
+            [&](int r, int c, double v) { L[(c0 + c) * ldc + r] = v; });
     };
     auto move_out = [&](int c0, int g0, int nc) {
-        for (int c = 0; c < nc; c++)
-            if (g0 + c < n)
-                for (int r = tid; r < m; r += BS) M[r + (size_t)(g0 + c) * ldm] = L[(c0 + c) * ldc + r];
+        wq_cols(
+            m, min(nc, n - g0), [&](int r, int c) { return L[(c0 + c) * ldc + r]; },
+            [&](int r, int c, double v) { M[r + (size_t)(g0 + c) * ldm] = v; });
     };
     // every pair of the first nc (even) LDS columns once
     auto all_pairs = [&](int nc) {
@@ -404,26 +453,285 @@ __device__ __forceinline__ int wj_jacobi(int m, int n, double *M, int ldm, doubl
     return sweep;
 }
 
+// ---- the same with 4 x 4 column blocks per group --------------------------
+// A group of G lanes holds eight columns (two blocks of four) in registers
+// and turns all pairs across the blocks, four independent rotations at a time, so
+// a column crosses the LDS once per four rotations (one per rotation bounds
+// wj_jacobi: 16 bytes per row each way at about 64 bytes per cycle).  The four
+// inner products are reduce-scattered over the lanes of each quad, lane j
+// (mod 4) computes rotation j, and DPP gives every lane all four.
+// What bounds it: the chain of dependent instructions of a step (one wave per SIMD,
+// about 350 instructions of 3.4 ns a step).  One workgroup per matrix, N=2700
+// tile 270 band 1: 33 -> 27 ms against wj_jacobi; 28 sketches of 266 columns
+// 43 -> 33 ms, of 160 13 -> 9 ms.
+
+#define WJ4_ROWS 10  // rows per lane
+
+__device__ __forceinline__ double wj_quad(double v, int j)
+{
+    switch (j) {
+    case 0: return dppd<0x00>(v);  // quad_perm [j, j, j, j]
+    case 1: return dppd<0x55>(v);
+    case 2: return dppd<0xAA>(v);
+    default: return dppd<0xFF>(v);
+    }
+}
+
+// Four independent rotations (u_j, v_j); nu, nv: squared norms, the same on
+// every lane.  nch chunks of two rows.  Returns as wj_pair.
+template <int G>
+__device__ __forceinline__ int wj_rot4(double (&u0)[WJ4_ROWS], double (&v0)[WJ4_ROWS], double (&u1)[WJ4_ROWS],
+                                       double (&v1)[WJ4_ROWS], double (&u2)[WJ4_ROWS], double (&v2)[WJ4_ROWS],
+                                       double (&u3)[WJ4_ROWS], double (&v3)[WJ4_ROWS], double &nu0, double &nv0,
+                                       double &nu1, double &nv1, double &nu2, double &nv2, double &nu3, double &nv3,
+                                       int nch, int sub, double tol, double nz)
+{
+    double p0 = 0.0, p1 = 0.0, p2 = 0.0, p3 = 0.0;
+#pragma unroll
+    for (int c = 0; c < WJ4_ROWS / 2; c++)
+        if (c < nch) {
+#pragma unroll
+            for (int q = 2 * c; q < 2 * c + 2; q++) {
+                p0 = fma(u0[q], v0[q], p0);
+                p1 = fma(u1[q], v1[q], p1);
+                p2 = fma(u2[q], v2[q], p2);
+                p3 = fma(u3[q], v3[q], p3);
+            }
+        }
+    const bool b0 = sub & 1, b1 = sub & 2;
+    const double q0 = (b0 ? p1 : p0) + dppd<DPP_XOR1>(b0 ? p0 : p1);
+    const double q1 = (b0 ? p3 : p2) + dppd<DPP_XOR1>(b0 ? p2 : p3);
+    double ga = (b1 ? q1 : q0) + dppd<DPP_XOR2>(b1 ? q0 : q1);  // product sub & 3 of this quad
+    ga += xor4d(ga);
+    ga += dppd<DPP_ROR8>(ga);
+    if (G >= 32) {
+        double x = ga, y = ga;
+        swap16d(x, y);
+        ga = x + y;
+    }
+    if (G >= 64) {
+        double x = ga, y = ga;
+        swap32d(x, y);
+        ga = x + y;
+    }
+    const double al = b1 ? (b0 ? nu3 : nu2) : (b0 ? nu1 : nu0), be = b1 ? (b0 ? nv3 : nv2) : (b0 ? nv1 : nv0);
+    double cs = 1.0, sn = 0.0;
+    bool rot = false;
+    if (fmin(al, be) > nz) rot = wj_rotation(al, be, ga, tol, cs, sn);
+    if (!rot) {
+        cs = 1.0;
+        sn = 0.0;
+    }
+    if (__ballot(rot) == 0) return 0;
+    const double na = rot ? cs * cs * al - 2.0 * cs * sn * ga + sn * sn * be : al;
+    const double nb = rot ? sn * sn * al + 2.0 * cs * sn * ga + cs * cs * be : be;
+    nu0 = wj_quad(na, 0), nu1 = wj_quad(na, 1), nu2 = wj_quad(na, 2), nu3 = wj_quad(na, 3);
+    nv0 = wj_quad(nb, 0), nv1 = wj_quad(nb, 1), nv2 = wj_quad(nb, 2), nv3 = wj_quad(nb, 3);
+    const double c0 = wj_quad(cs, 0), c1 = wj_quad(cs, 1), c2 = wj_quad(cs, 2), c3 = wj_quad(cs, 3);
+    const double s0 = wj_quad(sn, 0), s1 = wj_quad(sn, 1), s2 = wj_quad(sn, 2), s3 = wj_quad(sn, 3);
+    auto turn = [](double &x, double &y, double c, double s) {
+        const double xo = x, yo = y;
+        x = fma(c, xo, -(s * yo));
+        y = fma(s, xo, c * yo);
+    };
+#pragma unroll
+    for (int c = 0; c < WJ4_ROWS / 2; c++)
+        if (c < nch) {
+#pragma unroll
+            for (int q = 2 * c; q < 2 * c + 2; q++) {
+                turn(u0[q], v0[q], c0, s0);
+                turn(u1[q], v1[q], c1, s1);
+                turn(u2[q], v2[q], c2, s2);
+                turn(u3[q], v3[q], c3, s3);
+            }
+        }
+    return !rot ? 0 : (ga * ga > WJ_SMALL2 * al * be ? 3 : 1);
+}
+
+// rows and column stride in LDS; columns of neighbouring groups (G = 16) lie
+// sixteen banks apart
+template <int G>
+__host__ __device__ __forceinline__ int wj4_rows(int m) { return (m + 2 * G - 1) / (2 * G) * (2 * G); }
+template <int G>
+__host__ __device__ __forceinline__ int wj4_ldc(int m) { return wj4_rows<G>(m) + (G == 16 ? 4 : 0); }
+// LDS columns (a multiple of eight), 0 when a lane would hold too many rows
+template <int G>
+__host__ __device__ __forceinline__ int wj4_cols(int m)
+{
+    if (wj4_rows<G>(m) > WJ4_ROWS * G) return 0;
+    const int c = WQ_MAIN / wj4_ldc<G>(m) / 8 * 8, most = BS / G * 8;
+    return c < most ? c : most;
+}
+
+// wj_jacobi's contract.  The n columns stay in LDS when they fit; otherwise
+// blocks of up to half of the LDS columns take turns, as there.  Norms are
+// kept up to date through the rotations and computed anew in every sweep.
+template <int G>
+__device__ __forceinline__ int wj4_jacobi(int m, int n, double *M, int ldm, double nz, const WqLds &S)
+{
+    double *L = S.main, *nrm = S.T;  // 128 norms
+    const int tid = threadIdx.x, kp = tid / G, sub = tid % G;
+    const int rows = wj4_rows<G>(m), nch = rows / (2 * G), ldc = wj4_ldc<G>(m), cap = wj4_cols<G>(m);
+    const double tol = 4.0e-16 * sqrt((double)m);
+    auto move_in = [&](int c0, int g0, int nc) {
+        wq_cols(
+            rows, nc, [&](int r, int c) { return (g0 + c < n && r < m) ? M[r + (size_t)(g0 + c) * ldm] : 0.0; },
+            [&](int r, int c, double v) { L[(c0 + c) * ldc + r] = v; });
+    };
+    auto move_out = [&](int c0, int g0, int nc) {
+        wq_cols(
+            m, min(nc, n - g0), [&](int r, int c) { return L[(c0 + c) * ldc + r]; },
+            [&](int r, int c, double v) { M[r + (size_t)(g0 + c) * ldm] = v; });
+    };
+    auto norms = [&](int nc) {
+        const int lane = tid & 63;
+        for (int c = tid >> 6; c < nc; c += NWAVE) {
+            double s = 0.0;
+            for (int r = lane; r < rows; r += 64) s = fma(L[c * ldc + r], L[c * ldc + r], s);
+            s = wsum(s);
+            if (lane == 0) nrm[c] = s;
+        }
+        __syncthreads();
+    };
+    // blocks of four columns at ca and cb: all pairs across, and within both if `own`
+    auto visit = [&](int ca, int cb, bool own) -> int {
+        double *xa = L + ca * ldc + sub, *xb = L + cb * ldc + sub;
+        int nc_ = nch;
+        asm volatile("" : "+s"(nc_));  // no hoisted comparison per chunk
+        double x0[WJ4_ROWS], x1[WJ4_ROWS], x2[WJ4_ROWS], x3[WJ4_ROWS], y0[WJ4_ROWS], y1[WJ4_ROWS], y2[WJ4_ROWS],
+            y3[WJ4_ROWS];
+#pragma unroll
+        for (int c = 0; c < WJ4_ROWS / 2; c++)
+            if (c < nc_) {
+#pragma unroll
+                for (int q = 2 * c; q < 2 * c + 2; q++) {
+                    x0[q] = xa[G * q], x1[q] = xa[ldc + G * q], x2[q] = xa[2 * ldc + G * q], x3[q] = xa[3 * ldc + G * q];
+                    y0[q] = xb[G * q], y1[q] = xb[ldc + G * q], y2[q] = xb[2 * ldc + G * q], y3[q] = xb[3 * ldc + G * q];
+                }
+            }
+        double a0 = nrm[ca], a1 = nrm[ca + 1], a2 = nrm[ca + 2], a3 = nrm[ca + 3];
+        double b0 = nrm[cb], b1 = nrm[cb + 1], b2 = nrm[cb + 2], b3 = nrm[cb + 3];
+        int any = 0;
+        if (own) {
+            any |= wj_rot4<G>(x0, x1, x2, x3, y0, y1, y2, y3, a0, a1, a2, a3, b0, b1, b2, b3, nc_, sub, tol, nz);
+            any |= wj_rot4<G>(x0, x2, x1, x3, y0, y2, y1, y3, a0, a2, a1, a3, b0, b2, b1, b3, nc_, sub, tol, nz);
+            any |= wj_rot4<G>(x0, x3, x1, x2, y0, y3, y1, y2, a0, a3, a1, a2, b0, b3, b1, b2, nc_, sub, tol, nz);
+        }
+        any |= wj_rot4<G>(x0, y0, x1, y1, x2, y2, x3, y3, a0, b0, a1, b1, a2, b2, a3, b3, nc_, sub, tol, nz);
+        any |= wj_rot4<G>(x0, y1, x1, y2, x2, y3, x3, y0, a0, b1, a1, b2, a2, b3, a3, b0, nc_, sub, tol, nz);
+        any |= wj_rot4<G>(x0, y2, x1, y3, x2, y0, x3, y1, a0, b2, a1, b3, a2, b0, a3, b1, nc_, sub, tol, nz);
+        any |= wj_rot4<G>(x0, y3, x1, y0, x2, y1, x3, y2, a0, b3, a1, b0, a2, b1, a3, b2, nc_, sub, tol, nz);
+        if (__ballot(any) == 0) return 0;
+#pragma unroll
+        for (int c = 0; c < WJ4_ROWS / 2; c++)
+            if (c < nc_) {
+#pragma unroll
+                for (int q = 2 * c; q < 2 * c + 2; q++) {
+                    xa[G * q] = x0[q], xa[ldc + G * q] = x1[q], xa[2 * ldc + G * q] = x2[q], xa[3 * ldc + G * q] = x3[q];
+                    xb[G * q] = y0[q], xb[ldc + G * q] = y1[q], xb[2 * ldc + G * q] = y2[q], xb[3 * ldc + G * q] = y3[q];
+                }
+            }
+        if (sub == 0) {
+            nrm[ca] = a0, nrm[ca + 1] = a1, nrm[ca + 2] = a2, nrm[ca + 3] = a3;
+            nrm[cb] = b0, nrm[cb + 1] = b1, nrm[cb + 2] = b2, nrm[cb + 3] = b3;
+        }
+        return any;
+    };
+    // every pair of the first 4 nb4 LDS columns (nb4 even)
+    auto all_pairs = [&](int nb4) {
+        int any = 0;
+        for (int r = 0; r < nb4 - 1; r++) {
+            if (kp < nb4 / 2) {
+                int ca = kp == 0 ? 0 : kp - 1 + r, cb = nb4 - 2 - kp + r;
+                if (kp) {
+                    if (ca >= nb4 - 1) ca -= nb4 - 1;
+                    ca++;
+                }
+                if (cb >= nb4 - 1) cb -= nb4 - 1;
+                cb++;
+                any |= visit(4 * ca, 4 * cb, r == 0);
+            }
+            __syncthreads();
+        }
+        return any;
+    };
+    int sweep = 0;
+    if (n <= cap) {
+        const int nb4 = (n + 7) / 8 * 2;
+        move_in(0, 0, 4 * nb4);
+        __syncthreads();
+        for (; sweep < BLK_JACOBI_SWEEPS; sweep++) {
+            norms(4 * nb4);
+            if (!__syncthreads_or(all_pairs(nb4) & 2)) break;
+        }
+        move_out(0, 0, n);
+        __syncthreads();
+        return sweep;
+    }
+    // blocks of W columns, as many as needed and of even widths
+    const int nb = (n + cap / 2 - 1) / (cap / 2), W = ((n + nb - 1) / nb + 3) / 4 * 4, nbe = nb + (nb & 1);
+    for (; sweep < BLK_JACOBI_SWEEPS; sweep++) {
+        int any = 0;
+        for (int rd = 0; rd < nbe - 1; rd++)
+            for (int q = 0; q < nbe / 2; q++) {
+                int ba = q == 0 ? 0 : (q - 1 + rd) % (nbe - 1) + 1, bb = (nbe - 2 - q + rd) % (nbe - 1) + 1;
+                if (ba > bb) {
+                    const int s = ba;
+                    ba = bb;
+                    bb = s;
+                }
+                if (bb >= nb && rd > 0) continue;  // a block without a partner: its own pairs in round 0
+                move_in(0, ba * W, W);
+                move_in(W, bb < nb ? bb * W : n, W);
+                __syncthreads();
+                norms(2 * W);
+                int rot = 0;
+                const int w4 = W / 4;
+                if (rd == 0) {
+                    rot = all_pairs(2 * w4);
+                } else {
+                    for (int r = 0; r < w4; r++) {
+                        if (kp < w4) {
+                            const int cb = kp + r < w4 ? kp + r : kp + r - w4;
+                            rot |= visit(4 * kp, W + 4 * cb, false);
+                        }
+                        __syncthreads();
+                    }
+                }
+                any |= rot & 2;
+                if (__syncthreads_or(rot)) {
+                    move_out(0, ba * W, W);
+                    move_out(W, bb < nb ? bb * W : n, W);
+                }
+                __syncthreads();
+            }
+        if (!__syncthreads_or(any)) break;
+    }
+    return sweep;
+}
+
 // tallest matrix wj_svd takes (64 lanes per pair, 8 columns of LDS)
 #define WJ_MAXN 2304
-__device__ __forceinline__ int wj_svd(int m, int n, double *M, int ldm, double nz, double *L)
+__device__ __forceinline__ int wj_svd(int m, int n, double *M, int ldm, double nz, const WqLds &S)
 {
     if (n <= 1) return 0;
-    if (n <= 32 && wj_takes<16>(m, n)) return wj_jacobi<16>(m, n, M, ldm, nz, L);
-    if (n <= 64 && wj_takes<8>(m, n)) return wj_jacobi<8>(m, n, M, ldm, nz, L);
-    if (n <= 128 && wj_takes<4>(m, n)) return wj_jacobi<4>(m, n, M, ldm, nz, L);
-    if (wj_takes<8>(m, n)) return wj_jacobi<8>(m, n, M, ldm, nz, L);
-    if (wj_takes<16>(m, n)) return wj_jacobi<16>(m, n, M, ldm, nz, L);
-    if (wj_takes<32>(m, n)) return wj_jacobi<32>(m, n, M, ldm, nz, L);
-    return wj_jacobi<64>(m, n, M, ldm, nz, L);
+    // all columns resident with the fewest lanes per block pair, else the widest blocks
+    const int c16 = wj4_cols<16>(m), c32 = wj4_cols<32>(m), c64 = wj4_cols<64>(m);
+    if (n > 64 || c32 < n) {
+        if (c16 >= 64) return wj4_jacobi<16>(m, n, M, ldm, nz, S);
+    }
+    if (c32 >= 32) return wj4_jacobi<32>(m, n, M, ldm, nz, S);
+    if (c64 >= 16) return wj4_jacobi<64>(m, n, M, ldm, nz, S);
+    if (wj_takes<32>(m, n)) return wj_jacobi<32>(m, n, M, ldm, nz, S.main);
+    return wj_jacobi<64>(m, n, M, ldm, nz, S.main);
 }
 
 // squared Frobenius norm of M (n x n, ld ldm), the same on every thread
 __device__ __forceinline__ double wq_fro2(int n, const double *M, int ldm, double *red)
 {
     double s = 0.0;
-    for (int c = threadIdx.x >> 6; c < n; c += NWAVE)
-        for (int r = threadIdx.x & 63; r < n; r += 64) s = fma(M[r + (size_t)c * ldm], M[r + (size_t)c * ldm], s);
+    wq_cols(
+        n, n, [&](int r, int c) { return M[r + (size_t)c * ldm]; }, [&](int, int, double v) { s = fma(v, v, s); });
     return blk_sum(s, red);
 }
 
@@ -442,21 +750,11 @@ __device__ __forceinline__ void wq_sigma(int m, int n, const double *M, int ldm,
     blk_sort_pos(n, sig, pos);
 }
 
-// Right singular vectors of M (n x n, ld ldm): M = Q1 R, and one-sided Jacobi
-// on the columns of R^T (the rows of R) gives R^T J = Vs S.  The rows of an
-// (unpivoted) R are graded, which takes 5 .. 8 sweeps where the columns of M
-// or M^T take 8 .. 22 (stacks of 44 .. 115 columns of 2-D sqexp updates), and
-// the rows after the last one above the floor nz2 (a squared norm, see
-// wv_skip_floor) take no part.  M is overwritten by its QR; X (n x n, ld n)
-// returns Vs S in columns 0 .. n - 1 (unsorted).  Returns the sweeps.
-template <int R>
-__device__ __forceinline__ int wq_right_svd(int n, double *M, int ldm, double *X, double nz, double *Tsave, double *Vb,
-                                            const WqLds &S)
+// Jacobi on the columns of X (n x n, ld n), graded by rows of an R factor:
+// the columns after the last one above the floor nz (a squared norm) take no
+// part.  Returns the sweeps.
+__device__ __forceinline__ int wq_graded_svd(int n, double *X, double nz, const WqLds &S)
 {
-    wq_geqrf<R>(n, n, M, ldm, Tsave, Vb, S);
-    for (int i = threadIdx.x >> 6; i < n; i += NWAVE)
-        for (int r = threadIdx.x & 63; r < n; r += 64) X[r + (size_t)i * n] = r >= i ? M[i + (size_t)r * ldm] : 0.0;
-    __syncthreads();
     __shared__ int s_ke;
     if (threadIdx.x == 0) s_ke = 0;
     __syncthreads();
@@ -467,12 +765,31 @@ __device__ __forceinline__ int wq_right_svd(int n, double *M, int ldm, double *X
         if ((threadIdx.x & 63) == 0 && !(s <= nz)) atomicMax(&s_ke, i + 1);
     }
     __syncthreads();
-    return wj_svd(n, s_ke, X, n, nz, S.main);
+    return wj_svd(n, s_ke, X, n, nz, S);
+}
+
+// Right singular vectors of M (n x n, ld ldm): M = Q1 R, and one-sided Jacobi
+// on the columns of R^T (the rows of R) gives R^T J = Vs S.  The rows of an
+// (unpivoted) R are graded, which takes 5 .. 8 sweeps where the columns of M
+// or M^T take 8 .. 22 (stacks of 44 .. 115 columns of 2-D sqexp updates).  M is
+// overwritten by its QR; X (n x n, ld n) returns Vs S in columns 0 .. n - 1
+// (unsorted).  Returns the sweeps.
+template <int R>
+__device__ __forceinline__ int wq_right_svd(int n, double *M, int ldm, double *X, double nz, double *Tsave, double *Vb,
+                                            const WqLds &S)
+{
+    wq_geqrf<R>(n, n, M, ldm, Tsave, Vb, S);
+    // X(r, i) = R(i, r): threads run down the columns of R
+    wq_cols(
+        n, n, [&](int i, int r) { return r >= i ? M[i + (size_t)r * ldm] : 0.0; },
+        [&](int i, int r, double v) { X[r + (size_t)i * n] = v; });
+    return wq_graded_svd(n, X, nz, S);
 }
 
 // dst (n x n) <- upper triangle of src, zeros below the diagonal
 __device__ __forceinline__ void wq_triu(int n, const double *src, int lds, double *dst, int ldd)
 {
-    for (int c = threadIdx.x >> 6; c < n; c += NWAVE)
-        for (int r = threadIdx.x & 63; r < n; r += 64) dst[r + (size_t)c * ldd] = r <= c ? src[r + (size_t)c * lds] : 0.0;
+    wq_cols(
+        n, n, [&](int r, int c) { return r <= c ? src[r + (size_t)c * lds] : 0.0; },
+        [&](int r, int c, double v) { dst[r + (size_t)c * ldd] = v; });
 }
