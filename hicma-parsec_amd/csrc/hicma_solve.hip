@@ -3,20 +3,28 @@
 //
 // No counterpart in the reference (it stops at the factor); the solves read
 // the factor in the layout HiCMA_dpotrf_L leaves (dense band tiles, compact
-// [U | V] off-band tiles, each in the type the precision map gives).
-// Blocked substitution by tile columns:
-//   forward  (B <- L^-1 B):  X_k = L_kk^-1 B_k, then B_m -= L_mk X_k  (m > k)
-//   backward (B <- L^-T B):  X_k = L_kk^-T B_k, then B_j -= L_kj^T X_k (j < k)
-// with L_mk X_k = U (V^T X_k) for low-rank tiles.  Every L_kk^-1 is formed
-// once per call (the 64 x 64 diagonal-block inverses one wave each, the
-// blocks below on the matrix cores), so the diagonal step is a block
-// matrix-vector product over 64-row blocks in parallel instead of a chain
-// of dependent 64-row substitutions, and each update runs one workgroup per
-// 64-row block of each tile.  The NT diagonal/update launch pairs of a pass
-// remain a chain.  A pass reads its right-hand sides from one buffer and
-// writes its solution to another, so no launch updates in place what another
-// workgroup of it still reads.  All sums run in a fixed order: the results do
-// not depend on scheduling.
+// [U | V] off-band tiles, each in the type the precision map gives) and the
+// inverses of its diagonal tiles, which the factorization keeps (a descriptor
+// without them has them formed first, k_tri_inv and k_tile_inv).
+//
+// One pass (L^-1 B or L^-T B, in place) is one launch, k_solve_flow: by tile rows
+// in the order of the substitution (first to last forward, last to first
+// backward), row m has 8 or 16 update tasks, each summing its share of every
+// L_mk x_k, k before m, in that order, and one diagonal task per 32 rows of
+// x_m = L_mm^-1 (b_m - sum).  Workgroups claim tasks in this order from a
+// counter; a task waits only for tasks before it, so the schedule cannot
+// deadlock whatever is resident, and each wait is bounded all the same.  While an
+// update task waits for x_k it already holds its share of tile (m, k) in
+// registers, so the chain per row is one small product, a sum over the shares
+// and the block product with L_mm^-1.  All sums run in a fixed order: the
+// results do not depend on scheduling.
+//
+// What bounds it: the chain of 2 NT hand-overs between compute units through the
+// memory's coherence point.  The pass it replaced launched two kernels per tile
+// row and formed the inverses in every call.  One vector at N=90000 band 1
+// 7.5 -> 2.1 ms (0.55 TB/s of factor); Sigma^-1 b at N=2700 1.00 -> 0.21 ms; eight
+// right-hand sides at N=30011 band 16 7.7 -> 4.6 ms; twenty backward at N=8091
+// band 10 2.8 -> 0.9 ms.
 #include "internal.hpp"
 #include "mfma.hpp"
 #include "wave.hpp"
@@ -25,23 +33,17 @@
 #include <algorithm>
 #include <utility>
 
-#define SV_RC 4                // right-hand sides per pass
 #define SV_BK 64               // diagonal block edge
-#define SU_T 1024              // threads of the diagonal and update kernels
-#define SU_G (SU_T / SV_BK)    // their column groups (one wave each)
-
-// L_kk^-1 is held as nb packed block-column panels per diagonal tile: panel
-// c holds block rows c .. nb-1 of block column c, column major with
-// ld 64 (nb - c); the panels of tile k start at Xinv + k inv_tile(nb).
-__host__ __device__ __forceinline__ size_t inv_tile(int nb) { return (size_t)SV_BK * SV_BK * nb * (nb + 1) / 2; }
-__host__ __device__ __forceinline__ size_t inv_poff(int nb, int c)
-{
-    return (size_t)SV_BK * SV_BK * ((size_t)c * nb - (size_t)c * (c - 1) / 2);
-}
+#define SF_T 512               // threads of the flow kernel
+#define SF_W (SF_T / 64)
+#define SF_GMAX 16             // update tasks per tile row: sf_shares()
+#define SF_RB 32               // rows of x per diagonal task
+#define SF_PF 4                // blocks of L_mm^-1 a diagonal task loads ahead
+#define SF_SPIN_LIMIT (1 << 21)
 
 // W = L_bb^-1 for every 64 x 64 diagonal block b of every diagonal tile k,
-// into block 0 of panel b (rows and columns beyond the tile, NB not a
-// multiple of 64, hold the identity).  One wave per block: lane c forms
+// into block (b, b) of its inverse (rows and columns beyond the tile, NB not
+// a multiple of 64, hold the identity).  One wave per block: lane c forms
 // column c of W by forward substitution, W(i, c) = (e_c(i) - sum_{c <= l < i}
 // L(i, l) W(l, c)) / L(i, i), with L and W in LDS.
 __global__ void __launch_bounds__(64) k_tri_inv(TLR t, double *Xinv)
@@ -65,291 +67,459 @@ __global__ void __launch_bounds__(64) k_tri_inv(TLR t, double *Xinv)
         Ws[i * (SV_BK + 1) + c] = (i >= c) ? s / Lr[i * (SV_BK + 1) + i] : 0.0;
     }
     wv_sync();
-    const size_t ld = (size_t)SV_BK * (nbk - b);
-    double *W = Xinv + (size_t)k * inv_tile(nbk) + inv_poff(nbk, b);
-    for (int j = 0; j < SV_BK; j++) W[lane + (size_t)j * ld] = Ws[lane * (SV_BK + 1) + j];
+    double *W = Xinv + (size_t)k * inv_tile(nbk) + inv_blk(b, b) * SV_BK * SV_BK;
+    for (int j = 0; j < SV_BK; j++) W[lane + j * SV_BK] = Ws[lane * (SV_BK + 1) + j];
 }
 
 // The off-diagonal blocks of L_kk^-1, block column c of tile k per
 // workgroup (grid NT nb): X_bc = -W_b sum_{j=c}^{b-1} L_bj X_jc for
-// b = c+1 .. nb-1, each sum one matrix-core product of the row panel
-// L(b, c .. b-1) with the panel's blocks c .. b-1, stored into block b's
-// slot, then multiplied by W_b from panel b.
+// b = c+1 .. nb-1, the sum on the matrix cores, stored into block (b, c),
+// then multiplied by W_b.
 __global__ void __launch_bounds__(256) k_tile_inv(TLR t, double *Xinv)
 {
     __shared__ double sm[MK_SMEM];
     const int NB = t.NB, nb = (NB + SV_BK - 1) / SV_BK;
     const int k = blockIdx.x / nb, c = blockIdx.x % nb;
-    const int ldx = SV_BK * (nb - c);
     double *X0 = Xinv + (size_t)k * inv_tile(nb);
-    double *Xp = X0 + inv_poff(nb, c);
     const double *Lk = band_tile(t, k, k);
     for (int b = c + 1; b < nb; b++) {
         mk_d4 acc[2][2];
         mk_zero(acc);
-        // S = L(64b .., 64c .. 64b) Xp(0 .. 64(b - c), :)
-        const MkOps<false, true> op{Lk + (size_t)SV_BK * c * NB, NB, Xp, ldx};
-        mk_accum(op, NB, SV_BK, SV_BK * b, 0, 0, SV_BK * (b - c), acc, sm);
-        double *Sb = Xp + SV_BK * (b - c);
-        mk_store(acc, [&](int i, int j, double v) { Sb[i + (size_t)j * ldx] = v; });
+        for (int j = c; j < b; j++) {
+            const MkOps<false, true> op{Lk + (size_t)SV_BK * j * NB, NB, X0 + inv_blk(j, c) * SV_BK * SV_BK, SV_BK};
+            mk_accum(op, NB, SV_BK, SV_BK * b, 0, 0, SV_BK, acc, sm);
+        }
+        double *Sb = X0 + inv_blk(b, c) * SV_BK * SV_BK;
+        mk_store(acc, [&](int i, int j, double v) { Sb[i + j * SV_BK] = v; });
         __syncthreads();
-        // X_bc = -W_b S; W_b is block 0 of panel b
+        // X_bc = -W_b S
         mk_zero(acc);
-        const MkOps<false, true> op2{X0 + inv_poff(nb, b), SV_BK * (nb - b), Sb, ldx};
+        const MkOps<false, true> op2{X0 + inv_blk(b, b) * SV_BK * SV_BK, SV_BK, Sb, SV_BK};
         mk_accum(op2, SV_BK, SV_BK, 0, 0, 0, SV_BK, acc, sm);  // ends with a barrier: S is read
-        mk_store(acc, [&](int i, int j, double v) { Sb[i + (size_t)j * ldx] = -v; });
+        mk_store(acc, [&](int i, int j, double v) { Sb[i + j * SV_BK] = -v; });
         __syncthreads();
     }
 }
 
-// x_k = L_kk^-1 y_k (forward) or L_kk^-T y_k (backward), block row b per
-// workgroup (grid nb): y from the rows of tile k in Pin, x into Pout.
-// forward:  x_b = sum_{c <= b} X_bc y_c, thread (i, g) takes columns g + 16u
-//           of each block, the 16 groups summed in order;
-// backward: x_b = sum_{c >= b} X_cb^T y_c, wave g takes columns g + 16u of
-//           panel b, its lanes run down the rows.
-// LDS: y (64 nb x SV_RC), partial sums (16 x 64 x SV_RC).
-__global__ void __launch_bounds__(SU_T) k_solve_diag(TLR t, int k, const double *Xinv, const double *Pin,
-                                                     double *Pout, long ldp, int nrhs, int trans)
+// ---- the pass ---------------------------------------------------------------
+
+// Values that pass between workgroups are written and read past the L1 and the
+// XCD's L2 (agent scope); a counter follows them once every store of the
+// workgroup has completed.
+__device__ __forceinline__ double sf_ld(const double *p)
 {
-    extern __shared__ double sm[];
-    const int NB = t.NB, nb = (NB + SV_BK - 1) / SV_BK, NBp = nb * SV_BK;
-    double *y = sm;                            // y[l * SV_RC + q]
-    double *pt = y + (size_t)NBp * SV_RC;      // pt[(g * 64 + i) * SV_RC + q]
-    const int tid = threadIdx.x, i = tid & 63, g = tid >> 6, b = blockIdx.x;
-    const double *X0 = Xinv + (size_t)k * inv_tile(nb);
-    const double *Pk = Pin + (size_t)k * NB;
-    double *Po = Pout + (size_t)k * NB;
-    for (int r0 = 0; r0 < nrhs; r0 += SV_RC) {
-        const int nq = min(SV_RC, nrhs - r0);
-        for (int e = tid; e < NBp * SV_RC; e += SU_T) {
-            const int q = e / NBp, l = e - q * NBp;
-            y[l * SV_RC + q] = (l < NB && q < nq) ? Pk[l + (size_t)(r0 + q) * ldp] : 0.0;
-        }
-        __syncthreads();
-        if (!trans) {
-            double acc[SV_RC];
-#pragma unroll
-            for (int q = 0; q < SV_RC; q++) acc[q] = 0.0;
-#pragma unroll 2
-            for (int c = 0; c <= b; c++) {
-                const size_t ld = (size_t)SV_BK * (nb - c);
-                const double *Bp = X0 + inv_poff(nb, c) + SV_BK * (b - c) + i;
-                double v[SV_BK / SU_G];
-#pragma unroll
-                for (int u = 0; u < SV_BK / SU_G; u++) v[u] = Bp[(size_t)(g + SU_G * u) * ld];
-#pragma unroll
-                for (int u = 0; u < SV_BK / SU_G; u++)
-#pragma unroll
-                    for (int q = 0; q < SV_RC; q++)
-                        acc[q] = fma(v[u], y[(SV_BK * c + g + SU_G * u) * SV_RC + q], acc[q]);
-            }
-#pragma unroll
-            for (int q = 0; q < SV_RC; q++) pt[(g * SV_BK + i) * SV_RC + q] = acc[q];
-        } else {
-            const size_t ld = (size_t)SV_BK * (nb - b);
-            const double *Pb = X0 + inv_poff(nb, b) + i;
-            double acc[SV_BK / SU_G][SV_RC];
-#pragma unroll
-            for (int u = 0; u < SV_BK / SU_G; u++)
-#pragma unroll
-                for (int q = 0; q < SV_RC; q++) acc[u][q] = 0.0;
-#pragma unroll 2
-            for (int c = b; c < nb; c++) {
-                double v[SV_BK / SU_G];
-#pragma unroll
-                for (int u = 0; u < SV_BK / SU_G; u++) v[u] = Pb[SV_BK * (c - b) + (size_t)(g + SU_G * u) * ld];
-#pragma unroll
-                for (int u = 0; u < SV_BK / SU_G; u++)
-#pragma unroll
-                    for (int q = 0; q < SV_RC; q++) acc[u][q] = fma(v[u], y[(SV_BK * c + i) * SV_RC + q], acc[u][q]);
-            }
-#pragma unroll
-            for (int u = 0; u < SV_BK / SU_G; u++)
-#pragma unroll
-                for (int q = 0; q < SV_RC; q++) {
-                    const double s = wsum(acc[u][q]);
-                    if (i == 0) pt[(g + SU_G * u) * SV_RC + q] = s;
-                }
-        }
-        __syncthreads();
-        if (g == 0) {
-            const int row = SV_BK * b + i;
-#pragma unroll
-            for (int q = 0; q < SV_RC; q++) {
-                double s = pt[i * SV_RC + q];
-                if (!trans)
-                    for (int gg = 1; gg < SU_G; gg++) s += pt[(gg * SV_BK + i) * SV_RC + q];
-                if (row < NB && q < nq) Po[row + (size_t)(r0 + q) * ldp] = s;
-            }
-        }
-        __syncthreads();
-    }
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void sf_st(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int sf_cnt(const int *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void sf_publish(int *cnt)
+{
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) atomicAdd(cnt, 1);
 }
 
-// w = F^T x (F = NB x r held as TE, x in LDS): wave g takes columns g + 16u,
-// its lanes run down the rows; w[c * SV_RC + q] in LDS
-template <typename TE>
-__device__ __forceinline__ void su_lr_w(const TE *F, int NB, int r, const double *x, double *w)
+// a[c][j] = F(r, cb + c), r = tid + 512 j, for the columns below c1, else 0; F
+// (NB rows) held in type pr.  The resource ends with column c1 - 1.
+template <int CC, int RT>
+__device__ __forceinline__ void sf_cols(double (&a)[CC][RT], const void *F, int pr, int NB, int tid, int cb, int c1)
 {
-    const int lane = threadIdx.x & 63, g = threadIdx.x >> 6;
-    for (int c = g; c < r; c += SU_G) {
-        const TE *Fc = F + (size_t)c * NB;
-        double acc[SV_RC];
+    const int es = pr == LR_F64 ? 8 : (pr == LR_F32 ? 4 : 2);
+    const wv_rsrc rs = wv_col_rsrc((const double *)F, c1 * NB * es);
+    int off[RT];
 #pragma unroll
-        for (int q = 0; q < SV_RC; q++) acc[q] = 0.0;
-#pragma unroll 4
-        for (int i = lane; i < NB; i += 64) {
-            const double fv = (double)Fc[i];
+    for (int j = 0; j < RT; j++) off[j] = tid + SF_T * j < NB ? (tid + SF_T * j) * es : (int)WV_OOB;
+    if (pr == LR_F64) {
 #pragma unroll
-            for (int q = 0; q < SV_RC; q++) acc[q] = fma(fv, x[i * SV_RC + q], acc[q]);
-        }
+        for (int c = 0; c < CC; c++)
 #pragma unroll
-        for (int q = 0; q < SV_RC; q++) {
-            const double v = wsum(acc[q]);
-            if (lane == 0) w[c * SV_RC + q] = v;
-        }
-    }
-}
-
-// P_o(row) -= G(row, :) w for every row, one row per thread (G = NB x r
-// held as TE)
-template <typename TE>
-__device__ __forceinline__ void su_lr_rows(const TE *G, int NB, int r, const double *w, double *Po, long ldp, int nq)
-{
-    for (int row = threadIdx.x; row < NB; row += SU_T) {
-        double acc[SV_RC];
+            for (int j = 0; j < RT; j++) a[c][j] = wv_lds(rs, off[j], (cb + c) * NB * 8);
+    } else if (pr == LR_F32) {
 #pragma unroll
-        for (int q = 0; q < SV_RC; q++) acc[q] = 0.0;
-#pragma unroll 4
-        for (int c = 0; c < r; c++) {
-            const double gv = (double)G[row + (size_t)c * NB];
+        for (int c = 0; c < CC; c++)
 #pragma unroll
-            for (int q = 0; q < SV_RC; q++) acc[q] = fma(gv, w[c * SV_RC + q], acc[q]);
-        }
-        for (int q = 0; q < nq; q++) Po[row + (size_t)q * ldp] -= acc[q];
-    }
-}
-
-// The update by the solved block k of one block of the right-hand sides in
-// Pupd, x_k read from Psol:
-// forward:  P_m -= L_mk x_k for m = k + 1 + tile, tile < ntile;
-// backward: P_j -= L_kj^T x_k for j = tile, tile < ntile = k;
-// the ndense tiles inside the band (the first ones forward, the last ones
-// backward) take one workgroup per 64-row block (rb), each low-rank tile one
-// workgroup: w = F^T x_k (F = V forward, U backward), then the rows of G w
-// (G = U forward, V backward).  Grid: ndense nb + (ntile - ndense).
-// LDS: x_k (NB x SV_RC), w (cap x SV_RC), partial sums (16 x 64 x SV_RC).
-__global__ void __launch_bounds__(SU_T) k_solve_update(TLR t, int k, const double *Psol, double *Pupd, long ldp,
-                                                       int nrhs, int trans, int ndense)
-{
-    extern __shared__ double sm[];
-    const int NB = t.NB, nb = (NB + SV_BK - 1) / SV_BK;
-    int tile, rb = -1;
-    if ((int)blockIdx.x < ndense * nb) {
-        const int d = blockIdx.x / nb;
-        rb = blockIdx.x - d * nb;
-        tile = trans ? k - ndense + d : d;
+            for (int j = 0; j < RT; j++) a[c][j] = (double)wv_lds32(rs, off[j], (cb + c) * NB * 4);
     } else {
-        const int e = blockIdx.x - ndense * nb;
-        tile = trans ? e : ndense + e;
+#pragma unroll
+        for (int c = 0; c < CC; c++)
+#pragma unroll
+            for (int j = 0; j < RT; j++) a[c][j] = (double)lr_bf16{wv_lds16(rs, off[j], (cb + c) * NB * 2)};
     }
-    double *xk = sm;                            // xk[l * SV_RC + q]
-    double *w = xk + (size_t)NB * SV_RC;        // w[c * SV_RC + q]
-    double *pt = w + (size_t)t.cap * SV_RC;     // pt[(g * 64 + i) * SV_RC + q]
-    const int tid = threadIdx.x, i = tid & 63, g = tid >> 6;
-    int m, n, o;
-    if (!trans) { m = k + 1 + tile; n = k; o = m; }
-    else { m = k; n = tile; o = n; }
-    const int r = (rb >= 0) ? 0 : *rank_at(t, m, n);
-    if (rb < 0 && r <= 0) return;
-    const double *T = (rb >= 0) ? band_tile(t, m, n) : lr_tile(t, m, n);
-    const int p = (rb >= 0) ? LR_F64 : lr_prec(t, m, n);
-    const double *Pk = Psol + (size_t)k * NB;
-    double *Po = Pupd + (size_t)o * NB;
-    const int row = SV_BK * rb + i;
-    for (int r0 = 0; r0 < nrhs; r0 += SV_RC) {
-        const int nq = min(SV_RC, nrhs - r0);
-        for (int e = tid; e < NB * SV_RC; e += SU_T) {
-            const int q = e / NB, l = e - q * NB;
-            xk[l * SV_RC + q] = (q < nq) ? Pk[l + (size_t)(r0 + q) * ldp] : 0.0;
-        }
+}
+
+// wave totals of N = 4, 8 or 16 values: lane l gets that of value l / (64 / N)
+__device__ __forceinline__ double sf_scatter(double (&p)[4]) { return wrs4(p[0], p[1], p[2], p[3]); }
+__device__ __forceinline__ double sf_scatter(double (&p)[8]) { return wrs8(p); }
+__device__ __forceinline__ double sf_scatter(double (&p)[16]) { return wrs16(p); }
+
+// columns of a low-rank share held in registers (a wider share takes several rounds)
+template <int RT>
+struct SfCfg {
+    static constexpr int CC = RT <= 2 ? 4 : 2;
+};
+
+// update tasks of a tile row: a dense tile needs more of them than a low-rank
+// one (sixteen against eight: 4.6 and 5.6 ms for eight right-hand sides at N=30011
+// band 16, 2.2 and 2.0 ms for one at N=90000 band 1)
+__host__ __device__ __forceinline__ int sf_shares(const TLR &t) { return t.band_size > 1 ? SF_GMAX : 8; }
+
+// Q right-hand sides of one pass over the rows r of the tiles, RT rows per
+// thread (r = tid + 512 j).  Position p of the order is tile row p (forward) or
+// NT-1-p (backward).  Task order: position, group of right-hand sides, then the
+// updates and the diagonal tasks.  cnt: [0] task counter, then per (position,
+// group) the finished update and diagonal tasks.  Pw: the shares' sums, NB x Q per
+// (position, group, share).  LDS: x or y (64 nb x Q), partial sums.
+template <int Q, int RT>
+__global__ void __launch_bounds__(SF_T, 4)
+k_solve_flow(TLR t, const double *Xinv, double *B, long ldb, int nrhs, int trans, double *Pw, int *cnt, int *stall)
+{
+    constexpr int CC = SfCfg<RT>::CC, NV = CC * Q <= 4 ? 4 : CC * Q;  // values of a reduction: 4, 8 or 16
+    extern __shared__ double sm[];
+    __shared__ int s_task, s_ready;
+    const int NB = t.NB, NT = t.NT, nb = (NB + SV_BK - 1) / SV_BK, ngrp = (nrhs + Q - 1) / Q;
+    const int G = sf_shares(t), nd = (NB + SF_RB - 1) / SF_RB, per = G + nd, ntask = NT * ngrp * per;
+    double *xs = sm;                          // xs[i * Q + q]
+    double *pt = sm + (size_t)nb * SV_BK * Q;  // 16 x 32 x Q
+    for (;;) {
+        // opaque, so that no address of one kind of task is kept through the other
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int lane = tid & 63, w = uni(tid >> 6);
+        __syncthreads();  // s_task and the LDS are free
+        if (tid == 0) s_task = atomicAdd(cnt, 1);
         __syncthreads();
-        if (rb < 0) {
-            const size_t off = (size_t)NB * r;
-            const int fo = trans ? 0 : 1;
-            double *Pq = Po + (size_t)r0 * ldp;
-            if (p == LR_F64) su_lr_w(T + fo * off, NB, r, xk, w);
-            else if (p == LR_F32) su_lr_w((const float *)T + fo * off, NB, r, xk, w);
-            else su_lr_w((const lr_bf16 *)T + fo * off, NB, r, xk, w);
-            __syncthreads();
-            if (p == LR_F64) su_lr_rows(T + (1 - fo) * off, NB, r, w, Pq, ldp, nq);
-            else if (p == LR_F32) su_lr_rows((const float *)T + (1 - fo) * off, NB, r, w, Pq, ldp, nq);
-            else su_lr_rows((const lr_bf16 *)T + (1 - fo) * off, NB, r, w, Pq, ldp, nq);
-            __syncthreads();
-            continue;
-        }
-        if (!trans) {
-            // P_m(row) -= sum_l L_mk(row, l) x_k(l): thread (i, g), l = g + 16u
-            double acc[SV_RC];
-#pragma unroll
-            for (int q = 0; q < SV_RC; q++) acc[q] = 0.0;
-            if (row < NB) {
-                const double *Tr = T + row;
-#pragma unroll 8
-                for (int l = g; l < NB; l += SU_G) {
-                    const double lv = Tr[(size_t)l * NB];
-#pragma unroll
-                    for (int q = 0; q < SV_RC; q++) acc[q] = fma(lv, xk[l * SV_RC + q], acc[q]);
-                }
-            }
-#pragma unroll
-            for (int q = 0; q < SV_RC; q++) pt[(g * SV_BK + i) * SV_RC + q] = acc[q];
-        } else {
-            // P_j(l) -= sum_i L_kj(i, l) x_k(i) for the 64 columns l of the row
-            // block: wave g takes l = 64 rb + g + 16u, its lanes run down i
-            for (int u = 0; u < SV_BK / SU_G; u++) {
-                const int l = SV_BK * rb + g + SU_G * u;
-                double a2[SV_RC];
-#pragma unroll
-                for (int q = 0; q < SV_RC; q++) a2[q] = 0.0;
-                if (l < NB) {
-                    const double *Tl = T + (size_t)l * NB;
-#pragma unroll 4
-                    for (int ii = i; ii < NB; ii += 64) {
-                        const double lv = Tl[ii];
-#pragma unroll
-                        for (int q = 0; q < SV_RC; q++) a2[q] = fma(lv, xk[ii * SV_RC + q], a2[q]);
+        const int task = uni(s_task);
+        if (task >= ntask) break;
+        const int row = task / per, sub = task - row * per, p = row / ngrp, grp = row - p * ngrp;
+        const int m = trans ? NT - 1 - p : p, q0 = grp * Q, nq = min(Q, nrhs - q0);
+        int *uc = cnt + 16 + 2 * row, *dc = uc + 1;
+        double *Pm = Pw + (size_t)row * G * NB * Q;
+        const int rows_m = tdim(t, m);
+        // thread 0 waits until *c reaches n
+        auto wait = [&](const int *c, int n) {
+            if (tid == 0) {
+                int k = 0;
+                while (sf_cnt(c) < n) {
+                    __builtin_amdgcn_s_sleep(1);
+                    if (++k > SF_SPIN_LIMIT) {
+                        __hip_atomic_store(stall, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        break;
                     }
                 }
+            }
+            __syncthreads();
+        };
+        if (sub < G) {
+            // ---- update: acc = b_m (share 0) - sum over earlier rows of its share
+            const int g = sub;
+            double acc[RT][Q];
 #pragma unroll
-                for (int q = 0; q < SV_RC; q++) {
-                    const double s = wsum(a2[q]);
-                    if (i == 0) pt[(g + SU_G * u) * SV_RC + q] = s;
+            for (int j = 0; j < RT; j++)
+#pragma unroll
+                for (int q = 0; q < Q; q++) {
+                    const int r = tid + SF_T * j;
+                    acc[j][q] = (g == 0 && r < rows_m && q < nq) ? B[(size_t)m * NB + r + (q0 + q) * ldb] : 0.0;
+                }
+            double v[CC][RT], u[CC][RT], x[RT][Q];
+            int ready = 0;
+            bool have = false, xhave = false;  // v and u hold the first round of the tile, x its x
+            // the share's columns c0 .. c1 of the tile at position pk, its factors
+            struct Sh {
+                const void *F, *G;  // w = F^T x, acc -= G w
+                size_t off;
+                int c0, c1, pr;
+                bool dense;
+            };
+            auto share = [&](int pk) {
+                const int k = trans ? NT - 1 - pk : pk, hi = trans ? k : m, lo = trans ? m : k;
+                Sh s;
+                s.dense = hi - lo < t.band_size;
+                s.c0 = s.c1 = 0;
+                s.F = s.G = nullptr;
+                s.pr = LR_F64;
+                if (!s.dense) {
+                    const int r = uni(max(*rank_at(t, hi, lo), 0)), cs = (r + G - 1) / G;
+                    s.c0 = min(r, g * cs);
+                    s.c1 = min(r, s.c0 + cs);
+                    s.pr = uni(lr_prec(t, hi, lo));
+                    const char *T = (const char *)lr_tile(t, hi, lo);
+                    const size_t vo = (size_t)NB * r * (s.pr == LR_F64 ? 8 : (s.pr == LR_F32 ? 4 : 2));
+                    s.F = trans ? T : T + vo;
+                    s.G = trans ? T + vo : T;
+                } else {
+                    s.F = band_tile(t, hi, lo);
+                }
+                return s;
+            };
+            auto load_x = [&](int pk) {
+                const int k = trans ? NT - 1 - pk : pk, rk = tdim(t, k);
+#pragma unroll
+                for (int q = 0; q < Q; q++) {
+                    const wv_rsrc rs = wv_col_rsrc(B + (size_t)k * NB + (q0 + (q < nq ? q : 0)) * ldb, q < nq ? rk * 8 : 0);
+#pragma unroll
+                    for (int j = 0; j < RT; j++) x[j][q] = wv_lds<true>(rs, (tid + SF_T * j) * 8, 0);
+                }
+            };
+            Sh cur = share(0);
+            for (int pk = 0; pk < p; pk++) {
+                if (!have && cur.c0 < cur.c1) {
+                    sf_cols(v, cur.F, cur.pr, NB, tid, cur.c0, cur.c1);
+                    sf_cols(u, cur.G, cur.pr, NB, tid, cur.c0, cur.c1);
+                }
+                if (pk >= ready) {  // how many rows from pk on are solved
+                    if (w == 0) {
+                        const int *c = cnt + 16 + 2 * ((pk + lane) * ngrp + grp) + 1;
+                        int n = 0, k = 0;
+                        for (;;) {
+                            const bool done = pk + lane < p && sf_cnt(c) >= nd;
+                            const unsigned long long open = ~__ballot(done);
+                            n = open ? __builtin_ctzll(open) : 64;
+                            if (n > 0) break;
+                            __builtin_amdgcn_s_sleep(1);
+                            if (++k > SF_SPIN_LIMIT) {
+                                if (lane == 0) __hip_atomic_store(stall, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                                n = 1;
+                                break;
+                            }
+                        }
+                        if (lane == 0) s_ready = pk + n;
+                    }
+                    __syncthreads();
+                    ready = uni(s_ready);
+                    __syncthreads();
+                }
+                if (cur.dense) {
+                    const wv_rsrc T = wv_col_rsrc((const double *)cur.F, NB * NB * 8);
+                    const int k = trans ? NT - 1 - pk : pk, rk = tdim(t, k);
+                    // share g of the columns of T
+                    const int cs = (NB + G - 1) / G, l0 = min(NB, g * cs), l1 = min(NB, l0 + cs);
+                    const int i0 = trans ? 0 : l0, i1 = trans ? NB : l1;  // rows of x_k it needs
+                    for (int e = tid; e < (i1 - i0) * Q; e += SF_T) {
+                        const int q = e / (i1 - i0), i = i0 + e - q * (i1 - i0);
+                        xs[i * Q + q] = (i < rk && q < nq) ? sf_ld(B + (size_t)k * NB + i + (q0 + q) * ldb) : 0.0;
+                    }
+                    __syncthreads();
+                    if (!trans) {  // acc(r) -= sum over the share's columns T(r, l) x(l)
+#pragma unroll
+                        for (int j = 0; j < RT; j++) {
+                            const int r = tid + SF_T * j;
+                            if (r < NB) {
+#pragma unroll 8
+                                for (int l = l0; l < l1; l++) {
+                                    const double tv = wv_lds(T, r * 8, l * NB * 8);
+#pragma unroll
+                                    for (int q = 0; q < Q; q++) acc[j][q] = fma(-tv, xs[l * Q + q], acc[j][q]);
+                                }
+                            }
+                        }
+                    } else {  // acc(l) -= T(:, l)^T x for the share's columns l, one wave each in turn
+                        double *ob = pt;
+                        for (int l = l0 + w; l < l1; l += SF_W) {
+                            double d[Q];
+#pragma unroll
+                            for (int q = 0; q < Q; q++) d[q] = 0.0;
+#pragma unroll 8
+                            for (int i = lane; i < NB; i += 64) {
+                                const double tv = wv_lds(T, i * 8, uni(l) * NB * 8);
+#pragma unroll
+                                for (int q = 0; q < Q; q++) d[q] = fma(tv, xs[i * Q + q], d[q]);
+                            }
+#pragma unroll
+                            for (int q = 0; q < Q; q++) {
+                                const double sv = wsum(d[q]);
+                                if (lane == 0) ob[(l - l0) * Q + q] = sv;
+                            }
+                        }
+                        __syncthreads();
+#pragma unroll
+                        for (int j = 0; j < RT; j++) {
+                            const int r = tid + SF_T * j;
+                            if (r >= l0 && r < l1) {
+#pragma unroll
+                                for (int q = 0; q < Q; q++) acc[j][q] -= ob[(r - l0) * Q + q];
+                            }
+                        }
+                    }
+                    __syncthreads();
+                }
+                const Sh now = cur;
+                if (now.c0 < now.c1 && !xhave) load_x(pk);
+                if (pk + 1 < p) cur = share(pk + 1);
+                have = xhave = false;
+                for (int cb = now.c0; cb < now.c1; cb += CC) {
+                    // w = F^T x: the products summed over the rows of all waves
+                    double pr[NV];
+#pragma unroll
+                    for (int e = 0; e < NV; e++) pr[e] = 0.0;
+#pragma unroll
+                    for (int c = 0; c < CC; c++)
+#pragma unroll
+                        for (int q = 0; q < Q; q++)
+#pragma unroll
+                            for (int j = 0; j < RT; j++) pr[c * Q + q] = fma(v[c][j], x[j][q], pr[c * Q + q]);
+                    const double part = sf_scatter(pr);
+                    if (lane % (64 / NV) == 0) pt[w * 16 + lane / (64 / NV)] = part;
+                    // v is free: the next round, or the next tile's first one (and its x,
+                    // if that row is solved), loads while this one goes on
+                    const bool last = cb + CC >= now.c1, next = last && pk + 1 < p && cur.c0 < cur.c1;
+                    if (!last) sf_cols(v, now.F, now.pr, NB, tid, cb + CC, now.c1);
+                    if (next) {
+                        sf_cols(v, cur.F, cur.pr, NB, tid, cur.c0, cur.c1);
+                        if (pk + 1 < ready) {
+                            load_x(pk + 1);
+                            xhave = true;
+                        }
+                    }
+                    __syncthreads();
+                    // lanes 4e .. 4e+3 add value e's eight parts
+                    double tot = pt[(2 * (lane & 3)) * 16 + (lane >> 2)] + pt[(2 * (lane & 3) + 1) * 16 + (lane >> 2)];
+                    tot += dppd<DPP_XOR1>(tot);
+                    tot += dppd<DPP_XOR2>(tot);
+#pragma unroll
+                    for (int c = 0; c < CC; c++)
+#pragma unroll
+                        for (int q = 0; q < Q; q++) {
+                            const double wv = rdlane(tot, 4 * (c * Q + q));
+#pragma unroll
+                            for (int j = 0; j < RT; j++) acc[j][q] = fma(-u[c][j], wv, acc[j][q]);
+                        }
+                    if (!last) sf_cols(u, now.G, now.pr, NB, tid, cb + CC, now.c1);
+                    if (next) {
+                        sf_cols(u, cur.G, cur.pr, NB, tid, cur.c0, cur.c1);
+                        have = true;
+                    }
+                    __syncthreads();  // pt is free
                 }
             }
-        }
-        __syncthreads();
-        if (g == 0 && row < NB) {
 #pragma unroll
-            for (int q = 0; q < SV_RC; q++) {
-                double s = pt[i * SV_RC + q];
-                if (!trans)
-                    for (int gg = 1; gg < SU_G; gg++) s += pt[(gg * SV_BK + i) * SV_RC + q];
-                if (q < nq) Po[row + (size_t)(r0 + q) * ldp] -= s;
+            for (int j = 0; j < RT; j++)
+#pragma unroll
+                for (int q = 0; q < Q; q++) {
+                    const int r = tid + SF_T * j;
+                    if (r < NB) sf_st(Pm + ((size_t)g * Q + q) * NB + r, acc[j][q]);
+                }
+            sf_publish(uc);
+            continue;
+        }
+        // ---- diagonal: 32 rows of L_mm^-1 y or L_mm^-T y
+        const int h = sub - G, b = h >> 1;
+        const double *X0 = Xinv + (size_t)m * inv_tile(nb);
+        // forward: thread (row i, column group cg): columns cg + 16 e of block (b, c), c <= b;
+        // backward: wave w takes columns 4 w .. 4 w + 3 of the 32, lanes run down the rows of
+        // block (c, b), c >= b
+        const int i32 = tid & 31, cg = tid >> 5, ro = 32 * (h & 1);
+        const wv_rsrc xr = wv_col_rsrc(X0, (int)inv_tile(nb) * 8);
+        const int eo = trans ? (lane + SV_BK * (ro + 4 * w)) * 8 : (ro + i32 + SV_BK * cg) * 8;
+        auto elem = [&](int cc, int e) -> double {  // cc-th block of the product
+            const int blk = (int)(trans ? inv_blk(b + cc, b) : inv_blk(b, cc)) * SV_BK * SV_BK * 8;
+            return wv_lds(xr, eo + (trans ? SV_BK * 8 : 16 * SV_BK * 8) * e, blk);
+        };
+        const int nblk = trans ? nb - b : b + 1;
+        double pf[SF_PF][4];
+#pragma unroll
+        for (int cc = 0; cc < SF_PF; cc++)
+            if (cc < nblk) {
+#pragma unroll
+                for (int e = 0; e < 4; e++) pf[cc][e] = elem(cc, e);
             }
+        wait(uc, G);
+        for (int e = tid; e < nb * SV_BK * Q; e += SF_T) {
+            const int q = e / (nb * SV_BK), i = e - q * (nb * SV_BK);
+            double s = 0.0;
+            if (i < NB) {
+                for (int g0 = 0; g0 < G; g0 += 8) {
+                    double pv[8];
+#pragma unroll
+                    for (int g = 0; g < 8; g++) pv[g] = sf_ld(Pm + (unsigned)(((g0 + g) * Q + q) * NB + i));
+#pragma unroll
+                    for (int g = 0; g < 8; g++) s += pv[g];
+                }
+            }
+            xs[i * Q + q] = s;
         }
         __syncthreads();
+        double a[4 * Q];
+#pragma unroll
+        for (int e = 0; e < 4 * Q; e++) a[e] = 0.0;
+        if (!trans) {
+#pragma unroll
+            for (int cc = 0; cc < SF_PF; cc++)
+                if (cc < nblk) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int i = SV_BK * cc + cg + 16 * e;
+#pragma unroll
+                        for (int q = 0; q < Q; q++) a[q] = fma(pf[cc][e], xs[i * Q + q], a[q]);
+                    }
+                }
+#pragma unroll 2
+            for (int cc = SF_PF; cc < nblk; cc++) {
+                double f[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) f[e] = elem(cc, e);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int i = SV_BK * cc + cg + 16 * e;
+#pragma unroll
+                    for (int q = 0; q < Q; q++) a[q] = fma(f[e], xs[i * Q + q], a[q]);
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < Q; q++) pt[(cg * 32 + i32) * Q + q] = a[q];
+            __syncthreads();
+            for (int e = tid; e < 32 * nq; e += SF_T) {
+                const int q = e >> 5, i = e & 31, r = SF_RB * h + i;
+                double s = 0.0;
+#pragma unroll
+                for (int c = 0; c < 16; c++) s += pt[(c * 32 + i) * Q + q];
+                if (r < rows_m) sf_st(B + (size_t)m * NB + r + (q0 + q) * ldb, s);
+            }
+        } else {
+#pragma unroll
+            for (int cc = 0; cc < SF_PF; cc++)
+                if (cc < nblk) {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) {
+                        const int i = SV_BK * (b + cc) + lane;
+#pragma unroll
+                        for (int q = 0; q < Q; q++) a[e * Q + q] = fma(pf[cc][e], xs[i * Q + q], a[e * Q + q]);
+                    }
+                }
+#pragma unroll 2
+            for (int cc = SF_PF; cc < nblk; cc++) {
+                double f[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) f[e] = elem(cc, e);
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int i = SV_BK * (b + cc) + lane;
+#pragma unroll
+                    for (int q = 0; q < Q; q++) a[e * Q + q] = fma(f[e], xs[i * Q + q], a[e * Q + q]);
+                }
+            }
+#pragma unroll
+            for (int e = 0; e < 4; e++)
+#pragma unroll
+                for (int q = 0; q < Q; q++) {
+                    const double s = wsum(a[e * Q + q]);
+                    const int r = SF_RB * h + 4 * w + e;
+                    if (lane == 0 && q < nq && r < rows_m) sf_st(B + (size_t)m * NB + r + (q0 + q) * ldb, s);
+                }
+        }
+        sf_publish(dc);
     }
 }
 
-// P (ld ldp, NT NB rows) <- B (ld ldb, N rows), padding rows zeroed; or back
-__global__ void k_pad_copy(const double *src, long lds, double *dst, long ldd, int rows_src, int rows_dst, int nrhs)
+__global__ void k_sf_zero(int *p, int n)
 {
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= (long)rows_dst * nrhs) return;
-    const int q = (int)(e / rows_dst), i = (int)(e - (long)q * rows_dst);
-    dst[i + q * ldd] = (i < rows_src) ? src[i + q * lds] : 0.0;
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e < n) p[e] = 0;
 }
 
 // sum of squares of x(0 : n), per-block parts, and their fixed-order total
@@ -378,14 +548,29 @@ __global__ void __launch_bounds__(256) k_sum_seq(const double *part, int n, doub
 // ---------------------------------------------------------------------------
 // host side
 
-// doubles of workspace a solve needs: the panels of every L_kk^-1, two
-// padded right-hand-side blocks (a pass reads one and writes the other),
-// reduction parts (of the sum of squares, then of the log-det), three scalars
-size_t solve_ws_doubles(const TLR &t, int nrhs)
+// right-hand sides per group (groups of eight spill: 7.9 instead of 4.6 ms for
+// eight right-hand sides at N=30011 band 16)
+static int solve_q(int nrhs) { return nrhs >= 3 ? 4 : nrhs; }
+
+// doubles of workspace a solve needs: every L_kk^-1 (unless the descriptor
+// has them), the shares' sums, the counters, reduction parts (of the sum of
+// squares, then of the log-det), eight scalars
+static size_t solve_pw(const TLR &t, int nrhs)
+{
+    const size_t Q = solve_q(nrhs), ngrp = (nrhs + Q - 1) / Q;
+    return (size_t)t.NT * ngrp * sf_shares(t) * t.NB * Q;
+}
+static size_t solve_cnt(const TLR &t, int nrhs)
+{
+    const size_t Q = solve_q(nrhs), ngrp = (nrhs + Q - 1) / Q;
+    return 16 + 2 * (size_t)t.NT * ngrp;
+}
+size_t solve_ws_doubles(const TLR &t, int nrhs, bool have_inv)
 {
     const int nbk = (t.NB + SV_BK - 1) / SV_BK;
     const size_t Np = (size_t)t.NT * t.NB;
-    return (size_t)t.NT * inv_tile(nbk) + 2 * Np * (size_t)nrhs + std::max((Np + 255) / 256, (size_t)t.NT) + 8;
+    return (have_inv ? 0 : (size_t)t.NT * inv_tile(nbk)) + solve_pw(t, nrhs) + solve_cnt(t, nrhs) / 2 + 1 +
+           std::max((Np + 255) / 256, (size_t)t.NT) + 8;
 }
 
 size_t hicma_solve_bytes(int N, int NB)
@@ -394,17 +579,46 @@ size_t hicma_solve_bytes(int N, int NB)
     t.N = N;
     t.NB = NB;
     t.NT = (N + NB - 1) / NB;
-    return sizeof(double) * solve_ws_doubles(t, 1);
+    return sizeof(double) * solve_ws_doubles(t, 1, true);
 }
 
+// LDS the solve kernels of four right-hand sides may take (the limit of the
+// tile and rank sizes)
 static size_t diag_lds(const TLR &t)
 {
     const size_t nbk = (size_t)(t.NB + SV_BK - 1) / SV_BK;
-    return sizeof(double) * (nbk * SV_BK * SV_RC + (size_t)SU_G * SV_BK * SV_RC);
+    return sizeof(double) * (nbk * SV_BK * 4 + 4096);
 }
-static size_t update_lds(const TLR &t)
+static size_t update_lds(const TLR &t) { return sizeof(double) * (((size_t)t.NB + (size_t)t.cap) * 4 + 4096); }
+
+template <int Q, int RT>
+static int flow_launch_qr(hicma_ctx *ctx, const TLR &t, const double *Xinv, double *B, long ldb, int nrhs, int trans,
+                          double *Pw, int *cnt)
 {
-    return sizeof(double) * (((size_t)t.NB + (size_t)t.cap) * SV_RC + (size_t)SU_G * SV_BK * SV_RC);
+    const int nb = (t.NB + SV_BK - 1) / SV_BK, ngrp = (nrhs + Q - 1) / Q;
+    const int per = sf_shares(t) + (t.NB + SF_RB - 1) / SF_RB;
+    // a transposed dense share of up to NB / 8 columns, or 16 x 32 partial sums
+    const size_t part = std::max<size_t>(512, (size_t)t.NB / 8 + 1);
+    const size_t lds = sizeof(double) * ((size_t)nb * SV_BK + part) * Q;
+    const auto kern = k_solve_flow<Q, RT>;
+    HIPCHK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    const int ncnt = (int)solve_cnt(t, nrhs);
+    hipLaunchKernelGGL(k_sf_zero, dim3((unsigned)((ncnt + 255) / 256)), dim3(256), 0, ctx->stream, cnt, ncnt);
+    // two workgroups per CU
+    const long ntask = (long)t.NT * ngrp * per;
+    hipLaunchKernelGGL(kern, dim3((unsigned)std::min<long>(2L * ctx->ncu, ntask)), dim3(SF_T), lds, ctx->stream, t,
+                       Xinv, B, ldb, nrhs, trans, Pw, cnt, ctx->d_stall);
+    return 0;
+}
+template <int Q>
+static int flow_launch_q(hicma_ctx *ctx, const TLR &t, const double *Xinv, double *B, long ldb, int nrhs, int trans,
+                         double *Pw, int *cnt)
+{
+    // rows per thread
+    if (t.NB <= SF_T) return flow_launch_qr<Q, 1>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
+    if (t.NB <= 2 * SF_T) return flow_launch_qr<Q, 2>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
+    if (t.NB <= 4 * SF_T) return flow_launch_qr<Q, 4>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
+    return flow_launch_qr<Q, 8>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
 }
 
 // dirs: 1 forward, 2 backward, 3 both.  B: device, N x nrhs, ld ldb.
@@ -415,49 +629,44 @@ int solve_launch(hicma_ctx *ctx, hicma_tlr_desc *A, int dirs, int nrhs, double *
 {
     const TLR &t = A->t;
     const int NT = t.NT, NB = t.NB, nbk = (NB + SV_BK - 1) / SV_BK;
-    const long Np = (long)NT * NB;
     hipStream_t st = ctx->stream;
-    double *Xinv = ws;
-    double *P0 = Xinv + (size_t)NT * inv_tile(nbk);
-    double *P1 = P0 + (size_t)Np * nrhs;
-    double *parts = P1 + (size_t)Np * nrhs;
-    const size_t ld1 = diag_lds(t), ld2 = update_lds(t);
-    HIPCHK(hipFuncSetAttribute((const void *)k_solve_diag, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ld1));
-    HIPCHK(hipFuncSetAttribute((const void *)k_solve_update, hipFuncAttributeMaxDynamicSharedMemorySize, (int)ld2));
-    hipLaunchKernelGGL(k_tri_inv, dim3((unsigned)(NT * nbk)), dim3(64), 0, st, t, Xinv);
-    if (nbk > 1) hipLaunchKernelGGL(k_tile_inv, dim3((unsigned)(NT * nbk)), dim3(256), 0, st, t, Xinv);
-    const long ne = Np * nrhs;
-    hipLaunchKernelGGL(k_pad_copy, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, st, (const double *)B, ldb, P0, Np,
-                       t.N, (int)Np, nrhs);
-    // each pass reads the right-hand sides from src, leaves its solution in dst
-    double *src = P0, *dst = P1;
+    const double *Xinv = A->linv;
+    double *Pw = ws;
+    if (!A->linv_ok) {
+        hipLaunchKernelGGL(k_tri_inv, dim3((unsigned)(NT * nbk)), dim3(64), 0, st, t, ws);
+        if (nbk > 1) hipLaunchKernelGGL(k_tile_inv, dim3((unsigned)(NT * nbk)), dim3(256), 0, st, t, ws);
+        Xinv = ws;
+        Pw = ws + (size_t)NT * inv_tile(nbk);
+    }
+    int *cnt = (int *)(Pw + solve_pw(t, nrhs));
+    double *parts = (double *)cnt + solve_cnt(t, nrhs) / 2 + 1;
+    *ctx->h_stall = 0;
     auto pass = [&](int trans) {
-        for (int s = 0; s < NT; s++) {
-            const int k = trans ? NT - 1 - s : s;
-            hipLaunchKernelGGL(k_solve_diag, dim3((unsigned)nbk), dim3(SU_T), ld1, st, t, k, (const double *)Xinv,
-                               (const double *)src, dst, Np, nrhs, trans);
-            const int ntile = trans ? k : NT - 1 - k;
-            const int ndense = std::min(t.band_size - 1, ntile);
-            if (ntile > 0)
-                hipLaunchKernelGGL(k_solve_update, dim3((unsigned)(ndense * nbk + ntile - ndense)), dim3(SU_T), ld2,
-                                   st, t, k, (const double *)dst, src, Np, nrhs, trans, ndense);
-        }
-        std::swap(src, dst);
+        const int Q = solve_q(nrhs);
+        if (Q == 1) return flow_launch_q<1>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
+        if (Q == 2) return flow_launch_q<2>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
+        return flow_launch_q<4>(ctx, t, Xinv, B, ldb, nrhs, trans, Pw, cnt);
     };
     if (dirs & 1) {
-        pass(0);
+        RCHK(pass(0));
         if (d_quad) {
             const int nb = (int)((t.N + 255) / 256);
-            hipLaunchKernelGGL(k_sumsq_parts, dim3(nb), dim3(256), 0, st, (const double *)src, t.N, parts);
+            hipLaunchKernelGGL(k_sumsq_parts, dim3(nb), dim3(256), 0, st, (const double *)B, t.N, parts);
             hipLaunchKernelGGL(k_sum_seq, dim3(1), dim3(256), 0, st, (const double *)parts, nb, d_quad);
         }
     }
-    if (dirs & 2) pass(1);
+    if (dirs & 2) RCHK(pass(1));
     if (d_logdet) logdet_launch(t, parts, d_logdet, st);
-    hipLaunchKernelGGL(k_pad_copy, dim3((unsigned)(((long)t.N * nrhs + 255) / 256)), dim3(256), 0, st,
-                       (const double *)src, Np, B, ldb, (int)Np, t.N, nrhs);
     HIPCHK(hipGetLastError());
     return 0;
+}
+
+// after the stream has been waited for: whether a bounded device wait ran out
+int solve_stalled(hicma_ctx *ctx)
+{
+    if (!*(volatile int *)ctx->h_stall) return 0;
+    fprintf(stderr, "hicma_tlr: a wait of the solve's schedule ran out; the result is not valid\n");
+    return HICMA_ERR_HIP;
 }
 
 int check_solve_args(hicma_ctx *ctx, hicma_tlr_desc *A, int nrhs, const double *B, long ldb)
@@ -472,20 +681,20 @@ extern "C" int hicma_tlr_trsm(hicma_ctx *ctx, hicma_tlr_desc *A, int trans, int 
     RCHK(check_solve_args(ctx, A, nrhs, B, ldb));
     if (trans != 0 && trans != 1) return HICMA_ERR_ARG;
     HIPCHK(hipSetDevice(ctx->device));
-    RCHK(hicma_ensure_ws(ctx, sizeof(double) * solve_ws_doubles(A->t, nrhs)));
+    RCHK(hicma_ensure_ws(ctx, sizeof(double) * solve_ws_doubles(A->t, nrhs, A->linv_ok)));
     RCHK(solve_launch(ctx, A, trans ? 2 : 1, nrhs, B, ldb, ctx->ws, nullptr, nullptr));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    return 0;
+    return solve_stalled(ctx);
 }
 
 extern "C" int hicma_tlr_potrs(hicma_ctx *ctx, hicma_tlr_desc *A, int nrhs, double *B, int ldb)
 {
     RCHK(check_solve_args(ctx, A, nrhs, B, ldb));
     HIPCHK(hipSetDevice(ctx->device));
-    RCHK(hicma_ensure_ws(ctx, sizeof(double) * solve_ws_doubles(A->t, nrhs)));
+    RCHK(hicma_ensure_ws(ctx, sizeof(double) * solve_ws_doubles(A->t, nrhs, A->linv_ok)));
     RCHK(solve_launch(ctx, A, 3, nrhs, B, ldb, ctx->ws, nullptr, nullptr));
     HIPCHK(hipStreamSynchronize(ctx->stream));
-    return 0;
+    return solve_stalled(ctx);
 }
 
 // log-likelihood of one vector z (device, N entries; overwritten by L^-1 z)
@@ -496,6 +705,7 @@ int loglik_finish(hicma_ctx *ctx, const TLR &t, double *d_vals, double *logdet, 
     // waits for its stream holds the runtime's staging path meanwhile, and
     // other threads' copies queue behind it
     HIPCHK(hipStreamSynchronize(ctx->stream));
+    RCHK(solve_stalled(ctx));
     HIPCHK(hipMemcpy(h, d_vals, 2 * sizeof(double), hipMemcpyDeviceToHost));
     if (quad) *quad = h[0];
     if (logdet) *logdet = h[1];
@@ -508,7 +718,7 @@ extern "C" int hicma_tlr_loglik(hicma_ctx *ctx, hicma_tlr_desc *A, double *z, do
 {
     RCHK(check_solve_args(ctx, A, 1, z, A ? A->t.N : 0));
     HIPCHK(hipSetDevice(ctx->device));
-    const size_t need = solve_ws_doubles(A->t, 1);
+    const size_t need = solve_ws_doubles(A->t, 1, A->linv_ok);
     RCHK(hicma_ensure_ws(ctx, sizeof(double) * need));
     double *vals = ctx->ws + need - 8;
     RCHK(solve_launch(ctx, A, 1, 1, z, A->t.N, ctx->ws, vals, vals + 1));

@@ -154,6 +154,9 @@ extern "C" int hicma_init_ex(hicma_ctx **ctx, int device, int flags, int cu_shar
     HIPCHK(hipMemset(c->d_info, 0, 4 * sizeof(int)));
     c->d_ovf = c->d_info + 1;
     HIPCHK(hipMalloc(&c->d_scalar, 8 * sizeof(double)));
+    HIPCHK(hipHostMalloc((void **)&c->h_stall, 64, hipHostMallocMapped));
+    *c->h_stall = 0;
+    HIPCHK(hipHostGetDevicePointer((void **)&c->d_stall, c->h_stall, 0));
     RCHK(hicma_noalloc_setup(device));
     *ctx = c;
     return 0;
@@ -183,6 +186,7 @@ extern "C" int hicma_fini(hicma_ctx *c)
     hipStreamSynchronize(c->stream);
     hipFree(c->d_info);
     hipFree(c->d_scalar);
+    hipHostFree(c->h_stall);
     for (auto e : c->prof_ev) (void)hipEventDestroy(e);
     for (auto e : c->cp_ev) (void)hipEventDestroy(e);
     if (c->blas && c->blas_free) c->blas_free(c->blas);
@@ -284,6 +288,7 @@ extern "C" int hicma_desc_destroy(hicma_tlr_desc *A)
     ctx_free(c, A->d_tileops);
     ctx_free(c, A->d_opstat);
     ctx_free(c, A->rhist);
+    ctx_free(c, A->linv);
     if (A->gexec) (void)hipGraphExecDestroy(A->gexec);
     if (A->graph) (void)hipGraphDestroy(A->graph);
     free(A->h_xyz);
@@ -327,6 +332,7 @@ static int alloc_band(hicma_tlr_desc *A, int band_size)
 static int gen_band_tiles(hicma_tlr_desc *A)
 {
     TLR &t = A->t;
+    A->linv_ok = 0;
     dim3 grid((unsigned)(((size_t)t.NB * t.NB + BS - 1) / BS), (unsigned)(t.band_size * t.NT));
     hipLaunchKernelGGL(k_gen_band, grid, dim3(BS), 0, A->ctx->stream, t, 0);
     HIPCHK(hipGetLastError());
@@ -747,7 +753,7 @@ struct PotrfWs {
     RbWs gb;    // k_rc_big
     int ns, nbig, wgrid, wres, wcap;
     bool big, wave;
-    size_t rc_lds, winv_d, dag_d, linv_d, wws_d, wlist_d, lrd_pairs, syrk_d, lrd_d, qn_d, total;
+    size_t rc_lds, dag_d, linv_d, wws_d, wlist_d, lrd_pairs, syrk_d, lrd_d, qn_d, total;
 };
 
 static void plan_potrf_ws(hicma_ctx *ctx, int NT, int NB, int cap, int b, PotrfWs &P)
@@ -771,12 +777,11 @@ static void plan_potrf_ws(hicma_ctx *ctx, int NT, int NB, int cap, int b, PotrfW
     P.syrk_d = (size_t)NT * NB * cap + (size_t)NT * cap * cap;
     P.lrd_pairs = (b > 1) ? (size_t)NT * (b - 1) : 0;
     P.lrd_d = P.lrd_pairs * ((size_t)cap * NB + (size_t)cap * cap);
-    P.winv_d = (size_t)((NB + PBK - 1) / PBK) * PBK * PBK;
     // the diagonal potrf's task counter and done flags (ints packed in
-    // doubles) and the blocks of L_kk^-1
+    // doubles) and one tile's L_kk^-1
     const size_t nbk = (size_t)((NB + PBK - 1) / PBK);
     P.dag_d = (nbk * nbk + 2 + 1) / 2 + 1;
-    P.linv_d = nbk * nbk * PBK * PBK;
+    P.linv_d = inv_tile((int)nbk);
     // one-wave recompression (tasks with s <= WV_S2MAX): the s <= 32 and
     // s <= 48 variants run 4 waves per workgroup, s <= 64 two
     P.wave = P.big && (NB <= 64 * WV_KMAX);
@@ -791,10 +796,10 @@ static void plan_potrf_ws(hicma_ctx *ctx, int NT, int NB, int cap, int b, PotrfW
     // Qn = -B Av of the dense-B tasks with stacks up to QN_COLS (2-flow only)
     P.qn_d = (P.wave && b > 1) ? (size_t)(b - 1) * (NT - 1) * NB * QN_COLS : 0;
     // every part on a 128-byte line
-    for (size_t *d : {&g.stride, &P.gb.stride, &P.syrk_d, &P.lrd_d, &P.winv_d, &P.dag_d, &P.linv_d, &P.wws_d,
+    for (size_t *d : {&g.stride, &P.gb.stride, &P.syrk_d, &P.lrd_d, &P.dag_d, &P.linv_d, &P.wws_d,
                       &P.wlist_d, &P.qn_d})
         *d = (*d + 15) / 16 * 16;
-    P.total = g.stride * P.ns + P.gb.stride * P.nbig + P.syrk_d + P.lrd_d + P.winv_d + P.wws_d + P.wlist_d + P.dag_d +
+    P.total = g.stride * P.ns + P.gb.stride * P.nbig + P.syrk_d + P.lrd_d + P.wws_d + P.wlist_d + P.dag_d +
               P.linv_d + P.qn_d;
 }
 
@@ -817,13 +822,14 @@ size_t hicma_desc_bytes(int N, int NB, int cap, int band, int ndim)
 {
     const size_t NT = (size_t)(N + NB - 1) / NB;
     return sizeof(double) * (size_t)ndim * N + sizeof(int) * NT * NT + sizeof(double) * NT * (NT - 1) / 2 * NB * 2 * cap +
-           sizeof(unsigned long long) * (NT * NT + 16) + sizeof(double) * (size_t)band * NT * NB * NB + NT * NT;
+           sizeof(unsigned long long) * (NT * NT + 16) + sizeof(double) * (size_t)band * NT * NB * NB + NT * NT +
+           sizeof(double) * NT * inv_tile((NB + PBK - 1) / PBK);
 }
 
 // blocked Cholesky of diagonal tile k: per 64-column block, factor + invert
 // the diagonal block in LDS, panel = C W^T, lower trailing update.  The block
-// inverses (Winv, NB/64 blocks of 64x64) are reused by the low-rank trsm.
-static int launch_potrf(hicma_tlr_desc *A, int k, double *Winv, double *Linv, int *dflags, OpLog o, hipStream_t s)
+// inverse Inv (inv_blk) is reused by the trsms and the solves.
+static int launch_potrf(hicma_tlr_desc *A, int k, double *Inv, int *dflags, OpLog o, hipStream_t s)
 {
     TLR &t = A->t;
     const int nb = (t.NB + PBK - 1) / PBK;
@@ -831,8 +837,8 @@ static int launch_potrf(hicma_tlr_desc *A, int k, double *Winv, double *Linv, in
     // one worker per block column (a whole column of tasks can run at once),
     // on the XCD that the kernel elects among DAG_XCD_SPREAD times as many
     // workgroups
-    hipLaunchKernelGGL(k_potrf_dag, dim3(nb * DAG_XCD_SPREAD), dim3(BS), sizeof(double) * DAG_SMEM, s, t, k, Winv,
-                       Linv, dflags, A->ctx->d_info, A->ctx->d_info + 3, o);
+    hipLaunchKernelGGL(k_potrf_dag, dim3(nb * DAG_XCD_SPREAD), dim3(BS), sizeof(double) * DAG_SMEM, s, t, k, Inv,
+                       dflags, A->ctx->d_info, A->ctx->d_info + 3, o);
     HIPCHK(hipGetLastError());
     return 0;
 }
@@ -847,17 +853,17 @@ static int trsm_tc(int NB)
     return 0;
 }
 
-static void launch_trsm_lr(TLR &t, int k, int nlr, int cap, const double *Winv, const double *Linv, OpLog o,
+static void launch_trsm_lr(TLR &t, int k, int nlr, int cap, const double *Inv, OpLog o,
                            hipStream_t s)
 {
     const int tc = trsm_tc(t.NB);
     const size_t lds = sizeof(double) * ((size_t)PBK * ((t.NB + PBK - 1) / PBK) + 1) * tc;
     const dim3 grid((cap + tc - 1) / tc, nlr);
     switch (tc) {
-    case 16: hipLaunchKernelGGL(k_trsm_lr_inv<16>, grid, dim3(BS), lds, s, t, k, Winv, Linv, o); break;
-    case 8: hipLaunchKernelGGL(k_trsm_lr_inv<8>, grid, dim3(BS), lds, s, t, k, Winv, Linv, o); break;
-    case 4: hipLaunchKernelGGL(k_trsm_lr_inv<4>, grid, dim3(BS), lds, s, t, k, Winv, Linv, o); break;
-    default: hipLaunchKernelGGL(k_trsm_lr_inv<2>, grid, dim3(BS), lds, s, t, k, Winv, Linv, o); break;
+    case 16: hipLaunchKernelGGL(k_trsm_lr_inv<16>, grid, dim3(BS), lds, s, t, k, Inv, o); break;
+    case 8: hipLaunchKernelGGL(k_trsm_lr_inv<8>, grid, dim3(BS), lds, s, t, k, Inv, o); break;
+    case 4: hipLaunchKernelGGL(k_trsm_lr_inv<4>, grid, dim3(BS), lds, s, t, k, Inv, o); break;
+    default: hipLaunchKernelGGL(k_trsm_lr_inv<2>, grid, dim3(BS), lds, s, t, k, Inv, o); break;
     }
 }
 
@@ -909,13 +915,21 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     double *Zws = Yws + (size_t)NT * NB * cap;
     double *Wws = Yws + P.syrk_d;
     double *Xws = Wws + P.lrd_pairs * cap * NB;
-    double *Winv = Wws + P.lrd_d;
-    double *wws = Winv + P.winv_d;
+    double *wws = Wws + P.lrd_d;
     int *wcount = (int *)(wws + P.wws_d);             // 16 counters (k_classify_wave)
     int *wlist = wcount + 16;
-    double *Linv = (double *)wcount + P.wlist_d;
-    double *qnws = P.qn_d ? Linv + P.linv_d : nullptr;
-    int *dflags = (int *)(Linv + P.linv_d + P.qn_d);
+    double *inv1 = (double *)wcount + P.wlist_d;       // one tile's inverse, when the descriptor keeps none
+    double *qnws = P.qn_d ? inv1 + P.linv_d : nullptr;
+    int *dflags = (int *)(inv1 + P.linv_d + P.qn_d);
+    // every L_kk^-1 stays with the factor, for the solves (without the memory for
+    // it they form it themselves)
+    const size_t invk = inv_tile((NB + PBK - 1) / PBK);
+    A->linv_ok = 0;
+    if (!A->linv && ctx_malloc(ctx, (void **)&A->linv, sizeof(double) * invk * NT) != hipSuccess) {
+        (void)hipGetLastError();
+        A->linv = nullptr;
+    }
+    auto Inv = [&](int k) { return A->linv ? A->linv + invk * k : inv1; };
     const size_t big_lds = sizeof(double) * WQ_LDS;
     // tiles (and stacks) of up to 256, 512, 1024, 2048: 1, 2, 4, 8 rows per thread in k_rc_big's panels
     const int hi = std::max(NB, 2 * cap);
@@ -977,6 +991,7 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     key.ws = ctx->ws;
     key.tileops = A->d_tileops;
     key.opstat = A->d_opstat;
+    key.linv = A->linv;
     key.acc = acc;
     key.sigma2 = t.sigma2;
     key.beta = t.beta;
@@ -1013,7 +1028,7 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     hipStream_t sd = ctx->side[2];
     if (NT > 0) {
         HIPCHK(cp(0, 0, st));
-        if ((rc = launch_potrf(A, 0, Winv, Linv, dflags, o, st))) return rc;
+        if ((rc = launch_potrf(A, 0, Inv(0), dflags, o, st))) return rc;
         HIPCHK(cp(0, 1, st));
     }
     for (int k = 0; k < NT; k++) {
@@ -1021,10 +1036,10 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         int nlr = NT - k - b;
         HIPCHK(cp(k, 2, st));
         if (nbnd > 0)
-            hipLaunchKernelGGL(k_trsm_band, dim3(ntg, nbnd), dim3(BS), 0, st, t, k, (const double *)Winv,
-                               (const double *)Linv, o);
+            hipLaunchKernelGGL(k_trsm_band, dim3(ntg, nbnd), dim3(BS), 0, st, t, k, (const double *)Inv(k),
+                               o);
         if (nlr > 0)
-            launch_trsm_lr(t, k, nlr, cap, Winv, Linv, o, st);
+            launch_trsm_lr(t, k, nlr, cap, Inv(k), o, st);
         HIPCHK(cp(k, 3, st));
         HIPCHK(hipEventRecord(ctx->ev_join[2], st));
         HIPCHK(hipStreamWaitEvent(sd, ctx->ev_join[2], 0));
@@ -1037,7 +1052,7 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         HIPCHK(cp(k, 5, sd));
         if (k + 1 < NT) {
             HIPCHK(cp(k + 1, 0, sd));
-            if ((rc = launch_potrf(A, k + 1, Winv, Linv, dflags, od, sd))) return rc;
+            if ((rc = launch_potrf(A, k + 1, Inv(k + 1), dflags, od, sd))) return rc;
             HIPCHK(cp(k + 1, 1, sd));
         }
         if (nbnd >= 2)
@@ -1156,6 +1171,7 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         fprintf(stderr, "hicma_tlr: a wait of the diagonal-tile schedule ran out; the factor is not valid\n");
         return HICMA_ERR_HIP;
     }
+    A->linv_ok = A->linv != nullptr && hinfo[0] == 0;
     if (tileopcounters) {
         std::vector<unsigned long long> to((size_t)NT * NT);
         HIPCHK(hipMemcpy(to.data(), A->d_tileops, sizeof(unsigned long long) * to.size(), hipMemcpyDeviceToHost));
@@ -1240,6 +1256,19 @@ extern "C" int hicma_desc_copy(hicma_tlr_desc *dst, const hicma_tlr_desc *src)
     HIPCHK(hipMemcpyAsync(b.rank, a.rank, sizeof(int) * (size_t)a.NT * a.NT, hipMemcpyDeviceToDevice, c->stream));
     HIPCHK(hipMemcpyAsync(b.prec, a.prec, (size_t)a.NT * a.NT, hipMemcpyDeviceToDevice, c->stream));
     dst->demoted = src->demoted;
+    // the inverses go with a factor
+    dst->linv_ok = 0;
+    if (src->linv_ok) {
+        const size_t inv = sizeof(double) * a.NT * inv_tile((a.NB + PBK - 1) / PBK);
+        if (!dst->linv && ctx_malloc(c, (void **)&dst->linv, inv) != hipSuccess) {
+            (void)hipGetLastError();
+            dst->linv = nullptr;
+        }
+        if (dst->linv) {
+            HIPCHK(hipMemcpyAsync(dst->linv, src->linv, inv, hipMemcpyDeviceToDevice, c->stream));
+            dst->linv_ok = 1;
+        }
+    }
     HIPCHK(hipStreamSynchronize(c->stream));
     return 0;
 }
@@ -1413,6 +1442,7 @@ extern "C" int hicma_set_tile(hicma_tlr_desc *A, int m, int n, const double *buf
     size_t nb2 = (size_t)t.NB * t.NB;
     if (m - n < t.band_size) {
         double *dst = t.band + ((size_t)(m - n) * t.NT + m) * nb2;
+        if (m == n) A->linv_ok = 0;
         HIPCHK(hipMemcpy(dst, buf, sizeof(double) * nb2, hipMemcpyHostToDevice));
         return 0;
     }

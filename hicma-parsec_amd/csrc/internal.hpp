@@ -36,6 +36,7 @@ struct hicma_ctx {
     int *d_info;   // [0] info, [1] rank overflows, [2] unconverged Jacobi SVDs,
                    // [3] a bounded device wait ran out
     int *d_ovf;
+    int *h_stall, *d_stall;  // pinned host word (and its device address): a solve's bounded device wait ran out
     double *d_scalar;
     size_t lds_max;
     // schedule: panel steps with fewer low-rank gemm tasks than this run
@@ -58,7 +59,7 @@ struct hicma_ctx {
 // what a captured factorization graph depends on: every pointer and scalar
 // its kernels take (a replay is valid only while all are unchanged)
 struct GraphKey {
-    const void *band, *lr, *rank, *xyz, *ws, *tileops, *opstat;
+    const void *band, *lr, *rank, *xyz, *ws, *tileops, *opstat, *linv;
     double acc, sigma2, beta, nugget;
     int fixed_rank, maxrank, band_size, N, NB, NT, cap, kind, wave_min_tasks;
 };
@@ -78,6 +79,8 @@ struct hicma_tlr_desc {
     int last_unconv;
     int *rhist;                     // NT*NT x {initial, min, max, final} rank history, or null
     int rhist_on;
+    double *linv;                   // L_kk^-1 of every diagonal tile (inv_tile blocks each), or null;
+    int linv_ok;                    // the last factorization's, for the diagonal tiles held now
     int demoted;                    // off-band tiles held in FP32 or BF16 (hicma_tlr_demote)
     int use_graph;                  // capture the factorization once, replay it after
     hipGraph_t graph;
@@ -108,9 +111,10 @@ size_t hicma_work_bytes(hicma_ctx *ctx, int N, int NB, int cap, int band);
 // once per device (hicma_noalloc.hip)
 int hicma_noalloc_setup(int device);
 // the solve's launch sequence and its helpers (hicma_solve.hip)
-size_t solve_ws_doubles(const TLR &t, int nrhs);
+size_t solve_ws_doubles(const TLR &t, int nrhs, bool have_inv);
 void logdet_launch(const TLR &t, double *parts, double *out, hipStream_t s);
 int check_solve_args(hicma_ctx *ctx, hicma_tlr_desc *A, int nrhs, const double *B, long ldb);
 int solve_launch(hicma_ctx *ctx, hicma_tlr_desc *A, int dirs, int nrhs, double *B, long ldb, double *ws,
                  double *d_quad, double *d_logdet);
+int solve_stalled(hicma_ctx *ctx);
 int loglik_finish(hicma_ctx *ctx, const TLR &t, double *d_vals, double *logdet, double *quad, double *loglik);

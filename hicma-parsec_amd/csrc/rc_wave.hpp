@@ -245,40 +245,6 @@ __device__ __forceinline__ void wv_tall_mm(int NB, int kd, int nc, double alpha,
     }
 }
 
-// reduce-scatter of 4 values: lane l returns the wave total of value l >> 4
-__device__ __forceinline__ double wrs4(double p0, double p1, double p2, double p3)
-{
-    double x0 = p0, y0 = p2, x1 = p1, y1 = p3;
-    swap32d(x0, y0);  // lanes < 32: values 0, 1; lanes >= 32: values 2, 3
-    swap32d(x1, y1);
-    double a = x0 + y0, b = x1 + y1;
-    swap16d(a, b);    // value index = lane >> 4
-    return gsum<16>(a + b);
-}
-
-// reduce-scatter of 8 values: lane l returns the wave total of value l >> 3
-__device__ __forceinline__ double wrs8(double (&p)[8])
-{
-    const int lane = threadIdx.x & 63;
-    double q[4];
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        double x = p[k], y = p[k + 4];
-        swap32d(x, y);  // lanes < 32: values 0..3, lanes >= 32: values 4..7
-        q[k] = x + y;
-    }
-    double r[2];
-#pragma unroll
-    for (int k = 0; k < 2; k++) {
-        double x = q[k], y = q[k + 2];
-        swap16d(x, y);  // value bit 1 = lane bit 4
-        r[k] = x + y;
-    }
-    const bool up = (lane & 8) != 0;
-    const double keep = up ? r[1] : r[0], send = up ? r[0] : r[1];
-    return gsum<8>(keep + dppd<DPP_ROR8>(send));  // value bit 0 = lane bit 3
-}
-
 // reduce-scatter of N = 4, 8 or 16 values: lane l returns the wave total of
 // value l / (64 / N)
 template <int N>

@@ -52,6 +52,11 @@ __device__ __forceinline__ int lr_prec(const TLR &t, int m, int n) { return t.pr
 
 __device__ __forceinline__ int tdim(const TLR &t, int m) { return m == t.NT - 1 ? t.N - m * t.NB : t.NB; }
 
+// L_kk^-1 as the 64 x 64 blocks on and below its diagonal (column major, ld 64),
+// block row by block row: block (i, j), j <= i, at inv_blk(i, j) 4096
+__host__ __device__ __forceinline__ size_t inv_blk(int i, int j) { return (size_t)i * (i + 1) / 2 + j; }
+__host__ __device__ __forceinline__ size_t inv_tile(int nb) { return (size_t)4096 * nb * (nb + 1) / 2; }
+
 // covariance entry for global indices (identity on the padding)
 __device__ __forceinline__ double kval(const TLR &t, int gi, int gj)
 {

@@ -358,9 +358,8 @@ __device__ __forceinline__ void dag_done(int *flags, int task)
     if (threadIdx.x == 0) __hip_atomic_store(flags + 2 + task, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Linv: nb x nb blocks of 64 x 64 (column major, ld 64) at Linv + (i nb + j) 4096,
-// written for i > j; the diagonal blocks are Winv's
-__global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, double *Linv, int *flags, int *info,
+// Inv: the blocks of L_kk^-1 (inv_blk), W_j = block (j, j)
+__global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Inv, int *flags, int *info,
                                                  int *err, OpLog o)
 {
     extern __shared__ double sm[];
@@ -402,13 +401,13 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
             int ready = j;
             for (int l = j; l < i; l++) {
                 if (l >= ready) ready = dag_acquire(flags, l, i, dep, err);
-                const double *blk = (l == j) ? Winv + (size_t)j * PBK * PBK : Linv + ((size_t)l * nb + j) * PBK * PBK;
+                const double *blk = Inv + inv_blk(l, j) * PBK * PBK;
                 const MkOps<false, true, double, true> op{A + r0, NB, blk - (long)PBK * l, PBK};
                 mk_accum(op, ri, cj, 0, 0, (long)PBK * l, (long)PBK * l + PBK, acc, Mk);
             }
             mk_store(acc, [&](int ii, int jj, double v) { Lr[ii * PLR + jj] = v; });  // S(ii, jj)
             dag_acquire(flags, 0, 1, [&](int, int &a, int &b) { a = b = dag_fac(i, i, nb); }, err);
-            const double *Wi = Winv + (size_t)i * PBK * PBK;
+            const double *Wi = Inv + inv_blk(i, i) * PBK * PBK;
             for (int e = tid; e < PBK * PBK; e += BS) {
                 const int ii = e % PBK, l = e / PBK;  // W_i(ii, l), column major
                 Wc[ii * PLR + l] = (ii < ri && l < ri) ? mk_load<true>(Wi + ii + l * PBK) : 0.0;
@@ -416,7 +415,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
             __syncthreads();
             // Linv_ij(ii, c) = -sum_{l <= ii} W_i(ii, l) S(l, c); thread: row ii, columns cg + 4 q
             const int ii = tid % PBK, cg = tid / PBK;
-            double *Lo = Linv + ((size_t)i * nb + j) * PBK * PBK;
+            double *Lo = Inv + inv_blk(i, j) * PBK * PBK;
 #pragma unroll 4
             for (int q = 0; q < PBK / 4; q++) {
                 const int c = cg + 4 * q;
@@ -450,7 +449,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
                 } else {
                     // the whole 64 x 64 W_j, zero above the diagonal and outside
                     // cj x cj (the trsm multiplies the padding by zero rows)
-                    double *Wo = Winv + (size_t)j * PBK * PBK;
+                    double *Wo = Inv + inv_blk(j, j) * PBK * PBK;
                     for (int e = tid; e < PBK * PBK; e += BS) {
                         const int ii = e % PBK, c = e / PBK;
                         const bool in = c < cj && ii < cj && ii >= c;
@@ -464,7 +463,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
                     Lr[ii * PLR + jj] = (ii < ri && jj < cj) ? A[r0 + ii + (size_t)(c0 + jj) * NB] - v : 0.0;
                 });
                 dag_acquire(flags, 0, 1, [&](int, int &a, int &b) { a = b = dag_fac(j, j, nb); }, err);
-                const double *Wj = Winv + (size_t)j * PBK * PBK;
+                const double *Wj = Inv + inv_blk(j, j) * PBK * PBK;
                 for (int e = tid; e < PBK * PBK; e += BS) {
                     const int ii = e % PBK, c = e / PBK;  // W(ii, c), column major
                     Wc[c * PLR + ii] = (ii < cj && c < cj) ? mk_load<true>(Wj + ii + c * PBK) : 0.0;
@@ -494,7 +493,7 @@ __global__ void __launch_bounds__(BS) k_potrf_dag(TLR t, int k, double *Winv, do
 // loaded before its MFMAs.  grid (ceil(cap / TC), count).
 #define TRSM_LDS_MAX (150 * 1024)  // bytes of LDS the staged columns may take
 template <int TC>
-__global__ void __launch_bounds__(BS) k_trsm_lr_inv(TLR t, int k, const double *Winv, const double *Linv, OpLog o)
+__global__ void __launch_bounds__(BS) k_trsm_lr_inv(TLR t, int k, const double *Inv, OpLog o)
 {
     extern __shared__ double Vl[];
     const int NB = t.NB, nb = (NB + PBK - 1) / PBK, RLD = PBK * nb + 1, tid = threadIdx.x;
@@ -515,7 +514,7 @@ __global__ void __launch_bounds__(BS) k_trsm_lr_inv(TLR t, int k, const double *
     for (int b = 0; b < nb; b++) {
         mk_d4 acc = mk_d4{0.0, 0.0, 0.0, 0.0};
         for (int c = 0; c <= b; c++) {
-            const double *blk = (c == b) ? Winv + (size_t)b * PBK * PBK : Linv + ((size_t)b * nb + c) * PBK * PBK;
+            const double *blk = Inv + inv_blk(b, c) * PBK * PBK;
             const double *arow = blk + 16 * w + i16;
             double a[16];
 #pragma unroll
@@ -535,15 +534,14 @@ __global__ void __launch_bounds__(BS) k_trsm_lr_inv(TLR t, int k, const double *
 // ======================= trsm =======================
 
 // band tiles m = k+1 .. k+band-1: C <- C L^{-T} = C (L^{-1})^T on the matrix
-// cores with the block inverse of L_kk that k_potrf_dag leaves (Winv: the
-// diagonal blocks, Linv: the blocks below, 64 x 64 column major, Linv_bc at
-// Linv + (b nb + c) 4096).  One workgroup per 64-row stripe of a tile
+// cores with the block inverse of L_kk that k_potrf_dag leaves.  One workgroup
+// per 64-row stripe of a tile
 // (grid (ceil(NB/64), band-1)), in place: column block jb of the result,
 // X(:, jb) = sum_{ib <= jb} C(:, ib) Linv_{jb,ib}^T, reads column blocks
 // 0 .. jb of C only, so the blocks run from the last to the first.  For a
-// fixed jb the blocks Linv_{jb,0..jb-1} are contiguous, so the whole sum
-// over ib < jb is one operand with ld 64.
-__global__ void __launch_bounds__(BS) k_trsm_band(TLR t, int k, const double *Winv, const double *Linv, OpLog o)
+// fixed jb the blocks Linv_{jb,0..jb} are contiguous, so the whole sum is one
+// operand with ld 64.
+__global__ void __launch_bounds__(BS) k_trsm_band(TLR t, int k, const double *Inv, OpLog o)
 {
     __shared__ double sm[MK_SMEM];
     const int NB = t.NB, nb = (NB + PBK - 1) / PBK;
@@ -557,13 +555,9 @@ __global__ void __launch_bounds__(BS) k_trsm_band(TLR t, int k, const double *Wi
         const int kd = min(PBK, NB - PBK * jb);  // columns of block jb inside the tile
         mk_d4 acc[2][2];
         mk_zero(acc);
-        if (jb > 0) {
-            // B(kk, j) = L^-1(64 jb + j, kk) = Linv[(jb nb) 4096 + j + 64 kk] for kk < 64 jb
-            const MkOps<false, false> op{C, NB, Linv + (size_t)jb * nb * PBK * PBK, PBK};
-            mk_accum(op, NB, kd, r0, 0, 0, (long)PBK * jb, acc, sm);
-        }
-        const MkOps<false, false> od{C + (size_t)PBK * jb * NB, NB, Winv + (size_t)jb * PBK * PBK, PBK};
-        mk_accum(od, NB, kd, r0, 0, 0, kd, acc, sm);  // ends with a barrier: the block's reads are done
+        // B(kk, j) = L^-1(64 jb + j, kk) = row jb of blocks at [j + 64 kk]
+        const MkOps<false, false> op{C, NB, Inv + inv_blk(jb, 0) * PBK * PBK, PBK};
+        mk_accum(op, NB, kd, r0, 0, 0, (long)PBK * jb + kd, acc, sm);  // ends with a barrier: the block's reads are done
         mk_store(acc, [&](int i, int j, double v) {
             if (r0 + i < NB && j < kd) C[(r0 + i) + (size_t)(PBK * jb + j) * NB] = v;
         });

@@ -126,6 +126,40 @@ __device__ __forceinline__ double wrs16(double (&p)[16])
     return v;
 }
 
+// reduce-scatter of 4 values: lane l returns the wave total of value l >> 4
+__device__ __forceinline__ double wrs4(double p0, double p1, double p2, double p3)
+{
+    double x0 = p0, y0 = p2, x1 = p1, y1 = p3;
+    swap32d(x0, y0);  // lanes < 32: values 0, 1; lanes >= 32: values 2, 3
+    swap32d(x1, y1);
+    double a = x0 + y0, b = x1 + y1;
+    swap16d(a, b);    // value index = lane >> 4
+    return gsum<16>(a + b);
+}
+
+// reduce-scatter of 8 values: lane l returns the wave total of value l >> 3
+__device__ __forceinline__ double wrs8(double (&p)[8])
+{
+    const int lane = threadIdx.x & 63;
+    double q[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        double x = p[k], y = p[k + 4];
+        swap32d(x, y);  // lanes < 32: values 0..3, lanes >= 32: values 4..7
+        q[k] = x + y;
+    }
+    double r[2];
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+        double x = q[k], y = q[k + 2];
+        swap16d(x, y);  // value bit 1 = lane bit 4
+        r[k] = x + y;
+    }
+    const bool up = (lane & 8) != 0;
+    const double keep = up ? r[1] : r[0], send = up ? r[0] : r[1];
+    return gsum<8>(keep + dppd<DPP_ROR8>(send));  // value bit 0 = lane bit 3
+}
+
 // LDS ordering inside one wave: a code-motion barrier plus wavefront-scope
 // fences (LDS operations of one wave complete in order)
 __device__ __forceinline__ void wv_sync()
@@ -165,6 +199,21 @@ __device__ __forceinline__ wv_rsrc wv_col_rsrc(const double *p, int bytes)
 __device__ __forceinline__ double wv_ld(wv_rsrc r, int off)
 {
     return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+}
+// the same at a wave-uniform byte offset more; COH: past the L1 and the XCD's L2
+// (sc1, as an agent-scope load)
+template <bool COH = false>
+__device__ __forceinline__ double wv_lds(wv_rsrc r, int off, int soff)
+{
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(r, off, soff, COH ? 16 : 0));
+}
+__device__ __forceinline__ float wv_lds32(wv_rsrc r, int off, int soff)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, soff, 0));
+}
+__device__ __forceinline__ unsigned short wv_lds16(wv_rsrc r, int off, int soff)
+{
+    return __builtin_amdgcn_raw_buffer_load_b16(r, off, soff, 0);
 }
 __device__ __forceinline__ void wv_st(double v, wv_rsrc r, int off)
 {
