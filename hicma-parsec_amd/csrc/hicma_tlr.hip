@@ -6,7 +6,7 @@
 #include "internal.hpp"
 #include "tlr_kernels.hpp"
 #include "gen.hpp"
-#include "rc_wave.hpp"
+#include "rc_big.hpp"
 
 #include <math.h>
 #include <stdlib.h>
@@ -132,7 +132,7 @@ extern "C" int hicma_init_ex(hicma_ctx **ctx, int device, int flags, int cu_shar
     c->pool = (flags & HICMA_CTX_STREAM_ORDERED_ALLOC) != 0;
     c->lds_max = prop.sharedMemPerBlock;
     HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < 2; i++) {
         if (c->single) c->side[i] = c->stream;
         else HIPCHK(hipStreamCreateWithFlags(&c->side[i], hipStreamNonBlocking));
         HIPCHK(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
@@ -190,7 +190,7 @@ extern "C" int hicma_fini(hicma_ctx *c)
     for (auto e : c->prof_ev) (void)hipEventDestroy(e);
     for (auto e : c->cp_ev) (void)hipEventDestroy(e);
     if (c->blas && c->blas_free) c->blas_free(c->blas);
-    for (int i = 0; i < 3; i++) {
+    for (int i = 0; i < 2; i++) {
         (void)hipEventDestroy(c->ev_join[i]);
         if (!c->single) (void)hipStreamDestroy(c->side[i]);
     }
@@ -782,16 +782,14 @@ static void plan_potrf_ws(hicma_ctx *ctx, int NT, int NB, int cap, int b, PotrfW
     const size_t nbk = (size_t)((NB + PBK - 1) / PBK);
     P.dag_d = (nbk * nbk + 2 + 1) / 2 + 1;
     P.linv_d = inv_tile((int)nbk);
-    // one-wave recompression (tasks with s <= WV_S2MAX): the s <= 32 and
-    // s <= 48 variants run 4 waves per workgroup, s <= 64 two
+    // one-wave recompression (tasks with s <= WV_S2MAX), one workgroup per CU
     P.wave = P.big && (NB <= 64 * WV_KMAX);
-    P.wgrid = P.wave ? ctx->ncu : 0;  // times WvCfg<SM>::BPC resident workgroups
+    P.wgrid = P.wave ? ctx->ncu : 0;
     // CUs left to the lookahead stream (syrk(k) + potrf(k+1)) while the
     // recompression kernels of step k run
     P.wres = (P.wave && ctx->ncu > 64 && ctx->ncu == ctx->ncu_dev) ? 16 : 0;
     P.wcap = (int)maxtask;
-    // three concurrent variants, each with up to four resident waves per CU
-    P.wws_d = (size_t)3 * P.wgrid * 4 * wv_slot_doubles(NB);
+    P.wws_d = (size_t)P.wgrid * WV_WPB * wv_slot_doubles(NB);
     P.wlist_d = P.big ? ((size_t)5 * P.wcap + 16) / 2 + 1 : 0;
     // Qn = -B Av of the dense-B tasks with stacks up to QN_COLS (2-flow only)
     P.qn_d = (P.wave && b > 1) ? (size_t)(b - 1) * (NT - 1) * NB * QN_COLS : 0;
@@ -896,12 +894,11 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     TLR &t = A->t;
     const int NT = t.NT, NB = t.NB, cap = t.cap, b = band_size;
     if (A->rhist_on && !A->rhist) HIPCHK(ctx_malloc(ctx, (void **)&A->rhist, sizeof(int) * 4 * (size_t)NT * NT));
-    // one op log per executing stream: [8] context stream, [9] side 0,
-    // [10] side 1, [11] the lookahead stream
+    // one op log per executing stream: [8] context stream, [9] recompression
+    // side stream, [11] the lookahead stream
     OpLog o{A->d_tileops, A->d_opstat, A->d_opstat + 8, A->rhist_on ? A->rhist : nullptr, ctx->d_info + 2};
-    OpLog o0 = o, o1 = o, od = o;
+    OpLog o0 = o, od = o;
     o0.exec += 1;
-    o1.exec += 2;
     od.exec += 3;
 
     PotrfWs P;
@@ -947,18 +944,6 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                                (int)TRSM_LDS_MAX));
     if (big) HIPCHK(hipFuncSetAttribute((const void *)rc_big, hipFuncAttributeMaxDynamicSharedMemorySize, (int)big_lds));
     else HIPCHK(hipFuncSetAttribute((const void *)k_lr_gemm, hipFuncAttributeMaxDynamicSharedMemorySize, (int)P.rc_lds));
-    const size_t wlds32 = sizeof(double) * WvCfg<32>::LDS * WvCfg<32>::WPB;
-    const size_t wlds48 = sizeof(double) * WvCfg<48>::LDS * WvCfg<48>::WPB;
-    const size_t wlds64 = sizeof(double) * WvCfg<64>::LDS * WvCfg<64>::WPB;
-    if (wave) {
-        HIPCHK(hipFuncSetAttribute((const void *)k_rc_wave<32>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)wlds32));
-        HIPCHK(hipFuncSetAttribute((const void *)k_rc_wave<48>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)wlds48));
-        HIPCHK(hipFuncSetAttribute((const void *)k_rc_wave<64>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   (int)wlds64));
-    }
-
     // critical-path timing (hicma_parsec/HiCMA_dpotrf_L_2flow_wrapper.c:27-166):
     // potrf(k), trsm(k+1,k) and syrk(k,k+1) durations, each measured by a
     // pair of events on the stream that runs it (trsm of step k is one batched
@@ -1025,7 +1010,7 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     // Lookahead: syrk(k) and potrf(k+1) touch only diagonal tiles and the gemm
     // updates of step k only off-diagonal ones, so the former run on a side
     // stream while the latter run, and are joined back before trsm(k+1).
-    hipStream_t sd = ctx->side[2];
+    hipStream_t sd = ctx->side[1];
     if (NT > 0) {
         HIPCHK(cp(0, 0, st));
         if ((rc = launch_potrf(A, 0, Inv(0), dflags, o, st))) return rc;
@@ -1041,8 +1026,8 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         if (nlr > 0)
             launch_trsm_lr(t, k, nlr, cap, Inv(k), o, st);
         HIPCHK(cp(k, 3, st));
-        HIPCHK(hipEventRecord(ctx->ev_join[2], st));
-        HIPCHK(hipStreamWaitEvent(sd, ctx->ev_join[2], 0));
+        HIPCHK(hipEventRecord(ctx->ev_join[1], st));
+        HIPCHK(hipStreamWaitEvent(sd, ctx->ev_join[1], 0));
         HIPCHK(cp(k, 4, sd));
         if (nbnd > 0) hipLaunchKernelGGL(k_syrk_band, dim3(ntl, nbnd), dim3(BS), 0, sd, t, k, od);
         if (nlr > 0) {
@@ -1055,17 +1040,25 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
             if ((rc = launch_potrf(A, k + 1, Inv(k + 1), dflags, od, sd))) return rc;
             HIPCHK(cp(k + 1, 1, sd));
         }
-        if (nbnd >= 2)
-            hipLaunchKernelGGL(k_gemm_dense, dim3(ntg * ntg, nbnd * (nbnd - 1) / 2), dim3(BS), 0, st, t, k, o);
-        if (b > 1 && nlr > 0) {
-            int npair = nlr * (b - 1);
+        // updates of band tiles, behind the launches of the recompressions, which
+        // they do not depend on: N=16384 tile 512 band 3 61.5 -> 55.8 ms, N=2600
+        // tile 270 band 3 9.1 -> 8.8 ms
+        auto gemm_dense = [&](hipStream_t q, const OpLog &ol) {
+            if (nbnd >= 2)
+                hipLaunchKernelGGL(k_gemm_dense, dim3(ntg * ntg, nbnd * (nbnd - 1) / 2), dim3(BS), 0, q, t, k, ol);
+        };
+        auto gemm_lrd = [&]() {
+            if (b == 1 || nlr <= 0) return;
+            const int npair = nlr * (b - 1);
             hipLaunchKernelGGL(k_gemm_lrd_prep, dim3(npair), dim3(BS), 0, st, t, k, Wws, Xws, o);
-            hipLaunchKernelGGL(k_gemm_lrd_update, dim3(ntg * ntg, npair), dim3(BS), 0, st, t, k,
-                               (const double *)Wws);
-        }
+            hipLaunchKernelGGL(k_gemm_lrd_update, dim3(ntg * ntg, npair), dim3(BS), 0, st, t, k, (const double *)Wws);
+        };
         int T = NT - 1 - k;
         long long ntask = (long long)T * (T - 1) / 2;
-        if (ntask > 0 && T > b) {
+        if (!(ntask > 0 && T > b)) {
+            gemm_dense(st, o);
+            gemm_lrd();
+        } else {
             hipEvent_t e0 = nullptr, e1 = nullptr;
             if (ctx->profile) {
                 HIPCHK(hipEventCreate(&e0));
@@ -1082,39 +1075,26 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                 }
                 hipLaunchKernelGGL(k_classify_wave, dim3((unsigned)((ntask + 255) / 256)), dim3(256), 0, st, t, k,
                                    wlist, wcount, wcap, big_only, qnws ? 1 : 0);
-                // fork: k_rc_big and variant 64 on side streams 1 and 0,
-                // variants 48 and 32 on the context stream.  Launched longest
-                // tasks first: the dispatcher hands out CUs in launch order, so
-                // the long tasks start at once and the short ones fill the
-                // step's tail.
-                HIPCHK(hipEventRecord(ctx->ev_fork, st));
-                for (int i = 0; i < 2; i++) HIPCHK(hipStreamWaitEvent(ctx->side[i], ctx->ev_fork, 0));
+                // fork: k_rc_big on the context stream, so that its few long
+                // tasks are the first to get CUs, the waves on side stream 0
                 int *redo = wlist + 4 * (size_t)wcap;
                 int wg = (int)std::min<long long>(wave ? std::min(P.nbig, wgrid - wres) : P.nbig, ntask);
-                hipLaunchKernelGGL(rc_big, dim3(wg), dim3(BS), big_lds, ctx->side[1], t, k,
+                if (wave) HIPCHK(hipEventRecord(ctx->ev_fork, st));
+                hipLaunchKernelGGL(rc_big, dim3(wg), dim3(BS), big_lds, st, t, k,
                                    (const int *)(wlist + 3 * (size_t)wcap), (const int *)(wcount + 3), wcount + 7, rcws,
-                                   P.gb, acc, fixed_rank, maxrank, o1, ctx->d_ovf, (const double *)qnws);
+                                   P.gb, acc, fixed_rank, maxrank, o, ctx->d_ovf, (const double *)qnws);
                 if (wave) {
-                    const size_t wr = P.wws_d / 3;
-                    wg = (int)std::min<long long>((wgrid - wres) * WvCfg<64>::BPC, (ntask + WvCfg<64>::WPB - 1) / WvCfg<64>::WPB);
-                    hipLaunchKernelGGL(k_rc_wave<64>, dim3(wg), dim3(64 * WvCfg<64>::WPB), wlds64, ctx->side[0], t, k,
-                                       (const int *)(wlist + 2 * (size_t)wcap), (const int *)(wcount + 2), wcount + 6,
-                                       redo, wcount + 8, wws + 2 * wr, acc, fixed_rank, maxrank, o0, ctx->d_ovf,
-                                       (const double *)qnws);
-                    wg = (int)std::min<long long>((wgrid - wres) * WvCfg<48>::BPC, (ntask + WvCfg<48>::WPB - 1) / WvCfg<48>::WPB);
-                    hipLaunchKernelGGL(k_rc_wave<48>, dim3(wg), dim3(64 * WvCfg<48>::WPB), wlds48, st, t, k,
-                                       (const int *)(wlist + wcap), (const int *)(wcount + 1), wcount + 5, redo,
-                                       wcount + 8, wws + wr, acc, fixed_rank, maxrank, o, ctx->d_ovf,
-                                       (const double *)qnws);
-                    wg = (int)std::min<long long>((wgrid - wres) * WvCfg<32>::BPC, (ntask + WvCfg<32>::WPB - 1) / WvCfg<32>::WPB);
-                    hipLaunchKernelGGL(k_rc_wave<32>, dim3(wg), dim3(64 * WvCfg<32>::WPB), wlds32, st, t, k,
-                                       (const int *)wlist, (const int *)wcount, wcount + 4, redo, wcount + 8, wws, acc,
-                                       fixed_rank, maxrank, o, ctx->d_ovf, (const double *)qnws);
-                }
-                // join
-                for (int i = 0; i < 2; i++) {
-                    HIPCHK(hipEventRecord(ctx->ev_join[i], ctx->side[i]));
-                    HIPCHK(hipStreamWaitEvent(st, ctx->ev_join[i], 0));
+                    HIPCHK(hipStreamWaitEvent(ctx->side[0], ctx->ev_fork, 0));
+                    wg = (int)std::min<long long>(wgrid - wres, (ntask + WV_WPB - 1) / WV_WPB);
+                    RCHK(rc_wave_launch(ctx->side[0], wg, t, k, wlist, wcap, wcount, redo, wws, acc, fixed_rank,
+                                        maxrank, o0, ctx->d_ovf, qnws));
+                    gemm_dense(ctx->side[0], o0);
+                    HIPCHK(hipEventRecord(ctx->ev_join[0], ctx->side[0]));
+                    gemm_lrd();
+                    HIPCHK(hipStreamWaitEvent(st, ctx->ev_join[0], 0));
+                } else {
+                    gemm_dense(st, o);
+                    gemm_lrd();
                 }
                 // tasks a wave kernel could not vouch for
                 if (wave)
@@ -1123,6 +1103,8 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                                        wcount + 9, rcws, P.gb, acc, fixed_rank, maxrank, o, ctx->d_ovf,
                                        (const double *)qnws);
             } else {
+                gemm_dense(st, o);
+                gemm_lrd();
                 hipLaunchKernelGGL(k_lr_gemm, dim3((unsigned)std::min<long long>(P.ns, ntask)), dim3(BS), P.rc_lds, st, t,
                                    k, rcws, P.g, acc, fixed_rank, maxrank, o, ctx->d_ovf);
             }
@@ -1132,8 +1114,8 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                 ctx->prof_ev.push_back(e1);
             }
         }
-        HIPCHK(hipEventRecord(ctx->ev_join[2], sd));
-        HIPCHK(hipStreamWaitEvent(st, ctx->ev_join[2], 0));
+        HIPCHK(hipEventRecord(ctx->ev_join[1], sd));
+        HIPCHK(hipStreamWaitEvent(st, ctx->ev_join[1], 0));
         HIPCHK(hipGetLastError());
     }
     if (A->rhist_on)

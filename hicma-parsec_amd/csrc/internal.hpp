@@ -44,11 +44,13 @@ struct hicma_ctx {
     int wave_min_tasks;
     int profile;                     // record events around recompression launches
     std::vector<hipEvent_t> prof_ev; // pairs
-    // the recompression variants of one panel step run concurrently on side
-    // streams (default priority), forked from and joined back to `stream`
-    // (the device exposes 4 hardware queues per process: 4 streams in all)
-    hipStream_t side[3];             // [2]: syrk(k) + potrf(k+1), one step ahead
-    hipEvent_t ev_fork, ev_join[3];
+    // side streams (default priority), forked from and joined back to `stream`.
+    // A process has 4 hardware queues and the null stream may hold one: a
+    // fourth stream of the context would share a queue, and its kernels wait for
+    // the other stream's (k_rc_big behind the diagonal tile: 1.4 ms of a
+    // 4.3 ms step for N=90000 tile 900 next to a caller's null stream).
+    hipStream_t side[2];             // [0]: k_rc_wave; [1]: syrk(k) + potrf(k+1), one step ahead
+    hipEvent_t ev_fork, ev_join[2];
     // critical-path timing events (created on first request, reused)
     std::vector<hipEvent_t> cp_ev;
     // dense linear algebra handle of the checks (created on first use)
@@ -107,6 +109,9 @@ hipError_t ctx_free(hicma_ctx *c, void *p);
 // factorization of that shape allocates on a context (hicma_tlr.hip)
 size_t hicma_desc_bytes(int N, int NB, int cap, int band, int ndim);
 size_t hicma_work_bytes(hicma_ctx *ctx, int N, int NB, int cap, int band);
+// the one-wave recompressions of a step (hicma_rc_wave.hip)
+int rc_wave_launch(hipStream_t st, int grid, const TLR &t, int k, const int *wlist, int cap, int *wcount, int *redo,
+                   double *ws, double acc, int fixed_rk, int maxrank, const OpLog &o, int *ovf, const double *qn_dense);
 // device address of the allocation-free entry point's scratch array, fetched
 // once per device (hicma_noalloc.hip)
 int hicma_noalloc_setup(int device);

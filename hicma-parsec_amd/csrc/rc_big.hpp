@@ -24,16 +24,6 @@
 #include "tlr_kernels.hpp"
 #include "wglin.hpp"
 
-// Dense-B tasks (case iv: tile (n, k) in the band, (m, k) and (m, n) low
-// rank) get Qn = -B Av precomputed by k_qn_dense into a slot of QN_COLS
-// columns: slot (n - k - 1) T + (m - k - 1), T = NT - 1 - k.
-#define QN_COLS 128
-__host__ __device__ inline size_t qn_slot(int NT, int NB, int k, int m, int n)
-{
-    const int T = NT - 1 - k;
-    return ((size_t)(n - k - 1) * T + (size_t)(m - k - 1)) * NB * QN_COLS;
-}
-
 struct RbWs {
     size_t stride;  // doubles per workgroup
     int smax;       // 2 cap
@@ -153,4 +143,50 @@ k_rc_big(TLR t, int k, const int *list, const int *count, int *next, double *ws,
         }
         __syncthreads();
     }
+}
+
+// Qn = -B Av for the dense-B tasks of step k that the wave kernels take
+// (ra > 0, s <= 128); grid (64x64 tiles of an NB x 128 slot, (band - 1) T).
+__global__ void __launch_bounds__(BS) k_qn_dense(TLR t, int k, double *qn)
+{
+    __shared__ double sm[BLK_GEMM_SMEM];
+    const int NB = t.NB, NT = t.NT, b = t.band_size, T = NT - 1 - k;
+    const int m = k + 1 + (int)(blockIdx.y % T), n = k + 1 + (int)(blockIdx.y / T);
+    if (m - n < b) return;
+    const int ra = *rank_at(t, m, k), rc = *rank_at(t, m, n);
+    if (ra <= 0 || rc + ra > 128) return;
+    const int nrt = (NB + GT - 1) / GT;
+    const int ti = blockIdx.x % nrt, tj = blockIdx.x / nrt;
+    if (tj * GT >= ra) return;
+    const double *Av = lr_tile(t, m, k) + (size_t)NB * ra;
+    gemm_tile<false, false>(ti * GT, tj * GT, NB, ra, NB, -1.0, band_tile(t, n, k), NB, Av, NB, 0.0,
+                            qn + qn_slot(NT, NB, k, m, n), NB, sm);
+}
+
+// Sorts the low-rank results of step k into task lists (the order inside a
+// list is irrelevant: tasks of one step are independent): 0 (s, rb <= 32),
+// 1 (<= 48), 2 (s <= WV_S2MAX, rb <= WV_SMAX) run on one wave each; 3, every other
+// task, on one workgroup each (k_rc_big).  A dense B (band tile) needs its
+// Qn = -B Av from k_qn_dense to run on a wave.  With big_only every task goes to
+// list 3.  A low-rank update by a rank-0 factor changes nothing and is skipped.
+// wcount: [0..3] list lengths, [4..7] next-task counters, [8] length and [9]
+// next task of the redo list (list 4).
+__global__ void k_classify_wave(TLR t, int k, int *wlist, int *wcount, int cap, int big_only, int qn_dense)
+{
+    const int T = t.NT - 1 - k;
+    const long long ntask = (long long)T * (T - 1) / 2;
+    long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= ntask) return;
+    int hi, lo;
+    tri_decode(e, hi, lo);
+    const int m = k + 1 + hi, n = k + 1 + lo, b = t.band_size;
+    if (m - n < b) return;
+    const bool bdense = (n - k < b);
+    const int ra = *rank_at(t, m, k), rc = *rank_at(t, m, n), rb = bdense ? 0 : *rank_at(t, n, k);
+    const int s = rc + ra;
+    if (ra < 0 || rb < 0 || rc < 0 || (!bdense && (ra == 0 || rb == 0))) return;
+    int l = 3;
+    if (!big_only && ra > 0 && (!bdense || qn_dense))
+        l = (s <= 32 && rb <= 32) ? 0 : ((s <= 48 && rb <= 48) ? 1 : (s <= WV_S2MAX && rb <= WV_SMAX ? 2 : 3));
+    wlist[(size_t)l * cap + atomicAdd(wcount + l, 1)] = (int)e;
 }

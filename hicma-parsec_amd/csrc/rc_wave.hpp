@@ -20,30 +20,17 @@
 // Layout: lane l holds rows l, l+64, ... of every tall (NB-row) operand, so
 // tall data is read and written coalesced and row-locally.
 #pragma once
-#include "rc_big.hpp"
+#include "blk.hpp"
+#include "rc_task.hpp"
 
-#define WV_SMAX 64   // largest stack width s = rc + ra, and largest rb
-#define WV_KMAX 16   // rows per lane: NB <= 64 * WV_KMAX
-#define WV_PW 4      // Householder panel width
-#define WV_S2MAX 60  // widest stack of list 2 (k_rc_wave<64>); wider stacks go to k_rc_big
-
-
-// Per-variant sizes: SM = largest stack width of the variant (32, 48 or 64).
+// Per-class sizes: SM = largest stack width of the class (32, 48 or 64).
 template <int SM>
 struct WvCfg {
-    static constexpr int LDJ = SM + 2;             // Jacobi column stride in LDS
+    static constexpr int LDJ = SM + 2;             // column stride in LDS
     static constexpr int SIG = SM * LDJ;           // offset of the singular values
-    static constexpr int LDS = SIG + 2 * SM;       // doubles of LDS per wave
-    static constexpr int WPB = SM <= 48 ? 4 : 2;   // waves (tasks in flight) per workgroup
-    static constexpr int MINW = 1;                 // one wave per SIMD: the full register file
-    static constexpr int BPC = 4 / WPB;            // resident workgroups per CU
+    static constexpr int LDS = SIG + 2 * SM;       // doubles of LDS
 };
-
-// per-wave HBM workspace: W (QR copy), Qn, Out (2 blocks), Rp, Rq, Ku
-__host__ __device__ inline size_t wv_slot_doubles(int NB)
-{
-    return (size_t)NB * 4 * WV_SMAX + 4 * (size_t)WV_SMAX * WV_SMAX;
-}
+#define WV_LDS (WvCfg<WV_SMAX>::LDS)  // doubles per wave: those of the widest class
 
 // FP64 matrix core tile C += A B with A 16x4, B 4x16, C 16x16 (gfx950
 // V_MFMA_F64_16X16X4_F64).  Operand layout on the wave: A[i][k] on lane
@@ -278,16 +265,17 @@ struct WvRs {
 
 // One trailing pair (b0, b1) of a panel: b -= V (T^T (V^T b)), V = the
 // panel's reflectors (row block 0 in v0, the rest in a), result to W.
-__device__ __forceinline__ void wv_qr_pair(const double (&a)[WV_KMAX][WV_PW], const double (&v0)[WV_PW],
-                                           const double (&T)[WV_PW][WV_PW], double (&b0)[WV_KMAX],
-                                           double (&b1)[WV_KMAX], wv_rsrc w0, wv_rsrc w1, int lane)
+template <int KR>
+__device__ __forceinline__ void wv_qr_pair(const double (&a)[KR][WV_PW], const double (&v0)[WV_PW],
+                                           const double (&T)[WV_PW][WV_PW], double (&b0)[KR], double (&b1)[KR],
+                                           wv_rsrc w0, wv_rsrc w1, int lane)
 {
     double p[2 * WV_PW];
 #pragma unroll
     for (int c = 0; c < WV_PW; c++) {
         double a0 = v0[c] * b0[0], a1 = v0[c] * b1[0];
 #pragma unroll
-        for (int k = 1; k < WV_KMAX; k++) {
+        for (int k = 1; k < KR; k++) {
             a0 = fma(a[k][c], b0[k], a0);
             a1 = fma(a[k][c], b1[k], a1);
         }
@@ -326,7 +314,7 @@ __device__ __forceinline__ void wv_qr_pair(const double (&a)[WV_KMAX][WV_PW], co
         b1[0] = x1;
     }
 #pragma unroll
-    for (int k = 1; k < WV_KMAX; k++) {
+    for (int k = 1; k < KR; k++) {
         double x0 = b0[k], x1 = b1[k];
 #pragma unroll
         for (int c = 0; c < WV_PW; c++) {
@@ -340,14 +328,14 @@ __device__ __forceinline__ void wv_qr_pair(const double (&a)[WV_KMAX][WV_PW], co
     wv_st_col(b1, w1, lane);
 }
 
-// R factor of the NB x s stack (s <= SM <= 64, so pivot row j is on lane
-// j of the first row block).  Panels of WV_PW columns live in registers,
+// R factor of the NB x s stack (NB <= 64 KR; s <= SM <= 64, so pivot row j is on
+// lane j of the first row block).  Panels of WV_PW columns live in registers,
 // trailing columns stream through W in pairs: the pair after the current
 // one is loaded while the current one is updated (two register sets used in
 // turn, so no load is waited for before its use), and a panel's first pair
 // is loaded before the panel is factored.  R (row-major, ld WV_SMAX, zeros
 // below the diagonal) is written to Rout.
-template <int SM>
+template <int SM, int KR>
 __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const double *src1, int c0, double *W, int NB,
                                            double *Rout)
 {
@@ -356,15 +344,15 @@ __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const doub
     for (int j0 = 0; j0 < s; j0 += WV_PW) {
         const int jb = min(WV_PW, s - j0);
         const bool first = (j0 == 0);
-        double a[WV_KMAX][WV_PW];
+        double a[KR][WV_PW];
 #pragma unroll
         for (int c = 0; c < WV_PW; c++) {
             const wv_rsrc r = A.rd(j0 + c, first, c < jb);
 #pragma unroll
-            for (int k = 0; k < WV_KMAX; k++) a[k][c] = wv_ld(r, (lane + 64 * k) * 8);
+            for (int k = 0; k < KR; k++) a[k][c] = wv_ld(r, (lane + 64 * k) * 8);
         }
         const int t0 = j0 + jb;
-        double p0[WV_KMAX], p1[WV_KMAX], q0[WV_KMAX], q1[WV_KMAX];
+        double p0[KR], p1[KR], q0[KR], q1[KR];
         wv_ld_col(p0, A.rd(t0, first, t0 < s), lane);
         wv_ld_col(p1, A.rd(t0 + 1, first, t0 + 1 < s), lane);
         double T[WV_PW][WV_PW];
@@ -384,7 +372,7 @@ __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const doub
 #pragma unroll
                 for (int c = 0; c < WV_PW; c++) p[c] = y0 * (c == jj ? y0 : a[0][c]);
 #pragma unroll
-                for (int k = 1; k < WV_KMAX; k++)
+                for (int k = 1; k < KR; k++)
 #pragma unroll
                     for (int c = 0; c < WV_PW; c++) p[c] = fma(a[k][jj], a[k][c], p[c]);
                 const double red = wrsN<WV_PW>(p);
@@ -404,13 +392,13 @@ __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const doub
                 // reflector v in place of column jj: 1 at the pivot, y * scal below
                 a[0][jj] = (lane == j) ? 1.0 : y0 * scal;
 #pragma unroll
-                for (int k = 1; k < WV_KMAX; k++) a[k][jj] *= scal;
+                for (int k = 1; k < KR; k++) a[k][jj] *= scal;
 #pragma unroll
                 for (int c = 0; c < WV_PW; c++) {
                     if (c > jj) {
                         const double td = tau * (prow[c] + S[c] * scal);  // tau * v^T a_c
 #pragma unroll
-                        for (int k = 0; k < WV_KMAX; k++) a[k][c] = fma(-td, a[k][jj], a[k][c]);
+                        for (int k = 0; k < KR; k++) a[k][c] = fma(-td, a[k][jj], a[k][c]);
                     }
                 }
                 // row block 0 of column jj: beta at the pivot, R entries above it
@@ -450,52 +438,6 @@ __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const doub
             wv_qr_pair(a, v0, T, q0, q1, A.wr(t + 2, true), A.wr(t + 3, t + 3 < s), lane);
         }
     }
-}
-
-// Qn = -B Av for the dense-B tasks of step k that the wave kernels take
-// (ra > 0, s <= 128); grid (64x64 tiles of an NB x 128 slot, (band - 1) T).
-__global__ void __launch_bounds__(BS) k_qn_dense(TLR t, int k, double *qn)
-{
-    __shared__ double sm[BLK_GEMM_SMEM];
-    const int NB = t.NB, NT = t.NT, b = t.band_size, T = NT - 1 - k;
-    const int m = k + 1 + (int)(blockIdx.y % T), n = k + 1 + (int)(blockIdx.y / T);
-    if (m - n < b) return;
-    const int ra = *rank_at(t, m, k), rc = *rank_at(t, m, n);
-    if (ra <= 0 || rc + ra > 128) return;
-    const int nrt = (NB + GT - 1) / GT;
-    const int ti = blockIdx.x % nrt, tj = blockIdx.x / nrt;
-    if (tj * GT >= ra) return;
-    const double *Av = lr_tile(t, m, k) + (size_t)NB * ra;
-    gemm_tile<false, false>(ti * GT, tj * GT, NB, ra, NB, -1.0, band_tile(t, n, k), NB, Av, NB, 0.0,
-                            qn + qn_slot(NT, NB, k, m, n), NB, sm);
-}
-
-// Sorts the low-rank results of step k into task lists (the order inside a
-// list is irrelevant: tasks of one step are independent): 0 (s, rb <= 32),
-// 1 (<= 48), 2 (s <= WV_S2MAX, rb <= WV_SMAX) run on one wave each; 3, every other
-// task, on one workgroup each (k_rc_big).  A dense B (band tile) needs its
-// Qn = -B Av from k_qn_dense to run on a wave.  With big_only every task goes to
-// list 3.  A low-rank update by a rank-0 factor changes nothing and is skipped.
-// wcount: [0..3] list lengths, [4..7] next-task counters, [8] length and [9]
-// next task of the redo list (list 4).
-__global__ void k_classify_wave(TLR t, int k, int *wlist, int *wcount, int cap, int big_only, int qn_dense)
-{
-    const int T = t.NT - 1 - k;
-    const long long ntask = (long long)T * (T - 1) / 2;
-    long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= ntask) return;
-    int hi, lo;
-    tri_decode(e, hi, lo);
-    const int m = k + 1 + hi, n = k + 1 + lo, b = t.band_size;
-    if (m - n < b) return;
-    const bool bdense = (n - k < b);
-    const int ra = *rank_at(t, m, k), rc = *rank_at(t, m, n), rb = bdense ? 0 : *rank_at(t, n, k);
-    const int s = rc + ra;
-    if (ra < 0 || rb < 0 || rc < 0 || (!bdense && (ra == 0 || rb == 0))) return;
-    int l = 3;
-    if (!big_only && ra > 0 && (!bdense || qn_dense))
-        l = (s <= 32 && rb <= 32) ? 0 : ((s <= 48 && rb <= 48) ? 1 : (s <= WV_S2MAX && rb <= WV_SMAX ? 2 : 3));
-    wlist[(size_t)l * cap + atomicAdd(wcount + l, 1)] = (int)e;
 }
 
 // One-sided Jacobi on the rows of M (lane c owns row c of M in xm, zero
@@ -567,316 +509,307 @@ __device__ __forceinline__ double wv_jacobi(double (&xm)[SM], int s, double acc,
     return sqrt(f2);
 }
 
-template <int SM>
-__global__ void __launch_bounds__(64 * WvCfg<SM>::WPB, WvCfg<SM>::MINW)
-k_rc_wave(TLR t, int k, const int *wlist, const int *wcount, int *wnext, int *redo, int *nredo, double *ws, double acc,
-          int fixed_rk, int maxrank, OpLog o, int *ovf, const double *qn_dense)
+// The update of tile (m, n) = k + 1 + (hi, lo) of the packed triangle's entry e;
+// L: the wave's LDS, Wq: its workspace.
+template <int SM, int KR>
+__device__ __forceinline__ void rc_wave_task(const TLR &t, int k, int e, double *Wq, double *L, int *redo, int *nredo,
+                                             double acc, int fixed_rk, int maxrank, const OpLog &o, int *ovf,
+                                             const double *qn_dense)
 {
     using Cf = WvCfg<SM>;
-    extern __shared__ double smem[];
-    const int lane = threadIdx.x & 63;
-    const int wv = uni(threadIdx.x >> 6);
-    double *L = smem + (size_t)wv * Cf::LDS;
+    // opaque here, so that masks and offsets of one class are not kept live
+    // across the task loop (they would take the registers of all)
+    int lane = threadIdx.x & 63, NB = t.NB;
+    asm volatile("" : "+v"(lane));
+    asm volatile("" : "+s"(NB));
     double *sg = L + Cf::SIG;
-    const int NB = t.NB, NT = t.NT;
-    const int KR = (NB + 63) >> 6;
-    const int gw = blockIdx.x * Cf::WPB + wv;
-    double *Wq = ws + (size_t)gw * wv_slot_doubles(NB);
+    const int NT = t.NT;
     double *Qn = Wq + (size_t)NB * SM;
     double *Out = Qn + (size_t)NB * SM;
     double *Rp = Out + (size_t)NB * 2 * SM;
     double *Rq = Rp + SM * SM;
     double *Ku = Rq + SM * SM;
-    const int cnt = uni(*wcount);
-    // tasks are taken one at a time from a shared counter (costs differ)
-    for (;;) {
-        int idx = 0;
-        if (lane == 0) idx = atomicAdd(wnext, 1);
-        idx = uni(idx);
-        if (idx >= cnt) break;
-        const int e = uni(wlist[idx]);
-        int hi, lo;
-        tri_decode(e, hi, lo);
-        const int m = uni(k + 1 + hi), n = uni(k + 1 + lo);
-        const bool bdense = (n - k < t.band_size);
-        const int ra = uni(*rank_at(t, m, k)), rc = uni(*rank_at(t, m, n)), rb = bdense ? 0 : uni(*rank_at(t, n, k));
-        const int s = rc + ra;
-        const double *Au = lr_tile(t, m, k), *Av = Au + (size_t)NB * ra;
-        const double *Bu = bdense ? Au : lr_tile(t, n, k), *Bv = Bu + (size_t)NB * rb;
-        double *C = lr_tile(t, m, n);
-        // Q's second block: formed below, or precomputed for a dense B
-        const double *Qs = bdense ? qn_dense + qn_slot(NT, NB, k, m, n) : Qn;
+    int hi, lo;
+    tri_decode(e, hi, lo);
+    const int m = uni(k + 1 + hi), n = uni(k + 1 + lo);
+    const bool bdense = (n - k < t.band_size);
+    const int ra = uni(*rank_at(t, m, k)), rc = uni(*rank_at(t, m, n)), rb = bdense ? 0 : uni(*rank_at(t, n, k));
+    const int s = rc + ra;
+    const double *Au = lr_tile(t, m, k), *Av = Au + (size_t)NB * ra;
+    const double *Bu = bdense ? Au : lr_tile(t, n, k), *Bv = Bu + (size_t)NB * rb;
+    double *C = lr_tile(t, m, n);
+    // Q's second block: formed below, or precomputed for a dense B
+    const double *Qs = bdense ? qn_dense + qn_slot(NT, NB, k, m, n) : Qn;
 
-        // ---- X = Av^T Bv (ra x rb) on the matrix cores: 16x16 tiles of X,
-        //      k runs over the NB rows four at a time ----
-        if (!bdense) {
-            const int i16 = lane & 15, k4 = lane >> 4;
-            constexpr int TT = SM / 16, U = SM <= 32 ? 4 : (SM <= 48 ? 2 : 4);
-            wv_d4 xacc[TT][TT];
+    // ---- X = Av^T Bv (ra x rb) on the matrix cores: 16x16 tiles of X,
+    //      k runs over the NB rows four at a time ----
+    if (!bdense) {
+        const int i16 = lane & 15, k4 = lane >> 4;
+        constexpr int TT = SM / 16, U = SM <= 32 ? 4 : (SM <= 48 ? 2 : 4);
+        wv_d4 xacc[TT][TT];
 #pragma unroll
-            for (int ta = 0; ta < TT; ta++)
+        for (int ta = 0; ta < TT; ta++)
 #pragma unroll
-                for (int tb = 0; tb < TT; tb++) xacc[ta][tb] = wv_d4{0.0, 0.0, 0.0, 0.0};
-            // rows r0 .. r0 + 4U - 1 of Av's and Bv's columns by buffer loads;
-            // out-of-range lanes read 0 (no branch, no select)
-            const wv_rsrc ar = wv_col_rsrc(Av, ra * NB * 8), br = wv_col_rsrc(Bv, rb * NB * 8);
-            auto ldx = [&](double (&av)[U][TT], double (&bv)[U][TT], int r0) {
+            for (int tb = 0; tb < TT; tb++) xacc[ta][tb] = wv_d4{0.0, 0.0, 0.0, 0.0};
+        // rows r0 .. r0 + 4U - 1 of Av's and Bv's columns by buffer loads;
+        // out-of-range lanes read 0 (no branch, no select)
+        const wv_rsrc ar = wv_col_rsrc(Av, ra * NB * 8), br = wv_col_rsrc(Bv, rb * NB * 8);
+        auto ldx = [&](double (&av)[U][TT], double (&bv)[U][TT], int r0) {
 #pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const int row = r0 + 4 * u + k4;
+            for (int u = 0; u < U; u++) {
+                const int row = r0 + 4 * u + k4;
 #pragma unroll
-                    for (int tt = 0; tt < TT; tt++) {
-                        const int a = 16 * tt + i16;
-                        av[u][tt] = wv_ld(ar, (a < ra && row < NB) ? (row + a * NB) * 8 : WV_OOB);
-                        bv[u][tt] = wv_ld(br, (a < rb && row < NB) ? (row + a * NB) * 8 : WV_OOB);
-                    }
-                }
-            };
-            auto mulx = [&](const double (&av)[U][TT], const double (&bv)[U][TT]) {
-#pragma unroll
-                for (int u = 0; u < U; u++)
-#pragma unroll
-                    for (int ta = 0; ta < TT; ta++)
-                        if (16 * ta < ra) {
-#pragma unroll
-                            for (int tb = 0; tb < TT; tb++)
-                                if (16 * tb < rb) xacc[ta][tb] = mfma16(av[u][ta], bv[u][tb], xacc[ta][tb]);
-                        }
-            };
-            if constexpr (SM <= 48) {
-                // two register sets in turn: rows of the next step load
-                // while the current ones multiply
-                double av0[U][TT], bv0[U][TT], av1[U][TT], bv1[U][TT];
-                ldx(av0, bv0, 0);
-#pragma unroll 1
-                for (int r0 = 0; r0 < NB; r0 += 8 * U) {
-                    if (r0 + 4 * U < NB) ldx(av1, bv1, r0 + 4 * U);
-                    mulx(av0, bv0);
-                    if (r0 + 4 * U >= NB) break;
-                    if (r0 + 8 * U < NB) ldx(av0, bv0, r0 + 8 * U);
-                    mulx(av1, bv1);
-                }
-            } else {  // one set (the registers of the widest class are taken)
-#pragma unroll 1
-                for (int r0 = 0; r0 < NB; r0 += 4 * U) {
-                    double av[U][TT], bv[U][TT];
-                    ldx(av, bv, r0);
-                    mulx(av, bv);
+                for (int tt = 0; tt < TT; tt++) {
+                    const int a = 16 * tt + i16;
+                    av[u][tt] = wv_ld(ar, (a < ra && row < NB) ? (row + a * NB) * 8 : WV_OOB);
+                    bv[u][tt] = wv_ld(br, (a < rb && row < NB) ? (row + a * NB) * 8 : WV_OOB);
                 }
             }
-            // X^T into LDS as Xl[b * SM + a], zero outside ra x rb
-            double *Xl = L;
-            for (int q = lane; q < SM * SM; q += 64) Xl[q] = 0.0;
-            wv_sync();
+        };
+        auto mulx = [&](const double (&av)[U][TT], const double (&bv)[U][TT]) {
 #pragma unroll
-            for (int ta = 0; ta < TT; ta++)
+            for (int u = 0; u < U; u++)
 #pragma unroll
-                for (int tb = 0; tb < TT; tb++)
-                    if (16 * ta < ra && 16 * tb < rb) {
+                for (int ta = 0; ta < TT; ta++)
+                    if (16 * ta < ra) {
 #pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            const int a = 16 * ta + k4 + 4 * r, bb = 16 * tb + i16;
-                            if (a < ra && bb < rb) Xl[bb * SM + a] = xacc[ta][tb][r];
-                        }
+                        for (int tb = 0; tb < TT; tb++)
+                            if (16 * tb < rb) xacc[ta][tb] = mfma16(av[u][ta], bv[u][tb], xacc[ta][tb]);
                     }
-            wv_sync();
+        };
+        if constexpr (SM <= 48) {
+            // two register sets in turn: rows of the next step load
+            // while the current ones multiply
+            double av0[U][TT], bv0[U][TT], av1[U][TT], bv1[U][TT];
+            ldx(av0, bv0, 0);
+#pragma unroll 1
+            for (int r0 = 0; r0 < NB; r0 += 8 * U) {
+                if (r0 + 4 * U < NB) ldx(av1, bv1, r0 + 4 * U);
+                mulx(av0, bv0);
+                if (r0 + 4 * U >= NB) break;
+                if (r0 + 8 * U < NB) ldx(av0, bv0, r0 + 8 * U);
+                mulx(av1, bv1);
+            }
+        } else {  // one set (the registers of the widest class are taken)
+#pragma unroll 1
+            for (int r0 = 0; r0 < NB; r0 += 4 * U) {
+                double av[U][TT], bv[U][TT];
+                ldx(av, bv, r0);
+                mulx(av, bv);
+            }
         }
-        // ---- Qn = -Bu X^T (NB x ra): K = X^T, K[b][a] = Xl[b * SM + a] ----
-        if (!bdense) wv_tall_mm<SM>(NB, rb, ra, -1.0, WvSrc{Bu, rb, Bu, NB}, L, SM, Qn);
+        // X^T into LDS as Xl[b * SM + a], zero outside ra x rb
+        double *Xl = L;
+        for (int q = lane; q < SM * SM; q += 64) Xl[q] = 0.0;
         wv_sync();
-        // ---- R factors of P = [Cu Au] and Q = [Cv Qn] ----
-        for (int side = 0; side < 2; side++) {
-            wv_geqrf_r<SM>(s, side ? C + (size_t)NB * rc : C, side ? Qs : Au, rc, Wq, NB, side ? Rq : Rp);
+#pragma unroll
+        for (int ta = 0; ta < TT; ta++)
+#pragma unroll
+            for (int tb = 0; tb < TT; tb++)
+                if (16 * ta < ra && 16 * tb < rb) {
+#pragma unroll
+                    for (int r = 0; r < 4; r++) {
+                        const int a = 16 * ta + k4 + 4 * r, bb = 16 * tb + i16;
+                        if (a < ra && bb < rb) Xl[bb * SM + a] = xacc[ta][tb][r];
+                    }
+                }
+        wv_sync();
+    }
+    // ---- Qn = -Bu X^T (NB x ra): K = X^T, K[b][a] = Xl[b * SM + a] ----
+    if (!bdense) wv_tall_mm<SM>(NB, rb, ra, -1.0, WvSrc{Bu, rb, Bu, NB}, L, SM, Qn);
+    wv_sync();
+    // ---- R factors of P = [Cu Au] and Q = [Cv Qn] ----
+    for (int side = 0; side < 2; side++) {
+        wv_geqrf_r<SM, KR>(s, side ? C + (size_t)NB * rc : C, side ? Qs : Au, rc, Wq, NB, side ? Rq : Rp);
+    }
+    wv_sync();
+    // ---- rows of M = Rp Rq^T: lane c holds M(c, :) ----
+    double xm[SM];
+    {
+        for (int q = lane; q < s * SM; q += 64) {
+            const int l = q / SM, c = q - l * SM;
+            L[q] = (c < s) ? Rq[c * SM + l] : 0.0;  // L[l][c] = Rq(c, l)
         }
         wv_sync();
-        // ---- rows of M = Rp Rq^T: lane c holds M(c, :) ----
-        double xm[SM];
+#pragma unroll
+        for (int q = 0; q < SM; q++) xm[q] = 0.0;
+        // this lane's row of Rp, 16 entries per batch of loads
+        const wv_rsrc rpr = wv_col_rsrc(Rp, SM * SM * 8);
+        for (int l0 = 0; l0 < s; l0 += 16) {
+            double rv[16];
+#pragma unroll
+            for (int u = 0; u < 16; u++) {
+                const int l = l0 + u;
+                rv[u] = wv_ld(rpr, (lane < s && l < s && l >= lane) ? (lane * SM + l) * 8 : WV_OOB);
+            }
+#pragma unroll
+            for (int u = 0; u < 16; u++)
+                if (l0 + u < s) {
+                    const double *rq = L + (l0 + u) * SM;
+#pragma unroll
+                    for (int q8 = 0; q8 < SM; q8 += 8)
+                        if (q8 < s) {
+#pragma unroll
+                            for (int q = q8; q < q8 + 8; q++) xm[q] = fma(rv[u], rq[q], xm[q]);
+                        }
+                }
+        }
+        wv_sync();
+    }
+    // ---- one-sided Jacobi on the columns of M^T (lane c owns column c):
+    //      loops run over SM - 8 entries when s fits in them (entries
+    //      beyond s are zero, so the width changes no bit) ----
+    double fro;
+    if constexpr (SM <= 48) {
+        constexpr int WJ = SM - 8;
+        fro = (s <= WJ) ? wv_jacobi<SM, WJ>(xm, s, acc, fixed_rk, o.unconv)
+                        : wv_jacobi<SM, SM>(xm, s, acc, fixed_rk, o.unconv);
+    } else {  // one width: a second copy costs the widest class registers
+        fro = wv_jacobi<SM, SM>(xm, s, acc, fixed_rk, o.unconv);
+    }
+    // ---- singular values, order, rank ----
+    double sig = 0.0;
+#pragma unroll
+    for (int q = 0; q < SM; q++) sig = fma(xm[q], xm[q], sig);
+    sig = sqrt(sig);
+    if (lane < s) sg[lane] = sig;
+    wv_sync();
+    int pos = 0;
+    for (int q = 0; q < s; q++) {
+        const double o2 = sg[q];
+        pos += (o2 > sig) || (o2 == sig && q < lane);
+    }
+    int nr;
+    if (fixed_rk > 0) nr = fixed_rk < s ? fixed_rk : s;
+    else nr = __popcll(__ballot(lane < s && sig >= acc));
+    if (nr > maxrank) {
+        if (lane == 0) atomicAdd(ovf, 1);
+        nr = maxrank;
+    }
+    nr = uni(nr);
+    wv_sync();
+    if (nr > 0) {
+        // Vs_r into LDS, row-major: Vl[l * SM + pos]; sigma by position
+        double *Vl = L;
+        double *sgp = sg + SM;
+        if (lane < s && pos < nr) {
+            const double inv = sig > 0.0 ? 1.0 / sig : 0.0;
+#pragma unroll
+            for (int q = 0; q < SM; q++)
+                if (q < s) Vl[q * SM + pos] = xm[q] * inv;
+            sgp[pos] = sig;
+        }
+        wv_sync();
+        // Ku = Rq^T Vs_r: lane c computes row c -> Ku[c * SM + j]
         {
-            for (int q = lane; q < s * SM; q += 64) {
-                const int l = q / SM, c = q - l * SM;
-                L[q] = (c < s) ? Rq[c * SM + l] : 0.0;  // L[l][c] = Rq(c, l)
-            }
-            wv_sync();
+            double ac[SM];
 #pragma unroll
-            for (int q = 0; q < SM; q++) xm[q] = 0.0;
-            // this lane's row of Rp, 16 entries per batch of loads
-            const wv_rsrc rpr = wv_col_rsrc(Rp, SM * SM * 8);
+            for (int j = 0; j < SM; j++) ac[j] = 0.0;
+            // column `lane` of Rq, 16 entries per batch of loads
+            const wv_rsrc rqr = wv_col_rsrc(Rq, SM * SM * 8);
             for (int l0 = 0; l0 < s; l0 += 16) {
                 double rv[16];
 #pragma unroll
                 for (int u = 0; u < 16; u++) {
                     const int l = l0 + u;
-                    rv[u] = wv_ld(rpr, (lane < s && l < s && l >= lane) ? (lane * SM + l) * 8 : WV_OOB);
+                    rv[u] = wv_ld(rqr, (lane < s && l < s && l <= lane) ? (l * SM + lane) * 8 : WV_OOB);
                 }
 #pragma unroll
                 for (int u = 0; u < 16; u++)
                     if (l0 + u < s) {
-                        const double *rq = L + (l0 + u) * SM;
+                        const double *vr = Vl + (l0 + u) * SM;
 #pragma unroll
-                        for (int q8 = 0; q8 < SM; q8 += 8)
-                            if (q8 < s) {
+                        for (int j8 = 0; j8 < SM; j8 += 8)
+                            if (j8 < nr) {
 #pragma unroll
-                                for (int q = q8; q < q8 + 8; q++) xm[q] = fma(rv[u], rq[q], xm[q]);
+                                for (int j = j8; j < j8 + 8; j++) ac[j] = fma(rv[u], vr[j], ac[j]);
                             }
                     }
             }
-            wv_sync();
-        }
-        // ---- one-sided Jacobi on the columns of M^T (lane c owns column c):
-        //      loops run over SM - 8 entries when s fits in them (entries
-        //      beyond s are zero, so the width changes no bit) ----
-        double fro;
-        if constexpr (SM <= 48) {
-            constexpr int WJ = SM - 8;
-            fro = (s <= WJ) ? wv_jacobi<SM, WJ>(xm, s, acc, fixed_rk, o.unconv)
-                            : wv_jacobi<SM, SM>(xm, s, acc, fixed_rk, o.unconv);
-        } else {  // one width: a second copy costs the widest class registers
-            fro = wv_jacobi<SM, SM>(xm, s, acc, fixed_rk, o.unconv);
-        }
-        // ---- singular values, order, rank ----
-        double sig = 0.0;
+            if (lane < s) {
 #pragma unroll
-        for (int q = 0; q < SM; q++) sig = fma(xm[q], xm[q], sig);
-        sig = sqrt(sig);
-        if (lane < s) sg[lane] = sig;
-        wv_sync();
-        int pos = 0;
-        for (int q = 0; q < s; q++) {
-            const double o2 = sg[q];
-            pos += (o2 > sig) || (o2 == sig && q < lane);
-        }
-        int nr;
-        if (fixed_rk > 0) nr = fixed_rk < s ? fixed_rk : s;
-        else nr = __popcll(__ballot(lane < s && sig >= acc));
-        if (nr > maxrank) {
-            if (lane == 0) atomicAdd(ovf, 1);
-            nr = maxrank;
-        }
-        nr = uni(nr);
-        wv_sync();
-        if (nr > 0) {
-            // Vs_r into LDS, row-major: Vl[l * SM + pos]; sigma by position
-            double *Vl = L;
-            double *sgp = sg + SM;
-            if (lane < s && pos < nr) {
-                const double inv = sig > 0.0 ? 1.0 / sig : 0.0;
-#pragma unroll
-                for (int q = 0; q < SM; q++)
-                    if (q < s) Vl[q * SM + pos] = xm[q] * inv;
-                sgp[pos] = sig;
+                for (int j = 0; j < SM; j++)
+                    if (j < nr) Ku[lane * SM + j] = ac[j];
             }
-            wv_sync();
-            // Ku = Rq^T Vs_r: lane c computes row c -> Ku[c * SM + j]
-            {
-                double ac[SM];
-#pragma unroll
-                for (int j = 0; j < SM; j++) ac[j] = 0.0;
-                // column `lane` of Rq, 16 entries per batch of loads
-                const wv_rsrc rqr = wv_col_rsrc(Rq, SM * SM * 8);
-                for (int l0 = 0; l0 < s; l0 += 16) {
-                    double rv[16];
-#pragma unroll
-                    for (int u = 0; u < 16; u++) {
-                        const int l = l0 + u;
-                        rv[u] = wv_ld(rqr, (lane < s && l < s && l <= lane) ? (l * SM + lane) * 8 : WV_OOB);
-                    }
-#pragma unroll
-                    for (int u = 0; u < 16; u++)
-                        if (l0 + u < s) {
-                            const double *vr = Vl + (l0 + u) * SM;
-#pragma unroll
-                            for (int j8 = 0; j8 < SM; j8 += 8)
-                                if (j8 < nr) {
-#pragma unroll
-                                    for (int j = j8; j < j8 + 8; j++) ac[j] = fma(rv[u], vr[j], ac[j]);
-                                }
-                        }
-                }
-                if (lane < s) {
-#pragma unroll
-                    for (int j = 0; j < SM; j++)
-                        if (j < nr) Ku[lane * SM + j] = ac[j];
-                }
-            }
-            wv_sync();
-            // Kv = Rq^-1 Vs_r in place (lane j solves column j) by plain back
-            // substitution.  Q Kv = Qq Vs_r for any Kv with Rq Kv = Vs_r, and
-            // the substitution is backward stable, so the tiny pivots of a
-            // numerically rank-deficient Q are divided by, not dropped (dropping
-            // one breaks the solve when its row carries other entries).  Column
-            // j then errs in the tile by at most
-            // sigma_j s eps max_q sum_l |Rq(q,l)| |Kv(l,j)|; a task over the
-            // tolerance, or with an exactly zero pivot, is left untouched and
-            // handed to the Householder path (k_rc_big).
-            // Row q of Rq is loaded across the lanes (lane l: Rq(q, l), one
-            // load per row, the next row's issued ahead) and read by readlane.
-            bool bad = false;
-            {
-                const wv_rsrc rqr = wv_col_rsrc(Rq, SM * SM * 8);
-                double gmax = 0.0;
-                double rnext = wv_ld(rqr, (lane < s) ? ((s - 1) * SM + lane) * 8 : WV_OOB);
-                for (int q = s - 1; q >= 0; q--) {
-                    const double rrow = rnext;
-                    rnext = wv_ld(rqr, (q > 0 && lane < s) ? ((q - 1) * SM + lane) * 8 : WV_OOB);
-                    double v = Vl[q * SM + lane], gq = 0.0;
-                    for (int l = q + 1; l < s; l++) {
-                        const double rql = rdlane(rrow, l), xl = Vl[l * SM + lane];
-                        v = fma(-rql, xl, v);
-                        gq = fma(fabs(rql), fabs(xl), gq);
-                    }
-                    const double d = rdlane(rrow, q);
-                    const bool ok = fabs(d) > 1e-300;
-                    const double x = ok ? v / d : 0.0;
-                    bad = bad || !ok;
-                    gmax = fmax(gmax, fma(fabs(d), fabs(x), gq));
-                    if (lane < nr) Vl[q * SM + lane] = x;
-                }
-                bad = lane < nr && (bad || !(sgp[lane] * s * 2.3e-16 * gmax <= rc_solve_tol(acc, fixed_rk, fro)));
-            }
-            if (__ballot(bad) != 0) {
-                if (lane == 0) redo[atomicAdd(nredo, 1)] = e;
-                wv_sync();
-                continue;
-            }
-            wv_sync();
-            // ---- outputs, written in place into the tile.  A product reads a
-            //      batch of rows of all its sources before writing those rows,
-            //      and every column of the tile has stride NB, so an output
-            //      may overwrite its own sources.  The two products are
-            //      ordered so that neither overwrites the other's sources:
-            //      U' = P Ku (columns 0 .. nr-1, sources Cu = columns
-            //      0 .. rc-1) and V' = Q Kv (columns nr .. 2nr-1, sources
-            //      Cv = columns rc .. 2rc-1): U' first when nr <= rc, V'
-            //      first otherwise. ----
-            auto v_out = [&]() {  // Kv in LDS
-                wv_tall_mm<SM>(NB, s, nr, 1.0, WvSrc{C + (size_t)rc * NB, rc, Qs, NB}, Vl, SM, C + (size_t)nr * NB);
-                wv_sync();
-            };
-            auto u_out = [&]() {  // stages Ku into LDS
-                for (int q = lane; q < s * SM; q += 64) {
-                    const int c = q / SM, j = q - c * SM;
-                    Vl[q] = (j < nr) ? Ku[c * SM + j] : 0.0;
-                }
-                wv_sync();
-                wv_tall_mm<SM>(NB, s, nr, 1.0, WvSrc{C, rc, Au, NB}, Vl, SM, C);
-                wv_sync();
-            };
-            if (nr > rc) {
-                v_out();
-                u_out();
-            } else {
-                for (int q = lane; q < s * SM; q += 64) Out[q] = Vl[q];  // Kv aside while Ku uses the LDS
-                u_out();
-                for (int q = lane; q < s * SM; q += 64) Vl[q] = Out[q];
-                wv_sync();
-                v_out();
-            }
-        }
-        if (lane == 0) {
-            *rank_at(t, m, n) = nr;
-            rank_hist(o, NT, m, n, nr);
-            rc_oplog(o, t, m, n, ra, rb, rc, nr, bdense);
         }
         wv_sync();
+        // Kv = Rq^-1 Vs_r in place (lane j solves column j) by plain back
+        // substitution.  Q Kv = Qq Vs_r for any Kv with Rq Kv = Vs_r, and
+        // the substitution is backward stable, so the tiny pivots of a
+        // numerically rank-deficient Q are divided by, not dropped (dropping
+        // one breaks the solve when its row carries other entries).  Column
+        // j then errs in the tile by at most
+        // sigma_j s eps max_q sum_l |Rq(q,l)| |Kv(l,j)|; a task over the
+        // tolerance, or with an exactly zero pivot, is left untouched and
+        // handed to the Householder path (k_rc_big).
+        // Row q of Rq is loaded across the lanes (lane l: Rq(q, l), one
+        // load per row, the next row's issued ahead) and read by readlane.
+        bool bad = false;
+        {
+            const wv_rsrc rqr = wv_col_rsrc(Rq, SM * SM * 8);
+            double gmax = 0.0;
+            double rnext = wv_ld(rqr, (lane < s) ? ((s - 1) * SM + lane) * 8 : WV_OOB);
+            for (int q = s - 1; q >= 0; q--) {
+                const double rrow = rnext;
+                rnext = wv_ld(rqr, (q > 0 && lane < s) ? ((q - 1) * SM + lane) * 8 : WV_OOB);
+                double v = Vl[q * SM + lane], gq = 0.0;
+                for (int l = q + 1; l < s; l++) {
+                    const double rql = rdlane(rrow, l), xl = Vl[l * SM + lane];
+                    v = fma(-rql, xl, v);
+                    gq = fma(fabs(rql), fabs(xl), gq);
+                }
+                const double d = rdlane(rrow, q);
+                const bool ok = fabs(d) > 1e-300;
+                const double x = ok ? v / d : 0.0;
+                bad = bad || !ok;
+                gmax = fmax(gmax, fma(fabs(d), fabs(x), gq));
+                if (lane < nr) Vl[q * SM + lane] = x;
+            }
+            bad = lane < nr && (bad || !(sgp[lane] * s * 2.3e-16 * gmax <= rc_solve_tol(acc, fixed_rk, fro)));
+        }
+        if (__ballot(bad) != 0) {
+            if (lane == 0) redo[atomicAdd(nredo, 1)] = e;
+            wv_sync();
+            return;
+        }
+        wv_sync();
+        // ---- outputs, written in place into the tile.  A product reads a
+        //      batch of rows of all its sources before writing those rows,
+        //      and every column of the tile has stride NB, so an output
+        //      may overwrite its own sources.  The two products are
+        //      ordered so that neither overwrites the other's sources:
+        //      U' = P Ku (columns 0 .. nr-1, sources Cu = columns
+        //      0 .. rc-1) and V' = Q Kv (columns nr .. 2nr-1, sources
+        //      Cv = columns rc .. 2rc-1): U' first when nr <= rc, V'
+        //      first otherwise. ----
+        auto v_out = [&]() {  // Kv in LDS
+            wv_tall_mm<SM>(NB, s, nr, 1.0, WvSrc{C + (size_t)rc * NB, rc, Qs, NB}, Vl, SM, C + (size_t)nr * NB);
+            wv_sync();
+        };
+        auto u_out = [&]() {  // stages Ku into LDS
+            for (int q = lane; q < s * SM; q += 64) {
+                const int c = q / SM, j = q - c * SM;
+                Vl[q] = (j < nr) ? Ku[c * SM + j] : 0.0;
+            }
+            wv_sync();
+            wv_tall_mm<SM>(NB, s, nr, 1.0, WvSrc{C, rc, Au, NB}, Vl, SM, C);
+            wv_sync();
+        };
+        if (nr > rc) {
+            v_out();
+            u_out();
+        } else {
+            for (int q = lane; q < s * SM; q += 64) Out[q] = Vl[q];  // Kv aside while Ku uses the LDS
+            u_out();
+            for (int q = lane; q < s * SM; q += 64) Vl[q] = Out[q];
+            wv_sync();
+            v_out();
+        }
     }
+    if (lane == 0) {
+        *rank_at(t, m, n) = nr;
+        rank_hist(o, NT, m, n, nr);
+        rc_oplog(o, t, m, n, ra, rb, rc, nr, bdense);
+    }
+    wv_sync();
 }

@@ -188,7 +188,7 @@ int hicma_rank_overflows(const hicma_tlr_desc *A);
 int hicma_jacobi_unconverged(const hicma_tlr_desc *A);
 /* op counts of the last call per executing stream (the reference's
  * per-thread opcounters, hicma_parsec/testing_dpotrf.c:920-990): ops[0..3] =
- * context stream, two recompression side streams, lookahead stream; entries
+ * context stream, recompression side stream, 0, lookahead stream; entries
  * n > 4 are 0.  They sum to the total. */
 int hicma_exec_op_stats(const hicma_tlr_desc *A, unsigned long *ops, int n);
 /* record the initial / minimum / maximum / final rank of every off-band tile
@@ -285,11 +285,10 @@ int hicma_tlr_demote(hicma_tlr_desc *A, double thr32, double thr16, int *counts)
 
 /* hicma_tlr_loglik without any device allocation.  No counterpart in the
  * reference: for callers that cannot allocate (code under HIP graph capture,
- * serving loops).  Its workspace is an 88 MiB device array of the library
- * (8 Mi doubles: the lower 64 x 64 blocks of every L_kk^-1,
+ * serving loops).  Its workspace is an 88 MiB device array of the library.
+ * Problems above 8 Mi doubles (the lower 64 x 64 blocks of every L_kk^-1,
  * NT*4096*nb*(nb+1)/2 doubles with nb = (NB+63)/64, plus 2*NT*NB,
- * max(NT*NB/256 + 1, NT) and 8);
- * larger problems return HICMA_ERR_ARG.  Calls that
+ * max(NT*NB/256 + 1, NT) and 8) return HICMA_ERR_ARG.  Calls that
  * overlap on one GPU race on that array. */
 int hicma_tlr_loglik_noalloc(hicma_ctx *ctx, hicma_tlr_desc *A, double *z, double *logdet, double *quad,
                              double *loglik);
