@@ -4,13 +4,13 @@
 // reference's hcore_dgemm QR + SVD recompression, hicma_parsec_core.c).  The
 // wave owns its task from start to end: every reduction over the NB tile rows
 // is a wave reduction (permlane / DPP / readlane), LDS is private to the wave
-// and no barrier is shared with other waves, so a CU works on eight tasks at
+// and no barrier is shared with other waves, so a CU works on four tasks at
 // once and a step with thousands of tasks fills all CUs.
 //
 // Mathematics (the reference's up to rounding):
 //   X = Av^T Bv,  Qn = -Bu X^T,  P = [Cu Au],  Q = [Cv Qn]        (NB x s)
 //   Rp, Rq = R factors of P, Q (Householder, panels of WV_PW columns)
-//   M = Rp Rq^T (s x s);  one-sided Jacobi on the rows of M:  M^T J = Vs S
+//   M = Rp Rq^T (s x s) = Q1 R;  one-sided Jacobi on the rows of R:  R^T J = Vs S
 //   -> right singular vectors Vs and singular values S of M;
 //   r' = #{S >= acc} (or the fixed rank), capped at maxrank;
 //   U' = P (Rq^T Vs_r)   ( = Qp Us_r S_r because P = Qp Rp, M Vs = Us S )
@@ -19,6 +19,13 @@
 //
 // Layout: lane l holds rows l, l+64, ... of every tall (NB-row) operand, so
 // tall data is read and written coalesced and row-locally.
+//
+// What bounds it: FP64 VALU issue of one wave per SIMD and, in the Jacobi, the
+// LDS crossbar (s doubles per lane and round); the two tall QR are 37 % of a
+// task at NB = 900.  The rows of the unpivoted R are graded, which takes about half the
+// sweeps that the rows of M took, and a sweep pairs only rows above the
+// truncation floor: per panel step of N=90000 tile 900 (thousands of tasks)
+// 3.3 -> 2.7 ms, of N=8100 tile 465 (tens) 1.45 -> 1.02 ms.
 #pragma once
 #include "blk.hpp"
 #include "rc_task.hpp"
@@ -440,33 +447,86 @@ __device__ __forceinline__ void wv_geqrf_r(int s, const double *src0, const doub
     }
 }
 
-// One-sided Jacobi on the rows of M (lane c owns row c of M in xm, zero
-// beyond s), round-robin pairs; a lane reads its partner's row with
-// ds_bpermute (no LDS storage, no wave barrier).  Loops cover the first W
-// entries (W >= s).  Returns ||M||_F; counts a run out of sweeps in *unconv.
+// Lane q holds column q of the s x s matrix M in x (zero beyond s): R of the
+// Householder QR of M in place (rows i <= q; below is rounding noise).  Column j
+// reaches the other lanes by readlane, every lane forms its own column's product
+// with the reflector: no cross-lane sum.
+template <int SM>
+__device__ __forceinline__ void wv_qr_cols(double (&x)[SM], int s)
+{
+#pragma unroll
+    for (int c = 0; c < SM; c += 8) {
+        const int je = min(8, s - 1 - c);  // the last column needs no reflector
+#pragma unroll 1
+        for (int jj = 0; jj < je; jj++) {
+            const int j = c + jj;
+            double d4[4] = {0.0, 0.0, 0.0, 0.0}, xj = 0.0;
+#pragma unroll
+            for (int u = 0; u < 8; u++) {
+                const double v = rdlane(x[c + u], j);
+                d4[u & 3] = fma(u >= jj ? v : 0.0, x[c + u], d4[u & 3]);
+                xj = u == jj ? x[c + u] : xj;
+            }
+#pragma unroll
+            for (int i8 = c + 8; i8 < SM; i8 += 8)
+                if (i8 < s) {
+#pragma unroll
+                    for (int i = i8; i < i8 + 8; i++) d4[i & 3] = fma(rdlane(x[i], j), x[i], d4[i & 3]);
+                    __builtin_amdgcn_sched_barrier(0);  // 8 values in scalar registers at a time
+                }
+            const double d = (d4[0] + d4[1]) + (d4[2] + d4[3]);
+            const double alpha = rdlane(xj, j), nrm2 = rdlane(d, j);
+            if (nrm2 > 1e-290) {
+                // w = x_j with alpha - beta at row j;  H = I - w w^T / (nrm2 - alpha beta)
+                const double beta = -copysign(sqrt(nrm2), alpha);
+                const double g = (d - beta * xj) / (nrm2 - alpha * beta);
+#pragma unroll
+                for (int u = 0; u < 8; u++) {
+                    const double v = rdlane(x[c + u], j);
+                    x[c + u] = fma(u > jj ? -v : (u == jj ? beta - alpha : 0.0), g, x[c + u]);
+                }
+#pragma unroll
+                for (int i8 = c + 8; i8 < SM; i8 += 8)
+                    if (i8 < s) {
+#pragma unroll
+                        for (int i = i8; i < i8 + 8; i++) x[i] = fma(-rdlane(x[i], j), g, x[i]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+            }
+        }
+    }
+}
+
+// One-sided Jacobi on the rows of R (lane r owns row r in xm, zero beyond s),
+// round-robin pairs; a lane reads its partner's row with ds_bpermute (no LDS
+// storage, no wave barrier).  Loops cover the first W entries (W >= s); f2 =
+// ||R||_F^2.  Counts a run out of sweeps in *unconv.
 template <int SM, int W>
-__device__ __forceinline__ double wv_jacobi(double (&xm)[SM], int s, double acc, int fixed_rk, int *unconv)
+__device__ __forceinline__ void wv_jacobi(double (&xm)[SM], int s, double f2, double acc, int fixed_rk, int *unconv)
 {
     const int lane = threadIdx.x & 63;
-    const int npad = s + (s & 1);
     const double tol = 4.0e-16 * sqrt((double)s);
-    double al = 0.0;
-#pragma unroll
-    for (int q = 0; q < W; q++) al = fma(xm[q], xm[q], al);
-    // A pair is left alone when its smaller column is below the
+    // A pair is left alone when its smaller row is below the
     // rounding-noise floor (2.3e-16 s)^2 ||M||_F^2, or, when truncating
-    // at acc, below (1e-3 acc)^2: such columns stay below the
+    // at acc, below (1e-3 acc)^2: such rows stay below the
     // truncation threshold (all of them together hold less than
-    // 0.012 acc of energy) and rotating them moves a kept column by
-    // less than one rounding of its norm.
-    const double f2 = wsum(lane < s ? al : 0.0);
+    // 0.012 acc of energy) and rotating them moves a kept row by
+    // less than one rounding of its norm.  A sweep pairs only the rows
+    // above the floor (the others never change again).
     const double nz = wv_skip_floor(f2, s, acc, fixed_rk);
-    // position of column `lane` in round 0 of the round-robin schedule
-    const int p0 = (lane == 0) ? 0 : lane;
     int sweep = 0;
     for (; sweep < BLK_JACOBI_SWEEPS; sweep++) {
+        double al = 0.0;  // exact norms once per sweep
+#pragma unroll
+        for (int q = 0; q < W; q++) al = fma(xm[q], xm[q], al);
+        const bool act = lane < s && !(al <= nz);
+        const unsigned long long am = __ballot(act);
+        const int na = __popcll(am), npad = na + (na & 1);
+        const int idx = __builtin_amdgcn_mbcnt_hi((unsigned)(am >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)am, 0));
+        // row of the i-th active one, on lane i
+        const int row = __builtin_amdgcn_ds_permute(4 * (act ? idx : na + lane - idx), lane);
         int rot_any = 0;
-        int pos = p0;  // column at position p in round r: ((p - 1 + r) mod (npad - 1)) + 1
+        int pos = idx;  // row at position p in round r: ((p - 1 + r) mod (npad - 1)) + 1
         for (int r = 0; r < npad - 1; r++) {
             const int pp = npad - 1 - pos;
             int pc = 0;
@@ -474,17 +534,17 @@ __device__ __forceinline__ double wv_jacobi(double (&xm)[SM], int s, double acc,
                 pc = pp + r;
                 if (pc > npad - 1) pc -= npad - 1;
             }
-            const int src = 4 * pc;  // pc < npad <= 64
+            const int src = 4 * __builtin_amdgcn_ds_bpermute(4 * pc, row);
             double yv[W];
 #pragma unroll
             for (int q = 0; q < W; q++) yv[q] = wv_bperm(src, xm[q]);
             const double be = wv_bperm(src, al);
-            if (lane < s && pc < s) {
+            if (act && pc < na) {
                 double g4[4] = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
                 for (int q = 0; q < W; q++) g4[q & 3] = fma(xm[q], yv[q], g4[q & 3]);
                 const double ga = (g4[0] + g4[1]) + (g4[2] + g4[3]);
-                const bool lo_ = lane < pc;
+                const bool lo_ = idx < pc;
                 double cs, sn;
                 if (fmin(al, be) > nz && jacobi_rot(lo_ ? al : be, lo_ ? be : al, ga, tol, cs, sn)) {
                     rot_any = 1;
@@ -496,17 +556,12 @@ __device__ __forceinline__ double wv_jacobi(double (&xm)[SM], int s, double acc,
                              : (sn * sn * be + 2.0 * cs * sn * ga + cs * cs * al);
                 }
             }
-            // next round: every column but 0 moves one position down
-            if (lane > 0) pos = (pos == 1) ? npad - 1 : pos - 1;
+            // next round: every row but the first moves one position down
+            if (idx > 0) pos = (pos == 1) ? npad - 1 : pos - 1;
         }
-        // exact norms once per sweep
-        al = 0.0;
-#pragma unroll
-        for (int q = 0; q < W; q++) al = fma(xm[q], xm[q], al);
         if (__ballot(rot_any) == 0) break;
     }
     if (sweep >= BLK_JACOBI_SWEEPS && lane == 0) atomicAdd(unconv, 1);
-    return sqrt(f2);
 }
 
 // The update of tile (m, n) = k + 1 + (hi, lo) of the packed triangle's entry e;
@@ -623,49 +678,61 @@ __device__ __forceinline__ void rc_wave_task(const TLR &t, int k, int e, double 
         wv_geqrf_r<SM, KR>(s, side ? C + (size_t)NB * rc : C, side ? Qs : Au, rc, Wq, NB, side ? Rq : Rp);
     }
     wv_sync();
-    // ---- rows of M = Rp Rq^T: lane c holds M(c, :) ----
+    // ---- columns of M = Rp Rq^T: lane q holds M(:, q) ----
     double xm[SM];
     {
         for (int q = lane; q < s * SM; q += 64) {
             const int l = q / SM, c = q - l * SM;
-            L[q] = (c < s) ? Rq[c * SM + l] : 0.0;  // L[l][c] = Rq(c, l)
+            L[q] = (c < s) ? Rp[c * SM + l] : 0.0;  // L[l][c] = Rp(c, l)
         }
         wv_sync();
 #pragma unroll
         for (int q = 0; q < SM; q++) xm[q] = 0.0;
-        // this lane's row of Rp, 16 entries per batch of loads
-        const wv_rsrc rpr = wv_col_rsrc(Rp, SM * SM * 8);
+        // this lane's row of Rq, 16 entries per batch of loads
+        const wv_rsrc rqr = wv_col_rsrc(Rq, SM * SM * 8);
         for (int l0 = 0; l0 < s; l0 += 16) {
             double rv[16];
 #pragma unroll
             for (int u = 0; u < 16; u++) {
                 const int l = l0 + u;
-                rv[u] = wv_ld(rpr, (lane < s && l < s && l >= lane) ? (lane * SM + l) * 8 : WV_OOB);
+                rv[u] = wv_ld(rqr, (lane < s && l < s && l >= lane) ? (lane * SM + l) * 8 : WV_OOB);
             }
 #pragma unroll
             for (int u = 0; u < 16; u++)
                 if (l0 + u < s) {
-                    const double *rq = L + (l0 + u) * SM;
+                    const double *rp = L + (l0 + u) * SM;
 #pragma unroll
                     for (int q8 = 0; q8 < SM; q8 += 8)
                         if (q8 < s) {
 #pragma unroll
-                            for (int q = q8; q < q8 + 8; q++) xm[q] = fma(rv[u], rq[q], xm[q]);
+                            for (int q = q8; q < q8 + 8; q++) xm[q] = fma(rv[u], rp[q], xm[q]);
                         }
                 }
         }
         wv_sync();
     }
-    // ---- one-sided Jacobi on the columns of M^T (lane c owns column c):
-    //      loops run over SM - 8 entries when s fits in them (entries
+    // ---- M = Q1 R, rows of R to the lanes, one-sided Jacobi on them: R^T J =
+    //      Vs S.  Loops run over SM - 8 entries when s fits in them (entries
     //      beyond s are zero, so the width changes no bit) ----
-    double fro;
+    double f2 = 0.0;
+#pragma unroll
+    for (int q = 0; q < SM; q++) f2 = fma(xm[q], xm[q], f2);
+    f2 = wsum(f2);
+    const double fro = sqrt(f2);
+    wv_qr_cols<SM>(xm, s);
+#pragma unroll
+    for (int q = 0; q < SM; q++)
+        if (q < s && lane < s) L[q * Cf::LDJ + lane] = q <= lane ? xm[q] : 0.0;
+    wv_sync();
+#pragma unroll
+    for (int q = 0; q < SM; q++) xm[q] = (lane < s && q < s) ? L[lane * Cf::LDJ + q] : 0.0;
+    wv_sync();
     if constexpr (SM <= 48) {
         constexpr int WJ = SM - 8;
-        fro = (s <= WJ) ? wv_jacobi<SM, WJ>(xm, s, acc, fixed_rk, o.unconv)
-                        : wv_jacobi<SM, SM>(xm, s, acc, fixed_rk, o.unconv);
+        if (s <= WJ) wv_jacobi<SM, WJ>(xm, s, f2, acc, fixed_rk, o.unconv);
+        else wv_jacobi<SM, SM>(xm, s, f2, acc, fixed_rk, o.unconv);
     } else {  // one width: a second copy costs the widest class registers
-        fro = wv_jacobi<SM, SM>(xm, s, acc, fixed_rk, o.unconv);
+        wv_jacobi<SM, SM>(xm, s, f2, acc, fixed_rk, o.unconv);
     }
     // ---- singular values, order, rank ----
     double sig = 0.0;
