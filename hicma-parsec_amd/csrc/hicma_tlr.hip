@@ -138,6 +138,7 @@ extern "C" int hicma_init_ex(hicma_ctx **ctx, int device, int flags, int cu_shar
         HIPCHK(hipEventCreateWithFlags(&c->ev_join[i], hipEventDisableTiming));
     }
     HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
+    HIPCHK(hipEventCreateWithFlags(&c->ev_syrk, hipEventDisableTiming));
     if (c->pool) {
         // keep freed blocks in the device's pool instead of returning them,
         // and never let one context's allocation reuse another stream's
@@ -195,6 +196,7 @@ extern "C" int hicma_fini(hicma_ctx *c)
         if (!c->single) (void)hipStreamDestroy(c->side[i]);
     }
     (void)hipEventDestroy(c->ev_fork);
+    (void)hipEventDestroy(c->ev_syrk);
     hipStreamDestroy(c->stream);
     delete c;
     return 0;
@@ -1007,6 +1009,7 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     if (A->rhist_on) hipLaunchKernelGGL(k_rank_hist, dim3((NT * NT + 255) / 256), dim3(256), 0, st, t, A->rhist, 0);
     const int ntg = (NB + GT - 1) / GT;
     const int ntl = ntg * (ntg + 1) / 2;
+    const int nbc = std::min((cap + GT - 1) / GT, GRAM_NB);
     // Lookahead: syrk(k) and potrf(k+1) touch only diagonal tiles and the gemm
     // updates of step k only off-diagonal ones, so the former run on a side
     // stream while the latter run, and are joined back before trsm(k+1).
@@ -1019,6 +1022,15 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
     for (int k = 0; k < NT; k++) {
         int nbnd = std::min(b - 1, NT - 1 - k);
         int nlr = NT - k - b;
+        // the low-rank columns of row k + 1, for its diagonal tile: those of earlier
+        // steps are final, so their products run beside trsm(k)
+        const int nj = k + 1 < NT ? std::max(k + 2 - b, 0) : 0;
+        auto syrk_lr_y = [&](int j0, int j1) {
+            if (j0 >= j1) return;
+            hipLaunchKernelGGL(k_syrk_lr_gram, dim3(nbc * nbc, j1 - j0), dim3(BS), 0, sd, t, k + 1, j0, Zws, od);
+            hipLaunchKernelGGL(k_syrk_lr_y, dim3(ntg, j1 - j0), dim3(BS), 0, sd, t, k + 1, j0, (const double *)Zws, Yws);
+        };
+        syrk_lr_y(0, std::min(nj, k));
         HIPCHK(cp(k, 2, st));
         if (nbnd > 0)
             hipLaunchKernelGGL(k_trsm_band, dim3(ntg, nbnd), dim3(BS), 0, st, t, k, (const double *)Inv(k),
@@ -1030,10 +1042,10 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         HIPCHK(hipStreamWaitEvent(sd, ctx->ev_join[1], 0));
         HIPCHK(cp(k, 4, sd));
         if (nbnd > 0) hipLaunchKernelGGL(k_syrk_band, dim3(ntl, nbnd), dim3(BS), 0, sd, t, k, od);
-        if (nlr > 0) {
-            hipLaunchKernelGGL(k_syrk_lr_prep, dim3(nlr), dim3(BS), 0, sd, t, k, Yws, Zws, od);
-            hipLaunchKernelGGL(k_syrk_lr_update, dim3(ntl, nlr), dim3(BS), 0, sd, t, k, (const double *)Yws);
-        }
+        syrk_lr_y(std::min(nj, k), nj);
+        if (nj > 0)
+            hipLaunchKernelGGL(k_syrk_lr_update, dim3(ntl), dim3(BS), 0, sd, t, k + 1, nj, (const double *)Yws);
+        HIPCHK(hipEventRecord(ctx->ev_syrk, sd));
         HIPCHK(cp(k, 5, sd));
         if (k + 1 < NT) {
             HIPCHK(cp(k + 1, 0, sd));
@@ -1050,7 +1062,8 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
         auto gemm_lrd = [&]() {
             if (b == 1 || nlr <= 0) return;
             const int npair = nlr * (b - 1);
-            hipLaunchKernelGGL(k_gemm_lrd_prep, dim3(npair), dim3(BS), 0, st, t, k, Wws, Xws, o);
+            hipLaunchKernelGGL(k_gemm_lrd_gram, dim3(nbc * nbc, npair), dim3(BS), 0, st, t, k, Xws, o);
+            hipLaunchKernelGGL(k_gemm_lrd_w, dim3(ntg, nbc, npair), dim3(BS), 0, st, t, k, Wws, (const double *)Xws);
             hipLaunchKernelGGL(k_gemm_lrd_update, dim3(ntg * ntg, npair), dim3(BS), 0, st, t, k, (const double *)Wws);
         };
         int T = NT - 1 - k;
@@ -1078,6 +1091,11 @@ extern "C" int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma
                 // fork: k_rc_big on the context stream, so that its few long
                 // tasks are the first to get CUs, the waves on side stream 0
                 int *redo = wlist + 4 * (size_t)wcap;
+                // Waves that fill the chip hold their CUs for the whole step: the
+                // update of the next diagonal tile goes first, or its workgroups
+                // (and the tile's factorization) wait for k_rc_big's CUs
+                // (N=90000 tile 900: 336 instead of 303 ms).
+                if (wave && ntask > (long long)WV_WPB * (wgrid - wres)) HIPCHK(hipStreamWaitEvent(st, ctx->ev_syrk, 0));
                 int wg = (int)std::min<long long>(wave ? std::min(P.nbig, wgrid - wres) : P.nbig, ntask);
                 if (wave) HIPCHK(hipEventRecord(ctx->ev_fork, st));
                 hipLaunchKernelGGL(rc_big, dim3(wg), dim3(BS), big_lds, st, t, k,

@@ -50,7 +50,7 @@ struct hicma_ctx {
     // the other stream's (k_rc_big behind the diagonal tile: 1.4 ms of a
     // 4.3 ms step for N=90000 tile 900 next to a caller's null stream).
     hipStream_t side[2];             // [0]: k_rc_wave; [1]: syrk(k) + potrf(k+1), one step ahead
-    hipEvent_t ev_fork, ev_join[2];
+    hipEvent_t ev_fork, ev_syrk, ev_join[2];
     // critical-path timing events (created on first request, reused)
     std::vector<hipEvent_t> cp_ev;
     // dense linear algebra handle of the checks (created on first use)

@@ -584,40 +584,149 @@ __global__ void __launch_bounds__(BS) k_syrk_band(TLR t, int k, OpLog o)
                            sm, true);
 }
 
-// low rank prep: Y = U (V^T V) for m = k+band..NT-1; grid (count)
-__global__ void __launch_bounds__(BS) k_syrk_lr_prep(TLR t, int k, double *Yws, double *Zws, OpLog o)
+// One 64 x 64 block (i0, j0) of X = A^T B, A NB x ra, B NB x rb (ld NB), ld of X
+// ldx.  Tall operands: each wave takes every fourth group of 16 rows, operands go
+// from memory to the matrix cores without LDS (two register sets in turn), and
+// the waves' sums are added in a fixed order.  sm: GRAM_SMEM doubles.
+#define GRAM_SMEM (2 * GT * GT)
+__device__ __forceinline__ void gram_tile(int i0, int j0, int ra, int rb, int NB, const double *A, const double *B,
+                                          double *X, int ldx, double *sm)
 {
-    __shared__ double sm[BLK_GEMM_SMEM];
-    const int NB = t.NB, cap = t.cap;
-    int m = k + t.band_size + blockIdx.x;
-    int r = *rank_at(t, m, k);
-    if (threadIdx.x == 0) {
-        unsigned long long mm = tdim(t, m);
-        unsigned long long c = opc('m', r, r, mm, 0) + opc('m', mm, r, r, 0) + opc('m', mm, mm, r, 0);
-        oplog(o, t.NT, c, m, m, true, m - k == 1);
+    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4, w = uni(threadIdx.x >> 6);
+    const int na = min(GT, ra - i0), nb = min(GT, rb - j0);
+    const wv_rsrc ar = wv_col_rsrc(A + (size_t)i0 * NB, na * NB * 8), br = wv_col_rsrc(B + (size_t)j0 * NB, nb * NB * 8);
+    mk_d4 acc[4][4];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int b = 0; b < 4; b++) acc[a][b] = mk_d4{0.0, 0.0, 0.0, 0.0};
+    auto load = [&](double (&av)[4][4], double (&bv)[4][4], int r0) {
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const int row = r0 + 4 * u + k4;
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                const int q = 16 * c + i16;  // past the resource, and so 0, for q >= na (nb)
+                av[u][c] = 16 * c < na ? wv_ld(ar, row < NB ? (row + q * NB) * 8 : WV_OOB) : 0.0;
+                bv[u][c] = 16 * c < nb ? wv_ld(br, row < NB ? (row + q * NB) * 8 : WV_OOB) : 0.0;
+            }
+        }
+    };
+    auto mul = [&](const double (&av)[4][4], const double (&bv)[4][4]) {
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+#pragma unroll
+            for (int a = 0; a < 4; a++)
+                if (16 * a < na) {
+#pragma unroll
+                    for (int b = 0; b < 4; b++)
+                        if (16 * b < nb) acc[a][b] = mk_mfma(av[u][a], bv[u][b], acc[a][b]);
+                }
+    };
+    double a0[4][4], b0[4][4], a1[4][4], b1[4][4];
+    int r0 = 16 * w;
+    if (r0 < NB) load(a0, b0, r0);
+#pragma unroll 1
+    for (; r0 < NB; r0 += 128) {
+        if (r0 + 64 < NB) load(a1, b1, r0 + 64);
+        mul(a0, b0);
+        if (r0 + 64 >= NB) break;
+        if (r0 + 128 < NB) load(a0, b0, r0 + 128);
+        mul(a1, b1);
     }
-    if (r == 0) return;
-    const double *U = lr_tile(t, m, k), *V = U + (size_t)NB * r;
-    double *Z = Zws + (size_t)m * cap * cap, *Y = Yws + (size_t)m * NB * cap;
-    blk_gemm<true, false>(r, r, NB, 1.0, V, NB, V, NB, 0.0, Z, r, sm);
-    blk_gemm<false, false>(NB, r, r, 1.0, U, NB, Z, r, 0.0, Y, NB, sm);
+    // waves 2, 3 into waves 0, 1, then wave 1 into wave 0
+    auto put = [&](double *d) {
+#pragma unroll
+        for (int e = 0; e < 64; e++) d[64 * e + lane] = acc[e >> 4][(e >> 2) & 3][e & 3];
+    };
+    auto add = [&](const double *d) {
+#pragma unroll
+        for (int e = 0; e < 64; e++) acc[e >> 4][(e >> 2) & 3][e & 3] += d[64 * e + lane];
+    };
+    if (w >= 2) put(sm + (w - 2) * GT * GT);
+    __syncthreads();
+    if (w < 2) add(sm + w * GT * GT);
+    __syncthreads();
+    if (w == 1) put(sm);
+    __syncthreads();
+    if (w == 0) {
+        add(sm);
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int b = 0; b < 4; b++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int i = 16 * a + k4 + 4 * r, j = 16 * b + i16;
+                    if (i < na && j < nb) X[(i0 + i) + (size_t)(j0 + j) * ldx] = acc[a][b][r];
+                }
+    }
+    __syncthreads();
 }
 
-// low rank update: T_mm -= Y U^T; grid (lower tiles, count)
-__global__ void __launch_bounds__(BS) k_syrk_lr_update(TLR t, int k, const double *Yws)
+// The low-rank part of the update of the next diagonal tile m = k + 1, of all
+// columns j <= m - band at once, C -= sum_j U_j (V_j^T V_j) U_j^T: the tile is
+// read and written once, whereas an update per step and tile moved every later
+// diagonal tile in every step (1.9 ms a step of N=90000 tile 900 on the CUs the
+// recompressions leave, now 0.16; the factorization 345 -> 303 ms).  Z_j and Y_j
+// by one workgroup per tile took 120 us at NB = 900 and 515 us at ranks up to 175
+// (NB = 512); now 25 and 38 us.  Three launches, each over all columns:
+// Z_j = V_j^T V_j, Y_j = U_j Z_j, C -= sum_j Y_j U_j^T.
+
+// The grids of these and the k_gemm_lrd kernels take up to GRAM_NB blocks along a
+// rank and stride over more: a grid for ranks up to cap leaves thousands of empty
+// workgroups to the CUs beside the recompressions (Y_j 1.6 ms a step for N=90000).
+#define GRAM_NB 3
+
+// Z_j; grid (up to GRAM_NB x GRAM_NB blocks of 64 x 64, columns jb + j)
+__global__ void __launch_bounds__(BS) k_syrk_lr_gram(TLR t, int m, int jb, double *Zws, OpLog o)
+{
+    __shared__ double sm[GRAM_SMEM];
+    const int NB = t.NB, cap = t.cap, j = jb + blockIdx.y;
+    const int r = *rank_at(t, m, j), nbx = (r + GT - 1) / GT;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        unsigned long long mm = tdim(t, m);
+        unsigned long long c = opc('m', r, r, mm, 0) + opc('m', mm, r, r, 0) + opc('m', mm, mm, r, 0);
+        oplog(o, t.NT, c, m, m, true, m - j == 1);
+    }
+    const double *V = lr_tile(t, m, j) + (size_t)NB * r;
+    for (int e = blockIdx.x; e < nbx * nbx; e += gridDim.x)
+        gram_tile(e % nbx * GT, e / nbx * GT, r, r, NB, V, V, Zws + (size_t)j * cap * cap, r, sm);
+}
+
+// Y_j; grid (blocks of 64 rows, columns jb + j)
+__global__ void __launch_bounds__(BS) k_syrk_lr_y(TLR t, int m, int jb, const double *Zws, double *Yws)
+{
+    __shared__ double sm[BLK_GEMM_SMEM];
+    const int NB = t.NB, cap = t.cap, j = jb + blockIdx.y, i0 = blockIdx.x * GT;
+    const int r = *rank_at(t, m, j);
+    for (int j0 = 0; j0 < r; j0 += GT)
+        gemm_tile<false, false>(i0, j0, NB, r, r, 1.0, lr_tile(t, m, j), NB, Zws + (size_t)j * cap * cap, r, 0.0,
+                                Yws + (size_t)j * NB * cap, NB, sm);
+}
+
+// C -= sum_{j < nj} Y_j U_j^T, the lower triangle; grid (lower 64 x 64 blocks)
+__global__ void __launch_bounds__(BS) k_syrk_lr_update(TLR t, int m, int nj, const double *Yws)
 {
     __shared__ double sm[BLK_GEMM_SMEM];
     const int NB = t.NB, cap = t.cap;
-    int m = k + t.band_size + blockIdx.y;
-    int r = *rank_at(t, m, k);
-    if (r == 0) return;
     int ti, tj;
     tri_decode((long long)blockIdx.x, ti, tj);
     ti -= 1;
-    const double *U = lr_tile(t, m, k);
-    const double *Y = Yws + (size_t)m * NB * cap;
-    gemm_tile<false, true>(ti * GT, tj * GT, NB, NB, r, -1.0, Y, NB, U, NB, 1.0, band_tile(t, m, m), NB, sm,
-                           true);
+    const int i0 = ti * GT, j0 = tj * GT;
+    mk_d4 acc[2][2];
+    mk_zero(acc);
+    for (int j = 0; j < nj; j++) {
+        const int r = *rank_at(t, m, j);
+        // as C^T = U Y^T, so that consecutive lanes hold consecutive rows of C
+        const MkOps<false, false> op{lr_tile(t, m, j), NB, Yws + (size_t)j * NB * cap, NB};
+        mk_accum(op, NB, NB, j0, i0, 0, r, acc, sm);
+    }
+    double *C = band_tile(t, m, m);
+    mk_store(acc, [&](int jj, int ii, double v) {
+        const int gi = i0 + ii, gj = j0 + jj;
+        if (gi < NB && gi >= gj) C[gi + (size_t)gj * NB] -= v;
+    });
 }
 
 // ======================= gemm, dense cases =======================
@@ -641,31 +750,44 @@ __global__ void __launch_bounds__(BS) k_gemm_dense(TLR t, int k, OpLog o)
 }
 
 // (ii) A LR, B dense, C dense and (iii) A, B LR, C dense: W = Av^T B^T or
-// (Av^T Bv) Bu^T (rA x NB).  Pairs: m = k+band+p/(band-1), n = m-1-p%(band-1).
-__global__ void __launch_bounds__(BS) k_gemm_lrd_prep(TLR t, int k, double *Wws, double *Xws, OpLog o)
+// (Av^T Bv) Bu^T (rA x NB), C -= Au W.  Pairs: m = k+band+p/(band-1),
+// n = m-1-p%(band-1).  One workgroup per 64 x 64 block of X and W (one per pair
+// took 240 us at NB = 512, 720 us at ranks up to 175).
+
+// X = Av^T Bv of case (iii) and the op counts; grid (up to GRAM_NB x GRAM_NB blocks, pairs)
+__global__ void __launch_bounds__(BS) k_gemm_lrd_gram(TLR t, int k, double *Xws, OpLog o)
+{
+    __shared__ double sm[GRAM_SMEM];
+    const int NB = t.NB, cap = t.cap, b = t.band_size, pidx = blockIdx.y;
+    const int m = k + b + pidx / (b - 1), n = m - 1 - pidx % (b - 1);
+    const int ra = *rank_at(t, m, k), mm = tdim(t, m);
+    const bool bdense = n - k < b;
+    const int rb = bdense ? 0 : *rank_at(t, n, k);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (bdense) oplog(o, t.NT, opc('m', mm, mm, ra, 0) * 2, m, n, true, false);
+        else
+            oplog(o, t.NT, opc('m', mm, mm, ra < rb ? ra : rb, 0) + opc('m', mm, ra, rb, 0) * 2, m, n, true, false);
+    }
+    const int na = (ra + GT - 1) / GT, nb = (rb + GT - 1) / GT;
+    for (int e = blockIdx.x; e < na * nb; e += gridDim.x)
+        gram_tile(e % na * GT, e / na * GT, ra, rb, NB, lr_tile(t, m, k) + (size_t)NB * ra,
+                  lr_tile(t, n, k) + (size_t)NB * rb, Xws + (size_t)pidx * cap * cap, ra, sm);
+}
+
+// W; grid (blocks of 64 columns, up to GRAM_NB blocks along r_A, pairs)
+__global__ void __launch_bounds__(BS) k_gemm_lrd_w(TLR t, int k, double *Wws, const double *Xws)
 {
     __shared__ double sm[BLK_GEMM_SMEM];
-    const int NB = t.NB, cap = t.cap, b = t.band_size;
-    int pidx = blockIdx.x;
-    int m = k + b + pidx / (b - 1), n = m - 1 - pidx % (b - 1);
-    int ra = *rank_at(t, m, k);
-    const double *A = lr_tile(t, m, k), *Av = A + (size_t)NB * ra;
+    const int NB = t.NB, cap = t.cap, b = t.band_size, pidx = blockIdx.z, j0 = blockIdx.x * GT;
+    const int m = k + b + pidx / (b - 1), n = m - 1 - pidx % (b - 1);
+    const bool bdense = n - k < b;
+    const int ra = *rank_at(t, m, k), rb = bdense ? 0 : *rank_at(t, n, k);
+    if (!bdense && rb == 0) return;
+    const double *Av = lr_tile(t, m, k) + (size_t)NB * ra, *X = Xws + (size_t)pidx * cap * cap;
     double *W = Wws + (size_t)pidx * cap * NB;
-    int mm = tdim(t, m);
-    if (n - k < b) {
-        if (threadIdx.x == 0) oplog(o, t.NT, opc('m', mm, mm, ra, 0) * 2, m, n, true, false);
-        if (ra == 0) return;
-        blk_gemm<true, true>(ra, NB, NB, 1.0, Av, NB, band_tile(t, n, k), NB, 0.0, W, cap, sm);
-    } else {
-        int rb = *rank_at(t, n, k);
-        if (threadIdx.x == 0)
-            oplog(o, t.NT, opc('m', mm, mm, ra < rb ? ra : rb, 0) + opc('m', mm, ra, rb, 0) * 2, m, n, true,
-                  false);
-        if (ra == 0 || rb == 0) return;
-        const double *B = lr_tile(t, n, k), *Bv = B + (size_t)NB * rb;
-        double *X = Xws + (size_t)pidx * cap * cap;
-        blk_gemm<true, false>(ra, rb, NB, 1.0, Av, NB, Bv, NB, 0.0, X, ra, sm);
-        blk_gemm<false, true>(ra, NB, rb, 1.0, X, ra, B, NB, 0.0, W, cap, sm);
+    for (int i0 = blockIdx.y * GT; i0 < ra; i0 += gridDim.y * GT) {
+        if (bdense) gemm_tile<true, true>(i0, j0, ra, NB, NB, 1.0, Av, NB, band_tile(t, n, k), NB, 0.0, W, cap, sm);
+        else gemm_tile<false, true>(i0, j0, ra, NB, rb, 1.0, X, ra, lr_tile(t, n, k), NB, 0.0, W, cap, sm);
     }
 }
 
