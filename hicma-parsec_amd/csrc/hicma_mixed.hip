@@ -64,7 +64,10 @@ __device__ double lr_frob2_part(const TE *U, int NB, int r, double *sm)
 // Frobenius norm of every lower tile (m >= n) into nrm[n*NT + m]: band tiles
 // over their rows < tdim(m) and columns < tdim(n) (the padding left out),
 // low-rank tiles from their Gram matrices in the type they are held in.
-// One workgroup per tile, grid-stride over the NT (NT + 1) / 2 tiles.
+// One workgroup per tile, grid-stride over the NT (NT + 1) / 2 tiles.  What bounds
+// it: one workgroup's chain through its tile; a band tile element by element (a
+// 64-bit division and one load in flight) made it 366 us at N=8100 tile 465, now
+// 180 us (its low-rank tiles' Gram blocks).
 __global__ void __launch_bounds__(256) k_tile_normf(TLR t, double *nrm)
 {
     __shared__ double sm[MK_SMEM];
@@ -79,11 +82,20 @@ __global__ void __launch_bounds__(256) k_tile_normf(TLR t, double *nrm)
         if (m - n < t.band_size) {
             const double *T = band_tile(t, m, n);
             const int rows = tdim(t, m), cols = tdim(t, n);
-            for (long e = tid; e < (long)rows * cols; e += 256) {
-                const int j = (int)(e / rows), i = (int)(e - (long)j * rows);
-                const double v = T[i + (size_t)j * NB];
-                part = fma(v, v, part);
-            }
+            // a wave's lanes run down the columns, 8 columns of 4 row blocks
+            // (32 loads) at a time: the tile costs NB^2 / 8192 memory latencies
+            const int w = tid >> 6, lane = tid & 63;
+            for (int j = w; j < cols; j += 32)
+                for (int i = lane; i < rows; i += 256) {
+                    double v[32];
+#pragma unroll
+                    for (int q = 0; q < 32; q++) {
+                        const int jj = j + 4 * (q & 7), ii = i + 64 * (q >> 3);
+                        v[q] = (jj < cols && ii < rows) ? T[ii + (size_t)jj * NB] : 0.0;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 32; q++) part = fma(v[q], v[q], part);
+                }
         } else {
             const int r = *rank_at(t, m, n);
             if (r > 0) {
