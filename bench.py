@@ -40,7 +40,7 @@ HBM_PEAK_GBS = 8000.0
 # NB=900, maxrank 150, eps 1e-8), measured with two rocprofv3 --pmc passes
 # (FETCH_SIZE, WRITE_SIZE) summed over the group's kernels and scaled by the
 # counters' reading of a device copy of known size (x2.0 and x1.0).
-C2_TRAFFIC_BYTES_PER_GROUP = 6.399e9
+C2_TRAFFIC_BYTES_PER_GROUP = 6.937e9
 # HBM the serving sweep's admission may reserve (of 288 GB): the rest covers
 # what the stream-ordered pool holds beyond the reservations
 SERVE_BUDGET_GB = 200.0
@@ -235,7 +235,7 @@ def main():
     ap.add_argument("--no-serve", action="store_true")
     ap.add_argument("--no-autotune", action="store_true")
     ap.add_argument("--schedule", type=int, default=None,
-                    help="fixed schedule threshold (tasks per step below which the four-wave kernel runs)")
+                    help="fixed schedule threshold (tasks per step below which the workgroup kernel runs)")
     ap.add_argument("--serve-rates", default="2,8,32,128")
     ap.add_argument("--serve-requests", type=int, default=16)
     ap.add_argument("--serve-slots", type=int, default=4)
@@ -265,11 +265,11 @@ def main():
     if a.schedule is not None:
         sched = a.schedule
         ctx.set_wave_min_tasks(sched)
-        log(f"schedule: four-wave kernel below {sched} tasks per step (given)")
+        log(f"schedule: workgroup kernel below {sched} tasks per step (given)")
     elif not a.no_autotune:
         t0 = time.time()
         sched, ts = A.autotune_schedule(a.eps, a.maxrank, reps=2)
-        log(f"schedule autotuner: four-wave kernel below {sched} tasks per step ({ts:.3f}s; {time.time() - t0:.1f}s)")
+        log(f"schedule autotuner: workgroup kernel below {sched} tasks per step ({ts:.3f}s; {time.time() - t0:.1f}s)")
 
     for w in range(a.warmup):
         A.copy_from(pristine)
@@ -355,9 +355,9 @@ def main():
             "bound": "mfma",
             "pipe": ("FP64 compute roofline: the group's QR panels, trailing updates and Jacobi rotations are "
                      "VALU FMAs, its tall products MFMA; gfx950's FP64 vector and matrix peaks are both 78.6 TFLOP/s"),
-            "kernel": ("recompression launch group of a panel step: k_classify_wave + k_rc_wave<32|48|64> "
-                       "(one wave per low-rank gemm task: QR + Jacobi-SVD) + k_rc_wide (stacks of 61..128 "
-                       "columns, four waves per task), on three concurrent streams"),
+            "kernel": ("recompression launch group of a panel step: k_classify_wave + k_rc_wave (stacks up to 60 "
+                       "columns, one wave per low-rank gemm task: QR + Jacobi-SVD) beside k_rc_big (wider stacks, "
+                       "one workgroup per task)"),
             "achieved": round(achieved, 4),
             "peak": FP64_PEAK_TFLOPS,
             "unit": "TFLOP/s",

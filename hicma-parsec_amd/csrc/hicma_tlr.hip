@@ -1285,7 +1285,7 @@ extern "C" int hicma_set_wave_min_tasks(hicma_ctx *ctx, int ntask)
 }
 
 // Times HiCMA_dpotrf_L on a copy of A for each candidate schedule (steps
-// with fewer tasks than the threshold on the four-wave kernel) and keeps the
+// with fewer tasks than the threshold on k_rc_big) and keeps the
 // fastest in the context.  A is not modified.
 extern "C" int hicma_autotune_schedule(hicma_ctx *ctx, hicma_tlr_desc *A, double acc, int maxrank, int reps,
                                        int *best, double *best_seconds)

@@ -40,7 +40,7 @@ struct hicma_ctx {
     double *d_scalar;
     size_t lds_max;
     // schedule: panel steps with fewer low-rank gemm tasks than this run
-    // every task on the four-wave kernel (0: never)
+    // every task on k_rc_big (0: never)
     int wave_min_tasks;
     int profile;                     // record events around recompression launches
     std::vector<hipEvent_t> prof_ev; // pairs

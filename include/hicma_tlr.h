@@ -163,7 +163,7 @@ int HiCMA_dpotrf_L(hicma_ctx *ctx, int uplo, hicma_tlr_desc *A, hicma_tlr_desc *
 int hicma_factor_graph(hicma_tlr_desc *A, int enable);
 
 /* Schedule of the low-rank gemm + recompression tasks: panel steps with
- * fewer tasks than ntask run every task on the four-wave kernel (a task's
+ * fewer tasks than ntask run every task on k_rc_big (a task's
  * latency, not the step's throughput, bounds such steps); 0 (the default)
  * sorts each step's tasks by stack width over the one-wave kernels.  No counterpart
  * in the reference (its PaRSEC runtime schedules tasks on CPU cores).
