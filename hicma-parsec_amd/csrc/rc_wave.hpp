@@ -151,63 +151,15 @@ __device__ __forceinline__ void wv_tall_mul(const double (&av)[RT][SM / 4], cons
     }
 }
 
-// The same with K read from LDS, a chunk of 16 K rows at a time (for the
-// widest stacks, whose K does not fit in registers).
-template <int SM, int RT>
-__device__ __forceinline__ void wv_tall_mul_lds(const double (&av)[RT][SM / 4], const double (&ax)[RT], int NB, int kd,
-                                                int c0, int nc, double alpha, const double *Kl, int ldk, wv_rsrc dr,
-                                                int r0, int rstep)
-{
-    const int lane = threadIdx.x & 63, i16 = lane & 15, k4 = lane >> 4;
-    constexpr int KS = SM / 4, TN = SM / 16;
-    const int cx = 4 * (c0 >> 2) + k4;
-    const bool mix = (c0 & 3) != 0 && cx >= c0 && cx < kd;
-#pragma unroll
-    for (int tn = 0; tn < TN; tn++) {
-        if (16 * tn < nc) {
-            const double kbx = Kl[(mix ? cx : 0) * ldk + 16 * tn + i16];
-            wv_d4 acc[RT];
-#pragma unroll
-            for (int t = 0; t < RT; t++) acc[t] = mfma16(ax[t], mix ? kbx : 0.0, wv_d4{0.0, 0.0, 0.0, 0.0});
-#pragma unroll
-            for (int kc = 0; kc < KS; kc += 4) {
-                if (4 * kc < kd) {
-                    double kb[4];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const int kr = 4 * (kc + u) + k4;
-                        const double v = Kl[(kr < kd ? kr : 0) * ldk + 16 * tn + i16];
-                        kb[u] = kr < kd ? v : 0.0;
-                    }
-#pragma unroll
-                    for (int u = 0; u < 4; u++)
-#pragma unroll
-                        for (int t = 0; t < RT; t++) acc[t] = mfma16(av[t][kc + u], kb[u], acc[t]);
-                }
-            }
-            const int j = 16 * tn + i16;
-#pragma unroll
-            for (int t = 0; t < RT; t++) {
-                const int rt = r0 + rstep * t;
-#pragma unroll
-                for (int r = 0; r < 4; r++) {
-                    const int i = rt + k4 + 4 * r;
-                    wv_st(alpha * acc[t][r], dr, (j < nc && i < NB) ? (i + j * NB) * 8 : WV_OOB);
-                }
-            }
-        }
-    }
-}
-
 // Tall product D (NB x nc, ld NB) = alpha * A (NB x kd) K (kd x nc) with A's
 // columns given by a WvSrc and K in LDS (K[c][j] at Kl[c * ldk + j]).  Work
 // goes in batches of RT 16-row tiles (tiles t0, t0 + tstep, ... when several
 // waves share the product); a batch's A loads are all issued before its
-// first MFMA.  With PP, K is held in registers and batches alternate
+// first MFMA.  K is held in registers and batches alternate
 // between two register sets: batch i + 1 loads while batch i multiplies and
 // stores.  Rows of a batch are read before any of them is written, so D may
 // overwrite A's storage row for row.
-template <int SM, int RT = (SM <= 32 ? 2 : 1), bool PP = (SM <= 64)>
+template <int SM, int RT = (SM <= 32 ? 2 : 1)>
 __device__ __forceinline__ void wv_tall_mm(int NB, int kd, int nc, double alpha, WvSrc A, const double *Kl, int ldk,
                                            double *D, int t0 = 0, int tstep = 1)
 {
@@ -216,26 +168,17 @@ __device__ __forceinline__ void wv_tall_mm(int NB, int kd, int nc, double alpha,
     const wv_rsrc dr = wv_col_rsrc(D, NB * nc * 8);
     const int c0 = A.c0 < kd ? A.c0 : kd;
     const wv_rsrc r0s = wv_col_rsrc(A.s0, c0 * A.lda * 8), r1s = wv_col_rsrc(A.s1, (kd - c0) * A.lda * 8);
-    if constexpr (PP) {
-        double kv[SM / 4][SM / 16], kx[SM / 16];
-        wv_tall_k<SM>(kv, kx, kd, c0, Kl, ldk);
-        double a0[RT][SM / 4], x0[RT], a1[RT][SM / 4], x1[RT];
-        if (r0 < NB) wv_tall_ld<SM, RT>(a0, x0, NB, kd, r0s, r1s, c0, A.lda, r0, rstep);
+    double kv[SM / 4][SM / 16], kx[SM / 16];
+    wv_tall_k<SM>(kv, kx, kd, c0, Kl, ldk);
+    double a0[RT][SM / 4], x0[RT], a1[RT][SM / 4], x1[RT];
+    if (r0 < NB) wv_tall_ld<SM, RT>(a0, x0, NB, kd, r0s, r1s, c0, A.lda, r0, rstep);
 #pragma unroll 1
-        for (; r0 < NB; r0 += 2 * bstep) {
-            if (r0 + bstep < NB) wv_tall_ld<SM, RT>(a1, x1, NB, kd, r0s, r1s, c0, A.lda, r0 + bstep, rstep);
-            wv_tall_mul<SM, RT>(a0, x0, kv, kx, NB, kd, nc, alpha, dr, r0, rstep);
-            if (r0 + bstep >= NB) break;
-            if (r0 + 2 * bstep < NB) wv_tall_ld<SM, RT>(a0, x0, NB, kd, r0s, r1s, c0, A.lda, r0 + 2 * bstep, rstep);
-            wv_tall_mul<SM, RT>(a1, x1, kv, kx, NB, kd, nc, alpha, dr, r0 + bstep, rstep);
-        }
-    } else {
-#pragma unroll 1
-        for (; r0 < NB; r0 += bstep) {
-            double av[RT][SM / 4], ax[RT];
-            wv_tall_ld<SM, RT>(av, ax, NB, kd, r0s, r1s, c0, A.lda, r0, rstep);
-            wv_tall_mul_lds<SM, RT>(av, ax, NB, kd, c0, nc, alpha, Kl, ldk, dr, r0, rstep);
-        }
+    for (; r0 < NB; r0 += 2 * bstep) {
+        if (r0 + bstep < NB) wv_tall_ld<SM, RT>(a1, x1, NB, kd, r0s, r1s, c0, A.lda, r0 + bstep, rstep);
+        wv_tall_mul<SM, RT>(a0, x0, kv, kx, NB, kd, nc, alpha, dr, r0, rstep);
+        if (r0 + bstep >= NB) break;
+        if (r0 + 2 * bstep < NB) wv_tall_ld<SM, RT>(a0, x0, NB, kd, r0s, r1s, c0, A.lda, r0 + 2 * bstep, rstep);
+        wv_tall_mul<SM, RT>(a1, x1, kv, kx, NB, kd, nc, alpha, dr, r0 + bstep, rstep);
     }
 }
 
